@@ -138,32 +138,72 @@ __device__ __forceinline__ float tanh_exp(float y) {
   return 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
 }
 
-// Philox4x32-10 (Salmon, Moraes, Dror, Shaw, "Parallel random numbers: as easy as 1, 2, 3",
-// SC 2011): word 0 after ten rounds on the counter (idx, 0, 0) under the key `seed`. The
-// reference draws its dropout stream this way (kernels/fa_common.hpp:71-82).
-__device__ __forceinline__ uint32_t philox_w0(uint64_t seed, uint64_t idx) {
-  uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
-  uint32_t c0 = (uint32_t)idx, c1 = (uint32_t)(idx >> 32), c2 = 0u, c3 = 0u;
-#pragma unroll
-  for (int r = 0; r < 10; r++) {
-    const uint32_t hi0 = __umulhi(0xD2511F53u, c0), lo0 = 0xD2511F53u * c0;
-    const uint32_t hi1 = __umulhi(0xCD9E8D57u, c2), lo1 = 0xCD9E8D57u * c2;
-    c0 = hi1 ^ c1 ^ k0;
-    c1 = lo1;
-    c2 = hi0 ^ c3 ^ k1;
-    c3 = lo0;
-    k0 += 0x9E3779B9u;
-    k1 += 0xBB67AE85u;
-  }
-  return c0;
+// x ^ y ^ z in one instruction (v_bitop3_b32, truth table 0x96)
+__device__ __forceinline__ uint32_t xor3(uint32_t x, uint32_t y, uint32_t z) {
+  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)x, (int)y, (int)z, 0x96);
 }
 
-// Dropout multiplier of one score: keep_scale (= 1/(1-p)) when (word0 >> 8) * 2^-24 >= p,
-// otherwise 0; idx = (h*SQ + q)*SK + key with no batch term (fa_common.hpp:84-88,
-// fa_forward.hip:255-259).
-__device__ __forceinline__ float dropout_z(uint64_t seed, uint64_t idx, float p, float keep_scale) {
-  const float u = (float)(philox_w0(seed, idx) >> 8) * (1.0f / 16777216.0f);
-  return u >= p ? keep_scale : 0.0f;
+// Dropout stream: word 0 of Philox4x32-10 (Salmon, Moraes, Dror, Shaw, "Parallel random numbers:
+// as easy as 1, 2, 3", SC 2011) on the counter (idx, 0, 0) under the key `seed`. The reference
+// draws its dropout stream this way (kernels/fa_common.hpp:71-82). Of the ten rounds' 40
+// 32-bit half products only those that word 0 of this counter needs are formed, as 64-bit
+// products: counter words 2 and 3 start at zero, so the first round has one product and (word 1
+// being zero after it, and word 0 uniform when the high half of idx is) the second one that
+// varies by lane; the last round needs one high half, the one before it three halves.
+__device__ __forceinline__ uint32_t philox_w0(uint32_t k0, uint32_t k1, uint32_t lo, uint32_t hi) {
+  constexpr uint32_t kM0 = 0xD2511F53u, kM1 = 0xCD9E8D57u, kW0 = 0x9E3779B9u, kW1 = 0xBB67AE85u;
+  const uint64_t p0 = (uint64_t)kM0 * lo;
+  uint32_t c0 = hi ^ k0, c1 = 0u, c2 = (uint32_t)(p0 >> 32) ^ k1, c3 = (uint32_t)p0;
+#pragma unroll
+  for (int r = 1; r < 9; r++) {
+    k0 += kW0;
+    k1 += kW1;
+    const uint64_t a = (uint64_t)kM0 * c0, b = (uint64_t)kM1 * c2;
+    c0 = xor3((uint32_t)(b >> 32), c1, k0);
+    c2 = xor3((uint32_t)(a >> 32), c3, k1);
+    c1 = (uint32_t)b;
+    c3 = (uint32_t)a;
+  }
+  return xor3(__umulhi(kM1, c2), c1, k0 + kW0);
+}
+
+// The dropout decision of score idx = (h*SQ + q)*SK + key (no batch term, fa_common.hpp:84-88,
+// fa_forward.hip:255-259): kept when (word0 >> 8) * 2^-24 >= p, that is when word0 is at least
+// ceil(p * 2^24) * 2^8 (p < 1, so the product with 2^24 is exact and the bound fits 32 bits).
+__device__ __forceinline__ uint32_t dropout_bound(float p) {
+  return (uint32_t)ceilf(p * 16777216.0f) << 8;
+}
+
+// Keep bits of N <= 32 scores: bit i for index idx0 + off(i), where off is uniform and off(i) <=
+// `span`. The high word of the index is the same for all of a wave's scores nearly always, and
+// then uniform; a wave whose indices straddle a multiple of 2^32 takes the rolled loop.
+// What bounds it is VALU issue: 14 64-bit and 4 32-bit products, 18 xors and 4 others per score
+// (all of them issue at one rate on gfx950), against some 80 for the ten full rounds. Encoder
+// layers of B32 S509 H16 D64 fp16: the forward 359 -> 250 us, the pair dK/dV kernel 758 -> 625 us.
+template <int N, class Off>
+__device__ __forceinline__ uint32_t dropout_bits(uint64_t seed, uint64_t idx0, uint64_t span, uint32_t bound, Off&& off) {
+  static_assert(N <= 32, "one word of bits");
+  const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(idx0 >> 32));
+  const bool ok = (uint32_t)(idx0 >> 32) == hi && (uint32_t)((idx0 + span) >> 32) == hi;
+  uint32_t bits = 0u;
+  if (__builtin_amdgcn_ballot_w64(!ok) == 0) {
+    const uint32_t lo = (uint32_t)idx0;
+#pragma unroll
+    for (int i = N - 1; i >= 0; i--) bits = bits + bits + (philox_w0(k0, k1, lo + (uint32_t)off(i), hi) >= bound ? 1u : 0u);
+  } else {
+#pragma nounroll
+    for (int i = N - 1; i >= 0; i--) {
+      const uint64_t idx = idx0 + off(i);
+      bits = bits + bits + (philox_w0(k0, k1, (uint32_t)idx, (uint32_t)(idx >> 32)) >= bound ? 1u : 0u);
+    }
+  }
+  return bits;
+}
+
+// x where bit i of the keep bits is set, else 0
+__device__ __forceinline__ float dropout_keep(float x, uint32_t bits, int i) {
+  return __uint_as_float(__float_as_uint(x) & (uint32_t)__builtin_amdgcn_sbfe((int)bits, i, 1));
 }
 
 // Reductions across lanes l and l^32 (the two halves of one MFMA 32x32 C column) with

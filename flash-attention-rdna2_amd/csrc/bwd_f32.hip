@@ -129,6 +129,7 @@ bwd_dq_f32_kernel(FableBwdParams p, int nqt) {
   const float c_log2 = p.scale * kLog2e;
   const float slope = (FEAT && p.alibi) ? p.alibi[h] : 0.0f;
   const float inv_cap = p.softcap > 0.0f ? 1.0f / p.softcap : 0.0f;
+  const uint32_t drop_bound = DROP ? dropout_bound(p.dropout_p) : 0u;
 
   f32x4 dqacc[C::NDB];
 #pragma unroll
@@ -183,6 +184,10 @@ bwd_dq_f32_kernel(FableBwdParams p, int nqt) {
         }
       // s[bb][j]: key kb + 16bb + 4g + j, query qi
       const bool edge = FEAT || (CAUSAL && kb + C::BC - 1 > qw + delta) || kb + C::BC > SK;
+      uint32_t keep = 0u;  // bit 4*bb + j: score s[bb][j] is kept
+      if constexpr (DROP)
+        keep = dropout_bits<4 * C::NKB>(p.drop_seed, ((uint64_t)h * SQ + qi) * SK + kb + 4 * g, C::BC, drop_bound,
+                                        [](int i) { return (uint64_t)(16 * (i >> 2) + (i & 3)); });
 #pragma unroll
       for (int bb = 0; bb < C::NKB; bb++)
 #pragma unroll
@@ -192,8 +197,7 @@ bwd_dq_f32_kernel(FableBwdParams p, int nqt) {
           const float x = logit2_f32<FEAT>(p, s[bb][j], c_log2, slope, inv_cap, qi, key, deriv);
           float pr = exp2_fast(x - lse2);
           if (edge && !visible_b<CAUSAL, FEAT>(p, qi, key, delta, SQ, SK)) pr = 0.0f;
-          const float z = DROP ? dropout_z(p.drop_seed, ((uint64_t)h * SQ + qi) * SK + key, p.dropout_p, p.keep_scale)
-                               : 1.0f;
+          const float z = DROP ? dropout_keep(p.keep_scale, keep, 4 * bb + j) : 1.0f;
           s[bb][j] = pr * (z * dp[bb][j] - Di) * deriv;  // dS^T (backward.hip:170-176)
         }
       // dQ^T += K^T . dS^T over key pairs 16bb + 4g + j
@@ -286,6 +290,7 @@ bwd_dkdv_f32_kernel(FableBwdParams p, int nkt) {
   const int total = ntq * p.gqa;
   const float c_log2 = p.scale * kLog2e;
   const float inv_cap = p.softcap > 0.0f ? 1.0f / p.softcap : 0.0f;
+  const uint32_t drop_bound = DROP ? dropout_bound(p.dropout_p) : 0u;
 
   const int lrow = tid / C::CH, lcol = 4 * (tid % C::CH);
   f32x4 ldq[C::QJ], ldd[C::QJ];
@@ -364,6 +369,10 @@ bwd_dkdv_f32_kernel(FableBwdParams p, int nkt) {
           if ((u & 3) == 3) __builtin_amdgcn_sched_barrier(0);
         }
       const bool edge = FEAT || (CAUSAL && kw + 15 > qt0 + delta) || qt0 + C::BQ > SQ || kw + 16 > SK;
+      uint32_t keep = 0u;  // bit 4*qb + j: score s[qb][j] is kept
+      if constexpr (DROP)
+        keep = dropout_bits<4 * C::NQB>(p.drop_seed, ((uint64_t)h * SQ + qt0 + 4 * g) * SK + key, (uint64_t)C::BQ * SK, drop_bound,
+                                        [&](int i) { return (uint64_t)(16 * (i >> 2) + (i & 3)) * SK; });
 #pragma unroll
       for (int qb = 0; qb < C::NQB; qb++) {
         const f32x4 l4 = *(const f32x4*)&rowv[stage][0][16 * qb + 4 * g];
@@ -375,8 +384,7 @@ bwd_dkdv_f32_kernel(FableBwdParams p, int nkt) {
           const float x = logit2_f32<FEAT>(p, s[qb][j], c_log2, slope, inv_cap, q, key, deriv);
           float pr = exp2_fast(x - l4[j]);
           if (edge && !visible_b<CAUSAL, FEAT>(p, q, key, delta, SQ, SK)) pr = 0.0f;
-          const float z = DROP ? dropout_z(p.drop_seed, ((uint64_t)h * SQ + q) * SK + key, p.dropout_p, p.keep_scale)
-                               : 1.0f;
+          const float z = DROP ? dropout_keep(p.keep_scale, keep, 4 * qb + j) : 1.0f;
           s[qb][j] = z * pr;                               // P (dropped)
           dp[qb][j] = pr * (z * dp[qb][j] - d4[j]) * deriv;  // dS
         }

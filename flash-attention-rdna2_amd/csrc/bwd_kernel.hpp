@@ -133,6 +133,7 @@ bwd_dq_kernel(FableBwdParams p, int nqt) {
   }
   const float c_log2 = p.scale * kLog2e;
   const float slope = (FEAT && p.alibi) ? p.alibi[h] : 0.0f;
+  const uint32_t drop_bound = DROP ? dropout_bound(p.dropout_p) : 0u;
 
   f32x16 dqacc[C::NDB];
 #pragma unroll
@@ -195,6 +196,11 @@ bwd_dq_kernel(FableBwdParams p, int nqt) {
         }
       const bool edge = FEAT || (CAUSAL ? (kb + C::BC - 1 > qw + delta) : (kb + C::BC > SK));
       const int kq = kb + 4 * hh;
+      uint32_t keep = 0u;  // bit 16*jb + r: score s[jb][r] is kept
+      static_assert(!DROP || C::NB <= 2, "one word of keep bits per tile");
+      if constexpr (DROP)
+        keep = dropout_bits<16 * C::NB>(p.drop_seed, ((uint64_t)h * SQ + qi) * SK + kq, C::BC, drop_bound,
+                                        [](int i) { return (uint64_t)(32 * (i >> 4) + 8 * ((i >> 2) & 3) + (i & 3)); });
 #pragma unroll
       for (int jb = 0; jb < C::NB; jb++)
 #pragma unroll
@@ -204,9 +210,7 @@ bwd_dq_kernel(FableBwdParams p, int nqt) {
           const float x = bwd_logit2<FEAT>(p, s[jb][r], c_log2, slope, qi, key, deriv);
           float pr = exp2_fast(x - lse2);
           if (edge && !visible_b<CAUSAL, FEAT>(p, qi, key, delta, SQ, SK)) pr = 0.0f;
-          const float z = DROP ? dropout_z(p.drop_seed, ((uint64_t)h * SQ + qi) * SK + key,
-                                                          p.dropout_p, p.keep_scale)
-                                              : 1.0f;
+          const float z = DROP ? dropout_keep(p.keep_scale, keep, 16 * jb + r) : 1.0f;
           s[jb][r] = pr * (z * dp[jb][r] - Di) * deriv;  // dS^T (backward.hip:170-176)
         }
       V8 pb[C::NG];
@@ -320,6 +324,7 @@ bwd_dkdv_kernel(FableBwdParams p, int nkt) {
   const int ntq = bq1 > bq0 ? (bq1 - qstart + C::BQ - 1) / C::BQ : 0;
   const int total = ntq * p.gqa;
   const float c_log2 = p.scale * kLog2e;
+  const uint32_t drop_bound = DROP ? dropout_bound(p.dropout_p) : 0u;
   // dS workspace (the head-dim pass 0 of each key block stores it): this wave's 32-key block
   // in the compacted layout, a cursor over the tiles in the loop's order (q tiles of a head,
   // then the next head), as in the pair kernel
@@ -403,6 +408,10 @@ bwd_dkdv_kernel(FableBwdParams p, int nkt) {
       // s[r] is query qt0 + 8*(r/4) + 4*hh + (r%4), key `key`
       const bool edge = FEAT || (CAUSAL ? (kw + 31 > qt0 + delta) : false) || qt0 + C::BQ > SQ || kw + 32 > SK;
       V8 pP[2], pS[2];
+      uint32_t keep = 0u;  // bit r: score s[r] is kept
+      if constexpr (DROP)
+        keep = dropout_bits<16>(p.drop_seed, ((uint64_t)h * SQ + qt0 + 4 * hh) * SK + key, (uint64_t)C::BQ * SK, drop_bound,
+                                [&](int i) { return (uint64_t)(8 * (i >> 2) + (i & 3)) * SK; });
 #pragma unroll
       for (int rq = 0; rq < 4; rq++) {
         const f32x4 l4 = *(const f32x4*)&rowv[stage][0][8 * rq + 4 * hh];
@@ -414,9 +423,7 @@ bwd_dkdv_kernel(FableBwdParams p, int nkt) {
           const float x = bwd_logit2<FEAT>(p, s[r], c_log2, slope, q, key, deriv);
           float pr = exp2_fast(x - l4[c]);
           if (edge && !visible_b<CAUSAL, FEAT>(p, q, key, delta, SQ, SK)) pr = 0.0f;
-          const float z = DROP ? dropout_z(p.drop_seed, ((uint64_t)h * SQ + q) * SK + key,
-                                                          p.dropout_p, p.keep_scale)
-                                              : 1.0f;
+          const float z = DROP ? dropout_keep(p.keep_scale, keep, r) : 1.0f;
           const float dsv = pr * (z * dp[r] - d4[c]) * deriv;
           pP[r >> 3][r & 7] = (T)(z * pr);
           pS[r >> 3][r & 7] = (T)dsv;
@@ -591,6 +598,7 @@ __device__ __forceinline__ void bwd_pair_item(const FableBwdParams& p, int nkt, 
   }
   const int qi0 = ntq > 0 ? it0 % ntq : 0, hg0 = ntq > 0 ? it0 / ntq : 0;  // its first tile
   const float c_log2 = p.scale * kLog2e;
+  const uint32_t drop_bound = DROP ? dropout_bound(p.dropout_p) : 0u;
 
   // Q/dO tiles through buffer descriptors over rows qt0..SQ-1 (rows past SQ read as zeros);
   // each thread's first QJ chunk slots are Q, the rest dO. LSE/D row values are loaded
@@ -783,15 +791,17 @@ __device__ __forceinline__ void bwd_pair_item(const FableBwdParams& p, int nkt, 
       }
     }
     V8 pP[2];
+    uint32_t keep = 0u;  // bit r: score r is kept
+    if constexpr (DROP)
+      keep = dropout_bits<16>(p.drop_seed, ((uint64_t)(kvh * p.gqa + hg) * SQ + qt0 + 4 * hh) * SK + key,
+                              (uint64_t)C::BQ * SK, drop_bound, [&](int i) { return (uint64_t)(8 * (i >> 2) + (i & 3)) * SK; });
 #pragma unroll
     for (int rq = 0; rq < 4; rq++) {
       f32x4 pd4;
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        const int r = 4 * rq + c, q = qt0 + 8 * rq + 4 * hh + c;
-        const float z = DROP ? dropout_z(p.drop_seed, ((uint64_t)(kvh * p.gqa + hg) * SQ + q) * SK + key,
-                                         p.dropout_p, p.keep_scale)
-                             : 1.0f;
+        const int r = 4 * rq + c;
+        const float z = DROP ? dropout_keep(p.keep_scale, keep, r) : 1.0f;
         pP[r >> 3][r & 7] = (T)(z * pr[r]);
         // p * deriv >= 0; a dropped score hands it over negated, so the dP-wave knows z
         pd4[c] = z == 0.0f ? -(pr[r] * dv[r]) : pr[r] * dv[r];

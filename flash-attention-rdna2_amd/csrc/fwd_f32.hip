@@ -110,6 +110,7 @@ fwd_f32_kernel(FableFwdParams p, int nqt) {
   const float aslope2 = (FEAT && p.alibi_slopes) ? p.alibi_slopes[h] * kLog2e : 0.0f;
   const float inv_cap = p.softcap > 0.0f ? 1.0f / p.softcap : 0.0f;
   const float keep_scale = DROP ? 1.0f / (1.0f - p.dropout_p) : 1.0f;
+  const uint32_t drop_bound = DROP ? dropout_bound(p.dropout_p) : 0u;
 
   // tile loads: thread chunk j is row RSTEP*j + tid/CH, float4 column tid%CH
   const int lrow = tid / C::CH, lcol = 4 * (tid % C::CH);
@@ -186,18 +187,17 @@ fwd_f32_kernel(FableFwdParams p, int nqt) {
         m_run = m_cand;
       }
       const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+      uint32_t keep = 0u;  // bit 4*b + j: score s[b][j] is kept
+      if constexpr (DROP)
+        keep = dropout_bits<4 * C::NKB>(p.philox_seed, ((uint64_t)h * SQ + qi) * SK + kb + 4 * g, C::BC, drop_bound,
+                                        [](int i) { return (uint64_t)(16 * (i >> 2) + (i & 3)); });
 #pragma unroll
       for (int b = 0; b < C::NKB; b++)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           const float pe = exp2_fast(s[b][j] - m_use);
           l_run += pe;
-          float pz = pe;
-          if constexpr (DROP) {
-            const int key = kb + 16 * b + 4 * g + j;
-            pz *= dropout_z(p.philox_seed, ((uint64_t)h * SQ + qi) * SK + key, p.dropout_p, keep_scale);
-          }
-          s[b][j] = pz;
+          s[b][j] = DROP ? dropout_keep(pe, keep, 4 * b + j) : pe;
         }
       // O^T += V^T . P^T over key pairs 16b + 4g + j
       const float* vp = vl + st * C::TILE + 4 * g * C::STR + c16;
@@ -216,7 +216,7 @@ fwd_f32_kernel(FableFwdParams p, int nqt) {
 
   // epilogue: lane (q, g) holds O^T[16db + 4g + j][q]
   const float l_tot = quad_sum(l_run);
-  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+  const float inv = l_tot > 0.0f ? keep_scale / l_tot : 0.0f;
   if (qi < SQ) {
     float* orow = Og + (long long)qi * p.sO.s + 4 * g;
 #pragma unroll

@@ -347,8 +347,9 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
   const float pa1 = 0.9999995735192077f * lcap, pa3 = -0.3332972661781136f * lcap;
   const float pa5 = 0.1325057420337534f * lcap, pa7 = -0.046826030150687044f * lcap;
   const float aslope2 = aslope * kLog2e;
-  // dropout: probabilities are scaled after the row sum, O = sum z p V / sum p
+  // dropout: O = sum z p V / sum p; z is 0 or 1 / (1 - p), a factor of the epilogue
   const float keep_scale = DROP ? 1.0f / (1.0f - p.dropout_p) : 1.0f;
+  const uint32_t drop_bound = DROP ? dropout_bound(p.dropout_p) : 0u;
   // masked tiles: the lane's 16 keys of 32-key block jb sit at offsets 8*(r/4) + r%4 from
   // kb + 4*hh + 32*jb; the word has bit o set iff offset o is inside the row's interval
   // [rlo, rlo + rspan), so each score takes one bit extract and one bitfield insert (the
@@ -443,6 +444,11 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
     // fp16 backward rebuilt (its dQ/dK error against exact gradients rose from 3.7e-4 to 5.5e-4
     // on short causal rows). Dropout scales the probabilities after the sum either way.
     constexpr bool kPairSum = false;
+    uint32_t keep = 0u;  // bit 16*jb + r: score s[jb][r] is kept
+    static_assert(!DROP || C::NB <= 2, "one word of keep bits per tile");
+    if constexpr (DROP)
+      keep = dropout_bits<16 * C::NB>(p.philox_seed, ((uint64_t)h * SQ + qi) * SK + kq, C::BC, drop_bound,
+                                      [](int i) { return (uint64_t)(32 * (i >> 4) + 8 * ((i >> 2) & 3) + (i & 3)); });
     float r0 = 0.0f, r1 = 0.0f;
 #pragma unroll
     for (int jb = 0; jb < C::NB; jb++)
@@ -452,12 +458,7 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
         for (int e = 0; e < 8; e++) {
           const float x = s[jb][8 * sh + e];
           const float pe = FEAT ? exp2_fast(x - m_use) : exp2_fast(fmaf(x, c_log2, -m_use));
-          float pz = pe;
-          if constexpr (DROP) {
-            const int r = 8 * sh + e, key = kq + 32 * jb + 8 * (r >> 2) + (r & 3);
-            pz *= dropout_z(p.philox_seed, ((uint64_t)h * SQ + qi) * SK + key, p.dropout_p, keep_scale);
-          }
-          pb[2 * jb + sh][e] = (T)pz;
+          pb[2 * jb + sh][e] = (T)(DROP ? dropout_keep(pe, keep, 16 * jb + 8 * sh + e) : pe);
           if (!kPairSum) (e & 1 ? r1 : r0) += pe;
         }
     if (kPairSum) {
@@ -748,7 +749,7 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
   for (int i = 0; i < QB; i++) {
     const int qi = qw + 32 * i + l32;
     const float l_tot = half_sum(l_run[i]);
-    const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+    const float inv = l_tot > 0.0f ? keep_scale / l_tot : 0.0f;
     if (sp.n > 1) {
       const long long r = (long long)split * sp.rows + (long long)w * C::BR + (qi - qb);
 #pragma unroll

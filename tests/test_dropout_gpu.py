@@ -105,6 +105,32 @@ def test_forward_mask_varlen_per_sequence():
         assert np.array_equal(dropped, z == 0), f"sequence {i}"
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_forward_mask_past_32_bits(dt):
+    """Counters around 2^32 (64 heads x 17 rows x 2^22 + 100 keys): rows whose high counter word
+    is 0, 1, and the one where a lane's scores lie on both sides. Scores are all equal, and only
+    the 8 keys around 2^32 of that row have a value (a column each), so a zero is a drop."""
+    import torch
+
+    from fable_attn import _C
+    H, SQ, SK, D, p = 64, 17, (1 << 22) + 100, 8, 0.3
+    row, key = divmod(1 << 32, SK)
+    print(f"[dropout-mask] past 2^32 {dt}", flush=True)
+    t = {"bf16": torch.bfloat16, "f32": torch.float32}[dt]   # (bf16: a probability of 2^-22 stays normal)
+    q = torch.zeros(1, H, SQ, D, device="cuda", dtype=t)
+    k = torch.zeros(1, 1, SK, D, device="cuda", dtype=t)
+    v = torch.zeros(1, 1, SK, D, device="cuda", dtype=t)
+    first = key - 4
+    v[0, 0, first:first + 8] = torch.eye(8, device="cuda", dtype=t)
+    out, _ = _C.fwd(q, k, v, 1.0, False, -1, -1, 0.0, None, p, SEED)
+    torch.cuda.synchronize()
+    o = out[0].float().cpu().numpy().reshape(H * SQ, D)
+    pf = float(np.float32(p))
+    for r in (0, 5, row - 1, row, row + 1, H * SQ - 1):
+        want = [orc.oracle_drop_mul(SEED, r * SK + first + j, pf) == 0 for j in range(8)]
+        assert np.array_equal(o[r] == 0, np.array(want)), f"row {r}"
+
+
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 def test_forward_dropout_vs_oracle(case, dt):
