@@ -2,6 +2,8 @@
 // the fp16/bf16 kernels (bwd.hip) and the fp32 kernels (bwd_f32.hip). Mask contract and math of
 // the reference backward (kernels/backward.hip:109-202, FableBwdParams in include/fable_attn_abi.h).
 #pragma once
+#include <type_traits>
+
 #include "attn_device.hpp"
 
 namespace fa {
@@ -43,17 +45,29 @@ __device__ __forceinline__ void query_range_b(const FableBwdParams& p, int k0, i
   }
 }
 
+// Logit transforms of a FEAT kernel, one per step loop, chosen by a uniform switch outside it
+// (bwd_with_mode): plain (windows, dropout), alibi, softcap (alibi too, with slope 0 where there
+// is none). With the flags tested inside the loop, every score of every window or dropout call
+// went through the alibi term, two uniform branches and the mask: encoder layers with dropout
+// (B32 S509 H16 D64 fp16, interior tiles mostly) ran the pair dK/dV kernel in 625 us, now 360.
+enum : int { kBwdPlain = 0, kBwdAlibi = 1, kBwdCap = 2 };
+template <bool FEAT, typename F>
+__device__ __forceinline__ void bwd_with_mode(const FableBwdParams& p, F&& f) {
+  if constexpr (FEAT) {
+    if (p.softcap > 0.0f) return f(std::integral_constant<int, kBwdCap>{});
+    if (p.alibi) return f(std::integral_constant<int, kBwdAlibi>{});
+  }
+  f(std::integral_constant<int, kBwdPlain>{});
+}
+
 // logit transform of one score: returns log2-domain logit, and d(logit)/d(scale*q.k)
-template <bool FEAT>
+template <int MODE>
 __device__ __forceinline__ float bwd_logit2(const FableBwdParams& p, float s, float c_log2, float slope, int q,
                                             int key, float& deriv) {
-  if (!FEAT) {
-    deriv = 1.0f;
-    return s * c_log2;
-  }
-  float x = s * p.scale;
   deriv = 1.0f;
-  if (p.softcap > 0.0f) {
+  if constexpr (MODE == kBwdPlain) return s * c_log2;
+  float x = s * p.scale;
+  if constexpr (MODE == kBwdCap) {
     // (the reciprocal is uniform: one division per call site after hoisting, not per score)
     const float t = tanh_exp(x * (1.0f / p.softcap));
     x = p.softcap * t;
@@ -61,6 +75,19 @@ __device__ __forceinline__ float bwd_logit2(const FableBwdParams& p, float s, fl
   }
   x += slope * (float)(key - q);
   return x * kLog2e;
+}
+
+// whether some query of [q0, q0 + nq) does not see some key of [k0, k0 + nk) (or lies past the
+// sequence): only such tiles run the mask code
+template <bool CAUSAL, bool FEAT>
+__device__ __forceinline__ bool edge_tile_b(const FableBwdParams& p, int q0, int nq, int k0, int nk, int delta, int SQ, int SK) {
+  bool e = q0 + nq > SQ || k0 + nk > SK;
+  if (CAUSAL) e = e || k0 + nk - 1 > q0 + delta;
+  if (FEAT) {
+    e = e || (p.win_left >= 0 && k0 < q0 + nq - 1 + delta - p.win_left);
+    e = e || (p.win_right >= 0 && k0 + nk - 1 > q0 + delta + p.win_right);
+  }
+  return e;
 }
 
 // Lengths and first packed rows of sequence b (dense: the whole [SQ, SK] and row 0; varlen:

@@ -194,25 +194,27 @@ bwd_dq_kernel(FableBwdParams p, int nqt) {
           s[jb] = Dt<T>::mma32(*(const V8*)(ks + off), qreg[ds], s[jb]);
           dp[jb] = Dt<T>::mma32(*(const V8*)(vs + off), doreg[ds], dp[jb]);
         }
-      const bool edge = FEAT || (CAUSAL ? (kb + C::BC - 1 > qw + delta) : (kb + C::BC > SK));
+      const bool edge = edge_tile_b<CAUSAL, FEAT>(p, qw, 32, kb, C::BC, delta, SQ, SK);
       const int kq = kb + 4 * hh;
       uint32_t keep = 0u;  // bit 16*jb + r: score s[jb][r] is kept
       static_assert(!DROP || C::NB <= 2, "one word of keep bits per tile");
       if constexpr (DROP)
         keep = dropout_bits<16 * C::NB>(p.drop_seed, ((uint64_t)h * SQ + qi) * SK + kq, C::BC, drop_bound,
                                         [](int i) { return (uint64_t)(32 * (i >> 4) + 8 * ((i >> 2) & 3) + (i & 3)); });
+      bwd_with_mode<FEAT>(p, [&](auto mode) {
 #pragma unroll
-      for (int jb = 0; jb < C::NB; jb++)
+        for (int jb = 0; jb < C::NB; jb++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int key = kq + jb * 32 + 8 * (r >> 2) + (r & 3);
-          float deriv;
-          const float x = bwd_logit2<FEAT>(p, s[jb][r], c_log2, slope, qi, key, deriv);
-          float pr = exp2_fast(x - lse2);
-          if (edge && !visible_b<CAUSAL, FEAT>(p, qi, key, delta, SQ, SK)) pr = 0.0f;
-          const float z = DROP ? dropout_keep(p.keep_scale, keep, 16 * jb + r) : 1.0f;
-          s[jb][r] = pr * (z * dp[jb][r] - Di) * deriv;  // dS^T (backward.hip:170-176)
-        }
+          for (int r = 0; r < 16; r++) {
+            const int key = kq + jb * 32 + 8 * (r >> 2) + (r & 3);
+            float deriv;
+            const float x = bwd_logit2<decltype(mode)::value>(p, s[jb][r], c_log2, slope, qi, key, deriv);
+            float pr = exp2_fast(x - lse2);
+            if (edge && !visible_b<CAUSAL, FEAT>(p, qi, key, delta, SQ, SK)) pr = 0.0f;
+            const float z = DROP ? dropout_keep(p.keep_scale, keep, 16 * jb + r) : 1.0f;
+            s[jb][r] = pr * (z * dp[jb][r] - Di) * deriv;  // dS^T (backward.hip:170-176)
+          }
+      });
       V8 pb[C::NG];
 #pragma unroll
       for (int jb = 0; jb < C::NB; jb++)
@@ -406,29 +408,31 @@ bwd_dkdv_kernel(FableBwdParams p, int nkt) {
         dp = Dt<T>::mma32(*(const V8*)(dos + off), vreg[ds], dp);
       }
       // s[r] is query qt0 + 8*(r/4) + 4*hh + (r%4), key `key`
-      const bool edge = FEAT || (CAUSAL ? (kw + 31 > qt0 + delta) : false) || qt0 + C::BQ > SQ || kw + 32 > SK;
+      const bool edge = edge_tile_b<CAUSAL, FEAT>(p, qt0, C::BQ, kw, 32, delta, SQ, SK);
       V8 pP[2], pS[2];
       uint32_t keep = 0u;  // bit r: score s[r] is kept
       if constexpr (DROP)
         keep = dropout_bits<16>(p.drop_seed, ((uint64_t)h * SQ + qt0 + 4 * hh) * SK + key, (uint64_t)C::BQ * SK, drop_bound,
                                 [&](int i) { return (uint64_t)(8 * (i >> 2) + (i & 3)) * SK; });
+      bwd_with_mode<FEAT>(p, [&](auto mode) {
 #pragma unroll
-      for (int rq = 0; rq < 4; rq++) {
-        const f32x4 l4 = *(const f32x4*)&rowv[stage][0][8 * rq + 4 * hh];
-        const f32x4 d4 = *(const f32x4*)&rowv[stage][1][8 * rq + 4 * hh];
+        for (int rq = 0; rq < 4; rq++) {
+          const f32x4 l4 = *(const f32x4*)&rowv[stage][0][8 * rq + 4 * hh];
+          const f32x4 d4 = *(const f32x4*)&rowv[stage][1][8 * rq + 4 * hh];
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const int r = 4 * rq + c, q = qt0 + 8 * rq + 4 * hh + c;
-          float deriv;
-          const float x = bwd_logit2<FEAT>(p, s[r], c_log2, slope, q, key, deriv);
-          float pr = exp2_fast(x - l4[c]);
-          if (edge && !visible_b<CAUSAL, FEAT>(p, q, key, delta, SQ, SK)) pr = 0.0f;
-          const float z = DROP ? dropout_keep(p.keep_scale, keep, r) : 1.0f;
-          const float dsv = pr * (z * dp[r] - d4[c]) * deriv;
-          pP[r >> 3][r & 7] = (T)(z * pr);
-          pS[r >> 3][r & 7] = (T)dsv;
+          for (int c = 0; c < 4; c++) {
+            const int r = 4 * rq + c, q = qt0 + 8 * rq + 4 * hh + c;
+            float deriv;
+            const float x = bwd_logit2<decltype(mode)::value>(p, s[r], c_log2, slope, q, key, deriv);
+            float pr = exp2_fast(x - l4[c]);
+            if (edge && !visible_b<CAUSAL, FEAT>(p, q, key, delta, SQ, SK)) pr = 0.0f;
+            const float z = DROP ? dropout_keep(p.keep_scale, keep, r) : 1.0f;
+            const float dsv = pr * (z * dp[r] - d4[c]) * deriv;
+            pP[r >> 3][r & 7] = (T)(z * pr);
+            pS[r >> 3][r & 7] = (T)dsv;
+          }
         }
-      }
+      });
       if constexpr (DSW) {  // the dS tile (32 queries x this wave's 32 keys), streaming stores
         if (dpass == 0) {
           T* dst = ds_cur + 16 * l32 + 8 * hh;
@@ -761,7 +765,7 @@ __device__ __forceinline__ void bwd_pair_item(const FableBwdParams& p, int nkt, 
     }
   };
   // S-wave step `it` (set S holds tile it, stored an iteration ago): S, P, dV += dO^T . P
-  auto s_step = [&](auto set, int it) {
+  auto s_step = [&](auto mode, auto set, int it) {
     constexpr int S = decltype(set)::value;
     gload(set);
     const int st = it & 3, hg = w_hg, qt0 = qstart + w_qi * C::BQ;
@@ -769,7 +773,7 @@ __device__ __forceinline__ void bwd_pair_item(const FableBwdParams& p, int nkt, 
     const float slope = (FEAT && p.alibi) ? p.alibi[kvh * p.gqa + hg] : 0.0f;
     const T* qs = lds + st * C::STAGE;
     const f32x16 sv = rowprod(qs);
-    const bool edge = FEAT || (CAUSAL && kw + 31 > qt0 + delta) || qt0 + C::BQ > SQ || kw + 32 > SK;
+    const bool edge = edge_tile_b<CAUSAL, FEAT>(p, qt0, C::BQ, kw, 32, delta, SQ, SK);
     // probabilities; on an edge tile (one uniform branch, no per-score branches) the scores a
     // query does not see are zeroed
     float pr[16], dv[16];
@@ -779,7 +783,7 @@ __device__ __forceinline__ void bwd_pair_item(const FableBwdParams& p, int nkt, 
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         const int r = 4 * rq + c, q = qt0 + 8 * rq + 4 * hh + c;
-        const float x = bwd_logit2<FEAT>(p, sv[r], c_log2, slope, q, key, dv[r]);
+        const float x = bwd_logit2<decltype(mode)::value>(p, sv[r], c_log2, slope, q, key, dv[r]);
         pr[r] = exp2_fast(x - l4[c]);
       }
     }
@@ -878,8 +882,10 @@ __device__ __forceinline__ void bwd_pair_item(const FableBwdParams& p, int nkt, 
         for_sets(std::make_integer_sequence<int, NSET>{}, [&](auto set) { d_step(set, it + decltype(set)::value); });
       tprod(lds + ((it - 2) & 3) * C::STAGE, pS);  // the last step's tile (it-1 was the last step)
     } else {
-      for (int it = 0; it <= total; it += NSET)
-        for_sets(std::make_integer_sequence<int, NSET>{}, [&](auto set) { s_step(set, it + decltype(set)::value); });
+      bwd_with_mode<FEAT>(p, [&](auto mode) {
+        for (int it = 0; it <= total; it += NSET)
+          for_sets(std::make_integer_sequence<int, NSET>{}, [&](auto set) { s_step(mode, set, it + decltype(set)::value); });
+      });
     }
   }
   const float sc = dpw ? p.scale : 1.0f;

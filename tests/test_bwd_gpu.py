@@ -269,3 +269,22 @@ def test_backward_query_split_taken():
         bk = 128 if (D + 31) // 32 * 32 == 128 else 64      # keys per pair-kernel workgroup
         share = 2 * B * Hk * -(-SK // bk) * bk * D * 4       # dK and dV rows of every work item
         assert extra > 0 and extra % share == 0 and extra // share >= 2, (name, got, extra)
+
+
+# Feature calls long enough to hold tiles that every row sees in full (they run without mask code)
+# beside edge tiles, at both sides of the window's and the sequence's edges.
+INTERIOR = [
+    ("interior window (150,70) D64", 1, 2, 2, 333, 301, 64, False, 150, 70, 0.0, False),
+    ("interior window (127,0) D128", 1, 2, 1, 290, 290, 128, True, 127, 0, 0.0, False),
+    ("interior window (-1,33) D160", 1, 2, 1, 200, 264, 160, False, -1, 33, 0.0, False),
+    ("interior alibi+softcap D96", 1, 2, 2, 161, 224, 96, False, -1, -1, 15.0, True),
+    ("interior alibi causal D192", 1, 2, 2, 160, 192, 192, True, -1, -1, 0.0, True),
+]
+
+
+@pytest.mark.parametrize("path", list(PATHS))
+@pytest.mark.parametrize("case", INTERIOR, ids=[c[0] for c in INTERIOR])
+def test_backward_interior_tiles(case, path):
+    print(f"[bwd] {case[0]} {path}", flush=True)
+    res, ref, model = run(case, "bf16", path=path)
+    check_grads("bwd_" + path, case[0], "bf16", res[0], ref, model)
