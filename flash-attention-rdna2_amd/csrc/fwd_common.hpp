@@ -91,6 +91,58 @@ struct FwdSplit {
   float* lse;      // [n][rows], natural log; -inf where a split saw no key of the row
 };
 
+// K/V in pages of a cache (fwd_kernel with PGT = FwdPaged): row j of sequence z is row
+// j % page of page table[z][j / page]; p.sK / p.sV give the row and head strides, kpg / vpg the
+// page strides. The q heads that share a K/V head are packed into the rows of a query tile: row
+// r of a (sequence, K/V head) is token r / gqa, head r % gqa of the group, so each K/V row is
+// read once for the whole group.
+//  * ctx null: packed prompts; cu_q / cu_k / seqused as in the varlen forward.
+//  * ctx set: p.SQ new tokens per sequence, token t at position ctx[z] + t; the cache holds
+//    ctx[z] keys, and the new tokens' own when `append` (then p.causal is set).
+struct FwdPaged {
+  const int* table;      // [batch][max_blocks]
+  int max_blocks, page_shift;
+  long long kpg, vpg;    // elements
+  const int* ctx;        // cached keys per sequence, or null
+  int append;
+  const int* leftpad;    // first visible key per sequence, or null
+  const void* qlo;       // ROT: the low parts of the rotated q (p.Q holds the high parts)
+  long long lse_sq;      // LSE stride of a query (1: packed prompts)
+};
+struct NoPaged {};
+
+// lengths, key position of query 0 and row-0 offsets of sequence z (as seq_view; delta need not
+// be SK - SQ here: new tokens that are not in the cache follow its last key)
+struct PagedView {
+  int SQ, SK, delta;
+  long long q0, o0, lse0;
+};
+__device__ __forceinline__ PagedView paged_view(const FableFwdParams& p, const FwdPaged& pg, int z) {
+  PagedView v;
+  const int room = (int)min((long long)pg.max_blocks << pg.page_shift, 0x7FFFFFFFLL);
+  if (pg.ctx) {
+    const int c = pg.ctx[z];
+    v.SQ = p.SQ;
+    v.delta = c;
+    v.SK = max(min(c + (pg.append ? p.SQ : 0), room), 0);
+    v.q0 = (long long)z * p.sQ.b;
+    v.o0 = (long long)z * p.sO.b;
+    v.lse0 = (long long)z * p.lse_sb;
+  } else {
+    const int qs = p.cu_q[z];
+    v.SQ = p.cu_q[z + 1] - qs;
+    v.SK = p.cu_k[z + 1] - p.cu_k[z];
+    if (p.seqused_q) v.SQ = min(v.SQ, p.seqused_q[z]);
+    if (p.seqused_k) v.SK = p.seqused_k[z];
+    v.SK = min(v.SK, room);
+    v.delta = v.SK - v.SQ;
+    v.q0 = (long long)qs * p.sQ.s;
+    v.o0 = (long long)qs * p.sO.s;
+    v.lse0 = qs;
+  }
+  return v;
+}
+
 // A launch request: the caller's workspace for a key split (null / too small: no split), or a
 // query for the bytes a split of this call would use (nothing is launched).
 struct FwdWs {
@@ -111,7 +163,17 @@ int launch_fwd_d192(const FableFwdParams& p, int dtype, hipStream_t st, FwdWs& w
 int launch_fwd_d224(const FableFwdParams& p, int dtype, hipStream_t st, FwdWs& ws);
 int launch_fwd_d256(const FableFwdParams& p, int dtype, hipStream_t st, FwdWs& ws);
 int launch_fwd_f32(const FableFwdParams& p, hipStream_t st);
+// the fp16/bf16 forward over a paged cache (fwd_paged_d64/d128/d256.hip: kernel widths 64, 128
+// and 256), pages of at least 16 rows; rot: p.Q / pg.qlo are the two parts of a rotated q
+int launch_fwd_paged_d64(const FableFwdParams& p, const FwdPaged& pg, int dtype, bool rot, hipStream_t st, FwdWs& ws);
+int launch_fwd_paged_d128(const FableFwdParams& p, const FwdPaged& pg, int dtype, bool rot, hipStream_t st, FwdWs& ws);
+int launch_fwd_paged_d256(const FableFwdParams& p, const FwdPaged& pg, int dtype, bool rot, hipStream_t st, FwdWs& ws);
+inline int launch_fwd_paged(const FableFwdParams& p, const FwdPaged& pg, int dtype, bool rot, hipStream_t st, FwdWs& ws) {
+  return p.HD <= 64 ? launch_fwd_paged_d64(p, pg, dtype, rot, st, ws)
+                    : (p.HD <= 128 ? launch_fwd_paged_d128(p, pg, dtype, rot, st, ws) : launch_fwd_paged_d256(p, pg, dtype, rot, st, ws));
+}
 // merge of the key-split partials (fwd.hip)
 int launch_fwd_split_combine(const FableFwdParams& p, int dtype, const FwdSplit& sp, hipStream_t st);
+int launch_fwd_split_combine_paged(const FableFwdParams& p, const FwdPaged& pg, int dtype, const FwdSplit& sp, hipStream_t st);
 
 }  // namespace fa

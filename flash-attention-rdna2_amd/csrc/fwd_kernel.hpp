@@ -61,10 +61,23 @@ struct FwdCfg {
   static_assert(HD % 32 == 0 && BC % 32 == 0, "shape");
 };
 
-template <typename T, class C, bool CAUSAL, bool FEAT, bool DROP = false>
+// (the fields of a paged instance's argument; constants for the others)
+__device__ __forceinline__ int paged_leftpad(const FwdPaged& pg, int z) { return pg.leftpad ? max(pg.leftpad[z], 0) : 0; }
+__device__ __forceinline__ int paged_leftpad(const NoPaged&, int) { return 0; }
+__device__ __forceinline__ bool pg_ctx(const FwdPaged& pg) { return pg.ctx != nullptr; }
+__device__ __forceinline__ bool pg_ctx(const NoPaged&) { return false; }
+__device__ __forceinline__ long long paged_lse(const FwdPaged& pg, int t) { return (long long)t * pg.lse_sq; }
+__device__ __forceinline__ long long paged_lse(const NoPaged&, int) { return 0; }
+
+// PGT = FwdPaged: K/V in the pages of a cache (fwd_common.hpp); causal is then the run-time
+// p.causal (CAUSAL false). ROT: q comes in two parts whose sum the scores take (a rotated q is not
+// representable in T), at the price of a second S product.
+template <typename T, class C, bool CAUSAL, bool FEAT, bool DROP = false, class PGT = NoPaged, bool ROT = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(C::NT, C::NT),
                           amdgpu_waves_per_eu(C::WPE, C::WPE))) void
-fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
+fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
+  constexpr bool PG = std::is_same<PGT, FwdPaged>::value;
+  static_assert(!PG || (!CAUSAL && !DROP), "paged instances");
   using V8 = typename Dt<T>::V8;
   using V4 = typename Dt<T>::V4;
   // K/V rings of NST stages, a barrier every BP tiles. Iteration t reads K tile t+1 and V tile t
@@ -91,17 +104,27 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
   // u-major kept 1.04-1.17x there)
   const int umax = (CAUSAL && !FEAT && C::HD <= 128 && !p.cu_q) ? (p.SK <= 2048 ? kFwdUMajorCausal : kFwdUMajorCausal / 2)
                                                                 : kFwdUMajor;
-  const int w = xcd_group_remap(blockIdx.x - split * nitems, nitems, nqt, p.gqa, umax);
+  // (PG: items are (sequence, K/V head, tile of packed rows); h is the group's first q head)
+  const int gp = PG ? p.gqa : 1, nheads = p.NH / gp;
+  const int w = xcd_group_remap(blockIdx.x - split * nitems, nitems, nqt, PG ? 1 : p.gqa, umax);
   const int qti = w % nqt, zh = w / nqt;
-  const int h = zh % p.NH, z = zh / p.NH;
-  const int qt = CAUSAL ? (nqt - 1 - qti) : qti;
+  const int h = (zh % nheads) * gp, z = zh / nheads;
+  const int qt = (PG ? p.causal != 0 : CAUSAL) ? (nqt - 1 - qti) : qti;
   const int kvh = h / p.gqa;
 
-  const SeqView sv = seq_view(p, z, h);
+  SeqView sv;
+  int delta;
+  if constexpr (PG) {
+    const PagedView v = paged_view(p, pg, z);
+    sv = SeqView{v.SQ * gp, v.SK, v.q0, 0, 0, v.o0, v.lse0};  // SQ: packed rows
+    delta = v.delta;
+  } else {
+    sv = seq_view(p, z, h);
+    delta = sv.SK - sv.SQ;
+  }
   const int SQ = sv.SQ, SK = sv.SK;
   const int qb = qt * C::BR;
   if (qb >= SQ) return;
-  const int delta = SK - SQ;
 
   const T* Qg = (const T*)p.Q + sv.q0 + (long long)h * p.sQ.h;
   const T* Kg = (const T*)p.K + sv.k0 + (long long)kvh * p.sK.h;
@@ -110,12 +133,34 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
 
   // ---- block and wave key ranges
   constexpr int QB = C::QB;
+  static_assert(!PG || QB == 1, "paged instances");
+  const int lpad = PG && FEAT ? paged_leftpad(pg, z) : 0;
+  // keys visible to rows [r0, r1]
+  auto range = [&](int r0, int r1, int& k0, int& k1) {
+    if constexpr (PG) {
+      if (p.causal)
+        key_range<true, FEAT>(p, r0 / gp, r1 / gp, delta, SK, k0, k1);
+      else
+        key_range<false, FEAT>(p, r0 / gp, r1 / gp, delta, SK, k0, k1);
+      k0 = max(k0, lpad);
+    } else {
+      key_range<CAUSAL, FEAT>(p, r0, r1, delta, SK, k0, k1);
+    }
+  };
   int bk0, bk1;
-  key_range<CAUSAL, FEAT>(p, qb, min(qb + C::BR, SQ) - 1, delta, SK, bk0, bk1);
+  range(qb, min(qb + C::BR, SQ) - 1, bk0, bk1);
   const int qw = qb + wave * 32 * QB;  // first row of this wave; block i = rows qw+32i..+31
   const bool wave_rows = qw < SQ;
   int wk0 = 0, wk1 = 0;
-  if (wave_rows) key_range<CAUSAL, FEAT>(p, qw, min(qw + 32 * QB, SQ) - 1, delta, SK, wk0, wk1);
+  if (wave_rows) range(qw, min(qw + 32 * QB, SQ) - 1, wk0, wk1);
+  // PG: this lane's token and head within the group, and the end of its visible keys
+  int ptok = 0, phead = 0, pend = 0;
+  if constexpr (PG) {
+    const int r = qw + l32;
+    ptok = r / gp;
+    phead = r - ptok * gp;
+    pend = p.causal ? min(SK, ptok + delta + 1) : SK;
+  }
   int kstart = (bk0 / C::BC) * C::BC;
   int ntiles = bk1 > bk0 ? (bk1 - kstart + C::BC - 1) / C::BC : 0;
   if (sp.n > 1) {  // this workgroup's share of the key tiles: a contiguous run of them
@@ -130,16 +175,21 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
   // p.HD..C::HD-1 in Q, K and V: they add nothing to q.k, and the O columns they produce are
   // not stored.
   const int HDr = p.HD;
-  V8 qreg[QB][C::NDS];
+  V8 qreg[QB][C::NDS], qlo[ROT ? C::NDS : 1];
 #pragma unroll
   for (int i = 0; i < QB; i++) {
     const int qi = qw + 32 * i + l32;
+    const long long qo = PG ? (long long)ptok * p.sQ.s + (long long)phead * p.sQ.h : (long long)qi * p.sQ.s;
 #pragma unroll
     for (int ds = 0; ds < C::NDS; ds++) {
       if (qi < SQ && 16 * ds + 8 * hh < HDr)
-        qreg[i][ds] = *(const V8*)(Qg + (long long)qi * p.sQ.s + 16 * ds + 8 * hh);
+        qreg[i][ds] = *(const V8*)(Qg + qo + 16 * ds + 8 * hh);
       else
         qreg[i][ds] = bitcast<V8>(u32x4{0, 0, 0, 0});
+      if constexpr (ROT)
+        qlo[ds] = qi < SQ && 16 * ds + 8 * hh < HDr
+                      ? *(const V8*)((const T*)pg.qlo + (Qg - (const T*)p.Q) + qo + 16 * ds + 8 * hh)
+                      : bitcast<V8>(u32x4{0, 0, 0, 0});
     }
   }
 
@@ -169,9 +219,9 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
 #pragma unroll
     for (int i = 0; i < QB; i++) {
       // (64-bit: window and chunk sizes up to INT_MAX must not wrap)
-      const long long qd = qw + 32 * i + l32 + delta;
-      long long lo = 0, hi = SK;
-      if (CAUSAL) hi = min(hi, qd + 1);
+      const long long qd = (long long)(PG ? ptok : qw + 32 * i + l32) + delta;
+      long long lo = lpad, hi = SK;
+      if (PG ? p.causal != 0 : CAUSAL) hi = min(hi, qd + 1);
       if (p.win_left >= 0) lo = max(lo, qd - p.win_left);
       if (p.win_right >= 0) hi = min(hi, qd + p.win_right + 1);
       if (p.attn_chunk > 0) {
@@ -184,13 +234,16 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
     }
   }
   const float c_log2 = p.scale * kLog2e;
-  const float aslope = (FEAT && p.alibi_slopes) ? p.alibi_slopes[h] : 0.0f;
+  const float aslope = (FEAT && p.alibi_slopes) ? p.alibi_slopes[PG ? min(h + phead, p.NH - 1) : h] : 0.0f;
+  // alibi counts from the query's row (its position in the cache for new tokens)
+  const int aq0 = PG && pg_ctx(pg) ? delta : 0;
 
   // leading tiles that every row of the workgroup sees in full: no mask code for them
   int nint = 0;
   if (!FEAT) {
     int lim = SK;
     if (CAUSAL) lim = min(lim, qb + delta + 1);
+    if (PG && p.causal) lim = min(lim, qb / gp + delta + 1);
     nint = min(max((lim - kstart) / C::BC, 0), ntiles);
   }
 
@@ -232,14 +285,67 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
   const T* k_cur = Kg + (long long)kstart * p.sK.s;
   const T* v_cur = Vg + (long long)kstart * p.sV.s;
   long long k_left = (long long)(kvalid - kstart) * p.sK.s * 2, v_left = (long long)(kvalid - kstart) * p.sV.s * 2;
+  // PG: the rows of one wave's load (64 / DCH of them, at most 16) lie in one page. The page of
+  // each load of the next K tile is fetched a tile ahead by a vector load (a scalar one would
+  // share its counter with the LDS reads), and made uniform when the K tile is loaded; the V
+  // tile, one behind, takes the entries its K tile used.
+  constexpr int NE = PG ? C::KJ : 1;
+  static_assert(!PG || (kRowStep && 64 % C::DCH == 0 && 64 / C::DCH <= 16), "paged loads");
+  int ent[NE], ekey = kstart, pg_cur[NE], pg_prev[NE];  // next K tile's entries and first key
+  const int wrow = tid / 64 * (64 / C::DCH);            // first row of the wave's first load
+  auto pg_fetch = [&]() {
+    if constexpr (PG) {
+#pragma unroll
+      for (int j = 0; j < NE; j++)
+        ent[j] = pg.table[(long long)z * pg.max_blocks + (min(ekey + wrow + j * RSTEP, kvalid - 1) >> pg.page_shift)];
+    }
+  };
+  auto pg_load = [&](u32x4 (&ld)[C::KJ], const T* base, int key0, const int (&page)[NE], long long spg, long long srow,
+                     const int (&off)[C::KJ]) {
+    if constexpr (PG) {
+#pragma unroll
+      for (int j = 0; j < NE; j++) {
+        const int key = __builtin_amdgcn_readfirstlane(key0 + wrow + j * RSTEP);
+        const int in = key & ((1 << pg.page_shift) - 1);
+        const auto r = buf_rsrc(base + page[j] * spg + in * srow, (long long)(kvalid - key) * srow * 2);
+        ld[j] = buf_load16(r, off[j]);
+      }
+    }
+  };
+  if constexpr (PG) {
+    // (offsets within the wave's rows: the descriptor starts at the wave's first row)
+#pragma unroll
+    for (int j = 0; j < C::KJ; j++) {
+      const int r = lane / C::DCH, c = tid % C::DCH;
+      koff[j] = 8 * c < HDr ? r * (int)(p.sK.s * 2) + 16 * c : kBufZero;
+      voff[j] = 8 * c < HDr ? r * (int)(p.sV.s * 2) + 16 * c : kBufZero;
+    }
+    if (ntiles > 0) pg_fetch();
+  }
   auto gload_k = [&]() {
+    if constexpr (PG) {
+#pragma unroll
+      for (int j = 0; j < NE; j++) {
+        pg_prev[j] = pg_cur[j];
+        pg_cur[j] = __builtin_amdgcn_readfirstlane(ent[j]);
+      }
+      pg_load(ldk, Kg, ekey, pg_cur, pg.kpg, p.sK.s, koff);
+      ekey += C::BC;
+      pg_fetch();
+      return;
+    }
     const auto r = buf_rsrc(k_cur, k_left);
 #pragma unroll
     for (int j = 0; j < C::KJ; j++) ldk[j] = buf_load16(r, koff[j]);
     k_cur += k_step;
     k_left -= 2 * k_step;
   };
-  auto gload_v = [&]() {
+  // (PG: `ahead` K tiles have been loaded past this V tile, 0 or 1)
+  auto gload_v = [&](int ahead = 1) {
+    if constexpr (PG) {
+      pg_load(ldv, Vg, ekey - (1 + ahead) * C::BC, ahead ? pg_prev : pg_cur, pg.vpg, p.sV.s, voff);
+      return;
+    }
     const auto r = buf_rsrc(v_cur, v_left);
 #pragma unroll
     for (int j = 0; j < C::KJ; j++) ldv[j] = buf_load16(r, voff[j]);
@@ -291,7 +397,10 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
 #pragma unroll
             for (int jb = 0; jb < C::NB; jb++)
 #pragma unroll
-              for (int i = 0; i < QB; i++) s[i][jb] = Dt<T>::mma32(a[ds][jb], qreg[i][d0 + ds], s[i][jb]);
+              for (int i = 0; i < QB; i++) {
+                s[i][jb] = Dt<T>::mma32(a[ds][jb], qreg[i][d0 + ds], s[i][jb]);
+                if constexpr (ROT) s[i][jb] = Dt<T>::mma32(a[ds][jb], qlo[d0 + ds], s[i][jb]);
+              }
       }
     } else {
 #pragma unroll
@@ -300,7 +409,10 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
         for (int jb = 0; jb < C::NB; jb++) {
           const V8 a = *(const V8*)(kp + jb * 32 * C::KSTR + 16 * ds);
 #pragma unroll
-          for (int i = 0; i < QB; i++) s[i][jb] = Dt<T>::mma32(a, qreg[i][ds], s[i][jb]);
+          for (int i = 0; i < QB; i++) {
+            s[i][jb] = Dt<T>::mma32(a, qreg[i][ds], s[i][jb]);
+            if constexpr (ROT) s[i][jb] = Dt<T>::mma32(a, qlo[ds], s[i][jb]);
+          }
         }
     }
   };
@@ -378,7 +490,7 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
     }
     if constexpr ((decltype(cap)::value & 2) != 0) {
       const int key = kb + 4 * hh + jb * 32 + 8 * (r >> 2) + (r & 3);
-      x = fmaf(aslope2, (float)(key - (qw + 32 * i + l32)), x);
+      x = fmaf(aslope2, (float)(key - (PG ? ptok + aq0 : qw + 32 * i + l32)), x);
     }
     if constexpr (decltype(masked)::value) {
       const unsigned keep = (unsigned)__builtin_amdgcn_sbfe((int)vis, 8 * (r >> 2) + (r & 3), 1);
@@ -409,7 +521,7 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           const int key = kq + jb * 32 + 8 * (r >> 2) + (r & 3);
-          const bool ok = CAUSAL ? (key < SK && key <= qi + delta) : key < SK;
+          const bool ok = PG ? key < pend : (CAUSAL ? (key < SK && key <= qi + delta) : key < SK);
           if (!ok) s[jb][r] = -INFINITY;
         }
     }
@@ -481,9 +593,9 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
   // always takes the masked path
   auto interior = [&](int t) {
     const int kb = kstart + t * C::BC, ke = kb + C::BC - 1;
-    const int r0 = qw + delta, r1 = qw + 32 * QB - 1 + delta;
-    bool ok = ke < SK && p.attn_chunk <= 0;
-    if (CAUSAL) ok = ok && ke <= r0;
+    const int r0 = qw / gp + delta, r1 = (qw + 32 * QB - 1) / gp + delta;
+    bool ok = ke < SK && p.attn_chunk <= 0 && kb >= lpad;
+    if (PG ? p.causal != 0 : CAUSAL) ok = ok && ke <= r0;
     if (p.win_right >= 0) ok = ok && ke <= r0 + p.win_right;
     if (p.win_left >= 0) ok = ok && kb >= r1 - p.win_left;
     return ok;
@@ -516,8 +628,8 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
   if (ntiles > 0) {
 #pragma unroll
     for (int j = 0; j < BP; j++) {
-      gload_k();  // tile j
-      gload_v();  // tile j
+      gload_k();   // tile j
+      gload_v(0);  // tile j
       lstore_k(j);
       lstore_v(j);
     }
@@ -758,15 +870,63 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
       if (qi < SQ && hh == 0) sp.lse[r] = l_tot > 0.0f ? (m_run[i] + m_base) * kLn2 + __logf(l_tot) : -INFINITY;
       continue;
     }
-    T* orow = Og + (long long)qi * p.sO.s;
+    T* orow = Og + (PG ? (long long)ptok * p.sO.s + (long long)phead * p.sO.h : (long long)qi * p.sO.s);
 #pragma unroll
     for (int db = 0; db < C::NDB; db++)
       store_cblock<T>(orow + db * 32, oacc[i][db], inv, hh, qi < SQ, HDr - db * 32);
     if (qi < SQ) {
       if (p.LSE && hh == 0)
-        p.LSE[sv.lse0 + qi] = l_tot > 0.0f ? (m_run[i] + m_base) * kLn2 + __logf(l_tot) : -INFINITY;
+        p.LSE[PG ? sv.lse0 + (long long)(h + phead) * p.lse_sh + paged_lse(pg, ptok) : sv.lse0 + qi] = l_tot > 0.0f ? (m_run[i] + m_base) * kLn2 + __logf(l_tot) : -INFINITY;
     }
   }
+}
+
+template <class K>
+struct CfgTag {
+  using type = K;
+};
+
+// Launcher of the paged instances: C for the plain masks, CF for the feature masks and for a
+// rotated q. A grid that leaves CUs idle splits the keys of each tile (as fwd_split_count, up
+// to kPagedSplitMax shares of at least kPagedSplitTiles tiles of the longest cache the table holds).
+constexpr int kPagedSplitMax = 32, kPagedSplitTiles = 4;
+template <typename T, class C, class CF>
+static int launch_fwd_pg(const FableFwdParams& p, const FwdPaged& pg, bool rot, hipStream_t st, FwdWs& ws) {
+  const bool feat = p.softcap > 0.0f || p.alibi_slopes != nullptr || p.attn_chunk > 0 || p.win_left >= 0 || pg.leftpad ||
+                    (p.win_right >= 0 && !(p.win_right == 0 && p.causal));
+  auto go = [&](auto cfg, auto ft, auto rt) -> int {
+    using K = typename decltype(cfg)::type;
+    const long long rows_max = (long long)p.SQ * p.gqa;
+    if (rows_max > 0x7FFFFFFF) return fail(FA_ERR_ARG, "fable_attn_fwd: too many rows");
+    const int nqt = (int)((rows_max + K::BR - 1) / K::BR);
+    const long long nblk = (long long)nqt * (p.NH / p.gqa) * p.batch;
+    if (nblk <= 0) return FA_OK;
+    constexpr long long kSlots = 256LL * (4 * K::WPE / K::NW > 0 ? 4 * K::WPE / K::NW : 1);
+    const long long tiles = ((long long)p.SK + K::BC - 1) / K::BC;
+    long long n = kSlots / nblk;
+    n = n < tiles / kPagedSplitTiles ? n : tiles / kPagedSplitTiles;
+    n = n < kPagedSplitMax ? n : kPagedSplitMax;
+    FwdSplit sp{1, nqt, K::BR, 0, nullptr, nullptr};
+    ws.need = 0;
+    if (n >= 2) {
+      const long long rows = nblk * K::BR;
+      const long long obytes = (n * rows * p.HD * 4 + 255) / 256 * 256;
+      ws.need = obytes + n * rows * 4;
+      if (!ws.query && ws.ptr && ws.bytes >= ws.need && ((uintptr_t)ws.ptr & 255) == 0)
+        sp = FwdSplit{(int)n, nqt, K::BR, rows, (float*)ws.ptr, (float*)((char*)ws.ptr + obytes)};
+    }
+    if (ws.query) return FA_OK;
+    if (nblk * sp.n > 0x7FFFFFFF) return fail(FA_ERR_ARG, "fable_attn_fwd: grid too large");
+    hipLaunchKernelGGL((fwd_kernel<T, K, false, decltype(ft)::value, false, FwdPaged, decltype(rt)::value>),
+                       dim3((unsigned)(nblk * sp.n)), dim3(K::NT), 0, st, p, nqt, sp, pg);
+    const int rc = launch_status("fable_attn_fwd (paged)");
+    if (rc != FA_OK || sp.n == 1) return rc;
+    return launch_fwd_split_combine_paged(p, pg, std::is_same<T, _Float16>::value ? FA_F16 : FA_BF16, sp, st);
+  };
+  using Y = std::integral_constant<bool, true>;
+  using N = std::integral_constant<bool, false>;
+  if (rot) return feat ? go(CfgTag<CF>{}, Y{}, Y{}) : go(CfgTag<CF>{}, N{}, Y{});
+  return feat ? go(CfgTag<CF>{}, Y{}, N{}) : go(CfgTag<C>{}, N{}, N{});
 }
 
 // Workgroup shapes per head dim: C (the widest) runs the plain masks (causal / sequence end)
@@ -778,11 +938,6 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp) {
 // over few tiles, so shorter workgroups, more of them per CU, win; CL and CR the plain masks
 // on long and on short causal rows (below, at launch_fwd). Dropout has kernels of its own, so its Philox rounds cost the
 // other features no registers.
-template <class K>
-struct CfgTag {
-  using type = K;
-};
-
 // Key split of a small grid: splits per query tile when the tiles fill at most half the CUs,
 // up to one workgroup per CU, at least kSplitMinTiles key tiles per split, at most 16. A causal
 // grid of one round (at most one workgroup per CU) with rows of kSplitLongRow key tiles or more
@@ -851,7 +1006,7 @@ static int launch_fwd(const FableFwdParams& p, hipStream_t st, FwdWs& ws) {
     if (nblk <= 0) return FA_OK;
     if (nblk * sp.n > 0x7FFFFFFF) return fail(FA_ERR_ARG, "fable_attn_fwd: grid too large");
     hipLaunchKernelGGL((fwd_kernel<T, K, decltype(causal)::value, decltype(ft)::value, decltype(dr)::value>),
-                       dim3((unsigned)(nblk * sp.n)), dim3(K::NT), 0, st, p, nqt, sp);
+                       dim3((unsigned)(nblk * sp.n)), dim3(K::NT), 0, st, p, nqt, sp, NoPaged{});
     const int rc = launch_status("fable_attn_fwd");
     if (rc != FA_OK || sp.n == 1) return rc;
     return launch_fwd_split_combine(p, std::is_same<T, _Float16>::value ? FA_F16 : FA_BF16, sp, st);

@@ -385,23 +385,17 @@ def dec(q, k_cache, v_cache, block_table, cache_seqlens, new_k, new_v, rotary_co
                  f"{n}: contiguous, 16-byte aligned [B, seqlen_q, nheads_k, D] of q's dtype")
     else:
         _req(new_v is None, "new_k and new_v go together")
-    ctx_bound = block_table.shape[1] * page
-    nsplit = int(_L.fa_decode_num_splits(B, NQ, Hq, Hq // Hk, ctx_bound, int(num_splits or 0)))
     out = torch.empty((B, NQ, Hq, D), dtype=q.dtype, device=q.device)
-    # one fp16/bf16 split writes out (and lse) from the partial kernel: no scratch then
-    scratch = (torch.empty((B * NQ * Hq * nsplit * (D + 2),), dtype=torch.float32, device=q.device)
-               if nsplit > 1 or q.dtype == torch.float32 else None)
     lse = (torch.empty((B, NQ, Hq), dtype=torch.float32, device=q.device) if return_lse
            else torch.empty((0,), dtype=torch.float32, device=q.device))
     p = FableDecParams()
     p.q, p.Kc, p.Vc = q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr()
     p.block_table, p.o = block_table.data_ptr(), out.data_ptr()
-    p.scratch = scratch.data_ptr() if scratch is not None else None
     p.ctx_len = cache_seqlens.data_ptr()
     p.cos = rotary_cos.data_ptr() if rotary_cos is not None else None
     p.sin = rotary_sin.data_ptr() if rotary_sin is not None else None
     p.batch, p.NH, p.gqa, p.HD, p.page = B, Hq, Hq // Hk, D, page
-    p.max_blocks, p.nsplit, p.window = block_table.shape[1], nsplit, int(window)
+    p.max_blocks, p.nsplit, p.window = block_table.shape[1], int(num_splits or 0), int(window)
     p.rotary = (2 if rotary_interleaved else 1) if rotary_cos is not None else 0
     p.scale = float(scale)
     p.leftpad = cache_leftpad.data_ptr() if cache_leftpad is not None else None
@@ -410,9 +404,12 @@ def dec(q, k_cache, v_cache, block_table, cache_seqlens, new_k, new_v, rotary_co
     p.alibi = alibi.data_ptr() if alibi is not None else None
     p.nq, p.rotary_dim = NQ, int(rotary_dim)
     p.rotary_pos = rotary_pos.data_ptr() if rotary_pos is not None else None
+    # (split partials, the parts of a rotated q: the library says what this call uses)
+    ws_bytes = int(_L.fable_attn_dec_ws_bytes(p, _dt(q), 1 if new_k is not None else 0))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes > 0 else None
     with _on(q.device):
-        _lib.check(_L.fable_attn_dec(p, _dt(q), _stream(q), _ptr(new_k), _ptr(new_v)),
-                   "fable_attn_dec")
+        _lib.check(_L.fable_attn_dec_ws(p, _dt(q), _ptr(ws), max(ws_bytes, 0), _stream(q), _ptr(new_k),
+                                        _ptr(new_v)), "fable_attn_dec")
     return out, lse
 
 

@@ -71,6 +71,11 @@ class CombineParams(ctypes.Structure):
                 ("in_dtype", c_i32), ("out_dtype", c_i32)]
 
 
+class FablePagedKV(ctypes.Structure):
+    _fields_ = [("block_table", c_ptr), ("max_blocks", c_i32), ("page", c_i32),
+                ("k_page_stride", c_i64), ("v_page_stride", c_i64)]
+
+
 # The reference's layouts (package/csrc/fa_iface.h:9-63), taken by fa_forward_launch,
 # fable_attn_backward_launch and fa_decode_launch.
 class RefStrides(ctypes.Structure):
@@ -119,7 +124,8 @@ STRUCTS = {0: FableFwdParams, 1: FableBwdParams, 2: FableDecParams, 3: CombinePa
 # exported symbols of libfable_attn_hip.so (the C-ABI surface)
 EXPORTS = ("fa_forward_launch", "fable_attn_backward_launch", "fa_decode_launch",
            "fable_attn_fwd", "fable_attn_fwd_ws", "fable_attn_fwd_ws_bytes", "fable_attn_bwd", "fable_attn_dec", "fable_attn_dec_noalloc",
-           "fable_attn_dec_noalloc_max_floats",
+           "fable_attn_dec_noalloc_max_floats", "fable_attn_dec_ws", "fable_attn_dec_ws_bytes",
+           "fable_attn_fwd_paged", "fable_attn_fwd_paged_ws_bytes",
            "fa_decode_num_splits", "fa_combine_launch", "fable_attn_bwd_ds_bytes",
            "fable_attn_abi_version", "fable_attn_struct_size", "fable_attn_last_error")
 
@@ -149,7 +155,13 @@ def load():
     lib.fa_decode_launch.argtypes = [RefDecParams, c_i32, c_ptr, c_ptr, c_ptr]
     lib.fable_attn_dec_noalloc.argtypes = [FableDecParams, c_i32, c_ptr, c_ptr, c_ptr]
     lib.fable_attn_dec_noalloc_max_floats.restype = c_i64
-    for f in ("fable_attn_fwd", "fable_attn_fwd_ws", "fable_attn_bwd", "fable_attn_dec", "fable_attn_dec_noalloc",
+    lib.fable_attn_dec_ws.argtypes = [FableDecParams, c_i32, c_ptr, c_i64, c_ptr, c_ptr, c_ptr]
+    lib.fable_attn_dec_ws_bytes.argtypes = [FableDecParams, c_i32, c_i32]
+    lib.fable_attn_dec_ws_bytes.restype = c_i64
+    lib.fable_attn_fwd_paged.argtypes = [FableFwdParams, FablePagedKV, c_i32, c_ptr, c_i64, c_ptr]
+    lib.fable_attn_fwd_paged_ws_bytes.argtypes = [FableFwdParams, FablePagedKV, c_i32]
+    lib.fable_attn_fwd_paged_ws_bytes.restype = c_i64
+    for f in ("fable_attn_dec_ws", "fable_attn_fwd_paged", "fable_attn_fwd", "fable_attn_fwd_ws", "fable_attn_bwd", "fable_attn_dec", "fable_attn_dec_noalloc",
               "fa_forward_launch",
               "fable_attn_backward_launch", "fa_decode_launch",
               "fa_decode_num_splits", "fa_combine_launch", "fable_attn_abi_version"):

@@ -296,6 +296,23 @@ int fable_attn_fwd(FableFwdParams p, int dtype, void* stream);
 int64_t fable_attn_fwd_ws_bytes(FableFwdParams p, int dtype);
 int fable_attn_fwd_ws(FableFwdParams p, int dtype, void* ws, int64_t ws_bytes, void* stream);
 
+/* The forward of packed prompts (p.cu_q / p.cu_k set) whose K/V live in the pages of a cache: key
+ * j of sequence z is row j % page of page block_table[z*max_blocks + j / page]. p.K / p.V are the
+ * caches [num_blocks, page, NH/gqa, HD]; p.sK / p.sV give the strides of a head (.h) and of a row
+ * inside a page (.s), k_page_stride / v_page_stride those of a page (elements). cu_k (or seqused_k)
+ * gives the key counts; entries past a sequence's last page are not read. fp16/bf16, no dropout,
+ * page a power of two of at least 16, kernel widths 64, 128 and 256: for any other call the
+ * workspace query returns -2 (gather the pages and call fable_attn_fwd); -1: an invalid call. The
+ * workspace serves a key split, as in fable_attn_fwd_ws. The reference gathers the pages in Python
+ * (flash_attn_interface.py:455-470). */
+typedef struct FablePagedKV {
+  const int32_t* block_table;
+  int32_t max_blocks, page;
+  int64_t k_page_stride, v_page_stride;
+} FablePagedKV;
+int64_t fable_attn_fwd_paged_ws_bytes(FableFwdParams p, FablePagedKV kv, int dtype);
+int fable_attn_fwd_paged(FableFwdParams p, FablePagedKV kv, int dtype, void* ws, int64_t ws_bytes, void* stream);
+
 /* the backward (reference launcher kernels/backward.hip:508-521); dense or packed varlen */
 int fable_attn_bwd(FableBwdParams p, int dtype, void* stream);
 
@@ -310,6 +327,16 @@ int64_t fable_attn_bwd_ds_bytes(FableBwdParams p, int dtype);
  * new_k/new_v [batch, nq, NH/gqa, HD] (NULL = no append) are written into the paged cache
  * (with rotary on k) before attention, in stream order: no device-wide synchronisation. */
 int fable_attn_dec(FableDecParams p, int dtype, void* stream, const void* new_k, const void* new_v);
+
+/* fable_attn_dec with one workspace for whatever the call needs (p.scratch is ignored), and the
+ * choice of path left to the library: calls with many new tokens run on the forward's tile kernel
+ * (each K/V row read once per query tile instead of once per new token). p.nsplit is the caller's
+ * hint, 0 for the library's choice; the tile path does not take it. fable_attn_dec_ws_bytes gives
+ * the bytes to pass (256-byte aligned device memory, scratch per call); `append` tells whether
+ * new_k/new_v will be passed. Same results as fable_attn_dec up to fp32 summation order. */
+int64_t fable_attn_dec_ws_bytes(FableDecParams p, int dtype, int append);
+int fable_attn_dec_ws(FableDecParams p, int dtype, void* ws, int64_t ws_bytes, void* stream, const void* new_k,
+                      const void* new_v);
 
 /* fable_attn_dec without allocation. No counterpart in the reference: for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that
