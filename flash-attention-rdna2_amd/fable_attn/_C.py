@@ -13,6 +13,9 @@ bound at :239-268) with the same names, argument order and meaning:
     fwd_varlen(q, k, v, cu_q, cu_k, max_sq, max_sk, scale, causal, win_left, win_right,
                softcap, alibi, dropout_p, seed, attn_chunk=0, seqused_q=None,
                seqused_k=None, return_lse=False) -> out  (or (out, lse) when return_lse)
+    fwd_paged(q, k_cache, v_cache, block_table, cu_q, cu_k, max_sq, scale, causal, win_left, win_right,
+              softcap, alibi, attn_chunk=0, seqused_q=None, seqused_k=None) -> out or None
+        (no counterpart in the reference's _C: packed prompts over a paged cache)
     dec(q, k_cache, v_cache, block_table, cache_seqlens, new_k, new_v, rotary_cos,
         rotary_sin, rotary_interleaved, scale, window, num_splits, cache_leftpad=None,
         return_lse=False, softcap=0.0, alibi=None, rotary_dim=0, rotary_pos=None) -> (out, lse)
@@ -250,6 +253,46 @@ def fwd_varlen(q, k, v, cu_q, cu_k, max_sq, max_sk, scale, causal, win_left, win
     with _on(q.device):
         _launch_fwd(p, _dt(q), q.device, _stream(q))
     return (out, lse) if return_lse else out
+
+
+def fwd_paged(q, k_cache, v_cache, block_table, cu_q, cu_k, max_sq, scale, causal, win_left, win_right,
+              softcap, alibi, attn_chunk=0, seqused_q=None, seqused_k=None):
+    """Packed queries q (total_q, Hq, D) against caches [num_blocks, page, Hk, D] (strided pages,
+    rows and heads) through block_table int32 [batch, max_blocks]; key counts from cu_k or
+    seqused_k. Returns out, or None when the library has no paged kernel for the call (the
+    caller gathers the pages). The reference gathers in Python (flash_attn_interface.py:455-470)."""
+    Hq, D, page, Hk = q.shape[1], q.shape[2], k_cache.shape[1], k_cache.shape[2]
+    batch = _check_varlen_index(q, cu_q, cu_k, seqused_q, seqused_k)
+    _check_index("block_table", block_table, q.device, batch, at_least=True)
+    _req(block_table.dim() == 2 and block_table.shape[0] == batch, "block_table must be [batch, max_blocks]")
+    al = _alibi(alibi, Hq, q.device)
+    p = FableFwdParams()
+    p.Q, p.K, p.V = q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr()
+    p.sQ = Strides(0, q.stride(1), q.stride(0))
+    p.sK = Strides(0, k_cache.stride(2), k_cache.stride(1))
+    p.sV = Strides(0, v_cache.stride(2), v_cache.stride(1))
+    p.sO = Strides(0, D, Hq * D)
+    p.SQ, p.SK, p.HD, p.NH, p.gqa = int(max_sq), block_table.shape[1] * page, D, Hq, Hq // Hk
+    p.scale, p.softcap = float(scale), float(softcap)
+    p.win_left, p.win_right = int(win_left), int(win_right)
+    p.alibi_slopes = al.data_ptr() if al is not None else None
+    p.causal = 1 if causal else 0
+    p.cu_q, p.cu_k = cu_q.data_ptr(), cu_k.data_ptr()
+    p.batch, p.attn_chunk = batch, int(attn_chunk)
+    p.seqused_q = seqused_q.data_ptr() if seqused_q is not None else None
+    p.seqused_k = seqused_k.data_ptr() if seqused_k is not None else None
+    kv = _lib.FablePagedKV(block_table.data_ptr(), block_table.shape[1], page, k_cache.stride(0),
+                           v_cache.stride(0))
+    need = int(_L.fable_attn_fwd_paged_ws_bytes(p, kv, _dt(q)))
+    if need == -2:
+        return None
+    make = torch.zeros if seqused_q is not None else torch.empty   # (rows past seqused_q stay 0)
+    out = make(tuple(q.shape), dtype=q.dtype, device=q.device)
+    p.O = out.data_ptr()
+    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need > 0 else None
+    with _on(q.device):
+        _lib.check(_L.fable_attn_fwd_paged(p, kv, _dt(q), _ptr(ws), max(need, 0), _stream(q)), "fable_attn_fwd_paged")
+    return out
 
 
 def bwd(dout, q, k, v, out, lse, scale, causal, win_left, win_right, softcap, alibi, dropout_p,

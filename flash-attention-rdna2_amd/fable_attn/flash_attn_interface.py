@@ -178,12 +178,16 @@ def _bhsd(t):
     return v if aligned else t.clone(memory_format=torch.contiguous_format).transpose(1, 2)
 
 
+def _in_place(t):
+    """Whether the kernels can read t where it is: contiguous head dim, 16-byte aligned rows."""
+    st, el = t.stride(), t.element_size()
+    return st[-1] == 1 and t.data_ptr() % 16 == 0 and all((x * el) % 16 == 0 for x in st[:-1])
+
+
 def _aligned(t, dense=False):
     """t itself when the kernels can read it in place (contiguous head dim, 16-byte aligned
     base and strides; with dense, also contiguous), else a fresh contiguous copy."""
-    st, el = t.stride(), t.element_size()
-    ok = st[-1] == 1 and t.data_ptr() % 16 == 0 and all((x * el) % 16 == 0 for x in st[:-1])
-    if ok and (not dense or t.is_contiguous()):
+    if _in_place(t) and (not dense or t.is_contiguous()):
         return t
     return t.clone(memory_format=torch.contiguous_format)
 
@@ -432,7 +436,8 @@ def _as_index(t, device):
 
 
 def _pages_as_packed(k_cache, v_cache, block_table, cu_seqlens_k, seqused_k):
-    """Paged K/V of a varlen prefill as a packed batch without a host round trip: every
+    """Paged K/V of a varlen call without a paged kernel (_paged_prefill) as a packed batch, without a
+    host round trip: every
     sequence's block-table row is gathered whole (max_blocks * page rows per sequence, one
     device gather), so sequence b starts at row b * max_blocks * page, and its true length
     becomes seqused_k. Table entries past a sequence's ceil(len / page) pages are not read:
@@ -461,6 +466,35 @@ def _pages_as_packed(k_cache, v_cache, block_table, cu_seqlens_k, seqused_k):
     return flat(k_cache), flat(v_cache), cu, used, span
 
 
+def _paged_prefill(q, k_cache, v_cache, block_table, cu_q, cu_k, max_sq, seqused_q, seqused_k, **kw):
+    """Packed prompts over a paged cache without gathering the pages: the kernel reads K/V through
+    the block table. None sends the call to the gather (and to its checks): a gradient, dropout,
+    tensors or strides that the kernel cannot read in place, widths or pages without a paged
+    kernel."""
+    if torch.is_grad_enabled() and (q.requires_grad or k_cache.requires_grad or v_cache.requires_grad):
+        return None
+    if q.device.index is None or q.dtype not in (torch.float16, torch.bfloat16):
+        return None
+    if not (k_cache.dim() == v_cache.dim() == 4 and block_table.dim() == 2 and cu_q.dim() == cu_k.dim() == 1):
+        return None
+    D, page = q.shape[2], k_cache.shape[1]
+    if (v_cache.shape != k_cache.shape or k_cache.shape[3] != D or D % 8 or D > MAX_HEAD_DIM
+            or page < 16 or page & (page - 1) or k_cache.shape[2] < 1 or q.shape[1] % k_cache.shape[2]):
+        return None
+    if block_table.shape[0] != cu_k.numel() - 1 or cu_q.numel() != cu_k.numel() or block_table.shape[1] < 1:
+        return None
+    dev = q.device
+    if any(t.dtype != q.dtype or t.device != dev or not _in_place(t) for t in (q, k_cache, v_cache)):
+        return None
+    spec = _normalize(q, k_cache[0], v_cache[0], head_axis=1, **kw) if k_cache.shape[0] else None
+    if spec is None:
+        return None
+    idx = lambda t: _as_index(t, dev) if t is not None else None
+    return _C.fwd_paged(q, k_cache, v_cache, idx(block_table), idx(cu_q), idx(cu_k), int(max_sq), spec.scale,
+                        bool(spec.causal), spec.wl, spec.wr, spec.softcap, spec.alibi, spec.chunk,
+                        idx(seqused_q), idx(seqused_k))
+
+
 def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                            dropout_p=0.0, softmax_scale=None, causal=False,
                            window_size=(-1, -1), softcap=0.0, alibi_slopes=None,
@@ -478,6 +512,14 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
     if q.dim() != 3:
         raise ValueError(f"fable_attn: varlen expects (total, nheads, headdim), got {tuple(q.shape)}")
     if block_table is not None:
+        if not dropout_p and qv is None and not return_attn_probs:
+            out = _paged_prefill(q, k, v, block_table, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, seqused_q,
+                                 seqused_k, softmax_scale=softmax_scale, causal=causal,
+                                 window_size=window_size, softcap=softcap, alibi_slopes=alibi_slopes,
+                                 attention_chunk=attention_chunk, descale=(q_descale, k_descale, v_descale),
+                                 hints=(num_splits, pack_gqa, sm_margin))
+            if out is not None:
+                return out
         k, v, cu_seqlens_k, seqused_k, max_seqlen_k = _pages_as_packed(
             k, v, block_table, cu_seqlens_k, seqused_k)
     spec = _normalize(q, k, v, qv=qv, softmax_scale=softmax_scale, causal=causal,

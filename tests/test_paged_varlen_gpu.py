@@ -1,0 +1,89 @@
+"""Packed prompts over a paged cache, read in place by the paged tile kernel, against the same call
+with a gradient asked for (which gathers the pages and runs the packed forward) and, where that is
+also the same tile walk, against it bit for bit. The cases cover GQA groups packed into the rows,
+tiles around 256 rows, pages of 16 to 256 rows, lengths that end inside a page, sequences without
+queries or keys, seqused, windows on both sides, a chunk, softcap and alibi, the kernel widths, and
+caches whose pages, rows and heads are strided."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+from tests.helpers import TOL
+
+pytestmark = pytest.mark.gpu
+
+# name, D, Hq, Hk, page, q lengths, k lengths, options
+CASES = [
+    ("gqa4 p16", 128, 8, 2, 16, [37, 64, 100], [90, 64, 230], {}),
+    ("mha p32", 128, 2, 2, 32, [256, 257, 1], [256, 300, 700], {}),
+    ("gqa8 p256 long", 128, 8, 1, 256, [65, 30], [2500, 31], {}),
+    ("empty sequences", 128, 4, 2, 16, [0, 5, 20, 0], [33, 0, 20, 0], {}),
+    ("more queries than keys", 128, 4, 2, 16, [90, 40], [50, 40], {}),
+    ("full mask", 128, 4, 1, 16, [50, 3], [500, 129], {"causal": False}),
+    ("window", 128, 4, 2, 16, [200, 77], [600, 77], {"window_size": (100, 0)}),
+    ("two-sided window", 128, 4, 2, 16, [200, 77], [600, 90], {"causal": False, "window_size": (64, 33)}),
+    ("chunk", 128, 4, 2, 16, [200, 77], [600, 90], {"attention_chunk": 128}),
+    ("softcap", 128, 4, 2, 64, [200, 77], [300, 77], {"softcap": 20.0}),
+    ("alibi", 128, 4, 2, 64, [200, 77], [300, 77], {"alibi": True}),
+    ("D64", 64, 8, 2, 16, [150, 300], [900, 300], {}),
+    ("D40", 40, 4, 2, 16, [150, 30], [200, 30], {}),
+    ("D256", 256, 4, 2, 16, [70, 130], [400, 130], {}),
+    ("D256 window softcap", 256, 4, 2, 16, [70, 130], [400, 130], {"window_size": (96, 0), "softcap": 30.0}),
+    ("D96 gathers", 96, 4, 2, 16, [70], [100], {}),
+]
+
+
+def _call(case, dt, strided=False, used=False):
+    import torch
+
+    from fable_attn import flash_attn_varlen_func
+    name, D, Hq, Hk, page, lq, lk, opt = case
+    opt = dict(opt)
+    opt.setdefault("causal", True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=dt)
+    if opt.pop("alibi", False):
+        opt["alibi_slopes"] = torch.linspace(0.02, 0.3, Hq, device="cuda")
+    nb = max(1, max(-(-n // page) for n in lk))
+    q = rnd(sum(lq), Hq, D)
+    pool = len(lk) * nb + 2
+    if strided:   # (heads outside rows, and K and V interleaved per page)
+        kv = rnd(pool, 2, Hk, page, D)
+        kc, vc = kv[:, 0].transpose(1, 2), kv[:, 1].transpose(1, 2)
+    else:
+        kc, vc = rnd(pool, page, Hk, D), rnd(pool, page, Hk, D)
+    bt = torch.randperm(pool, generator=torch.Generator().manual_seed(5))[:len(lk) * nb].view(len(lk), nb).int()
+    for z, n in enumerate(lk):
+        bt[z, -(-n // page):] = 10 ** 6 + z      # never read
+    bt = bt.cuda()
+    cu = lambda n: torch.tensor([0] + list(np.cumsum(n)), dtype=torch.int32, device="cuda")
+    if used:
+        opt["seqused_q"] = torch.tensor([max(n - 3, 0) for n in lq], dtype=torch.int32, device="cuda")
+        opt["seqused_k"] = torch.tensor([max(n - 5, 0) for n in lk], dtype=torch.int32, device="cuda")
+    f = lambda qq: flash_attn_varlen_func(qq, kc, vc, cu(lq), cu(lk), max(lq), max(lk), block_table=bt, **opt)
+    with torch.no_grad():
+        got = f(q)
+    qg = q.clone()
+    if "attention_chunk" in opt:    # (no gradient with a chunk: the packed call itself)
+        from fable_attn import flash_attn_interface as fai
+        k, v, ck, uk, mk = fai._pages_as_packed(kc, vc, bt, cu(lk), opt.pop("seqused_k", None))
+        want = flash_attn_varlen_func(q, k, v, cu(lq), ck, max(lq), mk, seqused_k=uk, **opt)
+    else:
+        want = f(qg.requires_grad_(True)).detach()
+    torch.cuda.synchronize()
+    return got, want
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_paged_equals_gathered(case, dt):
+    import torch
+    print(f"[paged] {case[0]} {dt}", flush=True)
+    t = {"f16": torch.float16, "bf16": torch.bfloat16}[dt]
+    for kw in ({}, {"strided": True}, {"used": True}):
+        got, want = _call(case, t, **kw)
+        a, b = got.float().cpu().numpy(), want.float().cpu().numpy()
+        assert np.isfinite(a).all()
+        # both are within TOL of the exact result
+        assert orc.rel_rms(a, b) <= 2 * TOL[dt], kw
+        assert np.array_equal(a == 0, b == 0), kw   # rows without a key
