@@ -4,9 +4,11 @@
 // Replaces the reference decode (kernels/fa_decode.hip: fd_partial :57-252, fd_combine
 // :255-272, fd_append :275-302, launcher :319-362) with the same FableDecParams contract
 // (include/fable_attn_abi.h) and a different design:
-//  * one workgroup (4 waves) per (kv head, 16-head group, sequence*new token, split); the q
-//    heads sharing the kv head are packed into the N=16 dimension of v_mfma_f32_16x16x32, so
-//    K and V are read from HBM once per kv head whatever the GQA ratio;
+//  * one workgroup (4 waves) per (kv head, group of 16 rows, run of a sequence's keys): the new
+//    tokens x q heads that share a kv head are packed into the N=16 dimension of
+//    v_mfma_f32_16x16x32, so K and V are read from HBM once per kv head whatever the GQA ratio and
+//    for up to 16 rows of drafted tokens (4 tokens of 4 heads over 32000 keys: 66 -> 33 us, one
+//    pass per token before); fp32: one workgroup per new token;
 //  * K and V rows are read from the paged cache in whole rows (consecutive lanes cover one
 //    row) and staged per wave in LDS; S^T = K . Q^T reads its A operand (16 bytes of one key
 //    row per lane) back from the K slice, and the 16x16 result leaves every lane with one head
@@ -17,8 +19,9 @@
 //    four waves merge in LDS at the end and write one (max, sum, acc[HD]) partial per head and
 //    split;
 //  * the combine kernel merges the splits (natural-log LSE optional);
-//  * appending new_k/new_v (with rotary on k) is a kernel earlier in the same stream: the
-//    reference's hipDeviceSynchronize() after the append (fa_decode.hip:348-351) is gone.
+//  * appending new_k/new_v (with rotary on k) needs no synchronisation of the device (the
+//    reference's hipDeviceSynchronize(), fa_decode.hip:348-351): one new token is written by the
+//    workgroups that read it, several by a kernel earlier in the same stream.
 // Scores are handled in the log2 domain; partial maxima are stored in log2 units.
 #include <mutex>
 #include <type_traits>
@@ -41,23 +44,159 @@ __device__ __forceinline__ float xor16_max(float x) {
 }
 __device__ __forceinline__ float xor16_sum(float x) { return x + __shfl_xor(x, 16); }
 
-struct DecRange {
-  int qpos, hi, lo, start, end;
+// Rows of a (sequence, K/V head): its nq new tokens x the gqa q heads of its group, token first;
+// workgroups take them in groups of 16. The keys of a sequence some row sees are [lo, hi); row
+// masks cut them down (a row of token tk sees [max(leftpad, pos - window + 1), ctx + (append ? tk +
+// 1 : 0))). With `append` the span reaches down to ctx, so that it holds every new key.
+struct DecSpan {
+  int ctx, lo, hi;
+};
+// The lengths and tables are read as constant memory, which no kernel here writes: uniform entries
+// then come by scalar loads (the kernels' own stores otherwise turn them into vector loads, whose
+// in-order counter they would share with the row loads: C4 311 -> 319 us).
+typedef const __attribute__((address_space(4))) int* cint_ptr;
+__device__ __forceinline__ cint_ptr cmem(const int* p) { return (cint_ptr)(uintptr_t)p; }
+__device__ __forceinline__ int dec_room(const FableDecParams& p) {
+  return (int)min((long long)p.max_blocks * p.page, 0x7FFFFFFFLL);
+}
+__device__ __forceinline__ int dec_lo(const FableDecParams& p, int b, int ctx, int tk) {
+  int lo = p.leftpad ? cmem(p.leftpad)[b] : 0;
+  if (p.window >= 0) lo = max(lo, ctx + tk - p.window + 1);
+  return max(lo, 0);
+}
+__device__ __forceinline__ int dec_hi(const FableDecParams& p, int ctx, int tk, int append) {
+  return min(ctx + (append ? tk + 1 : 0), dec_room(p));
+}
+__device__ __forceinline__ DecSpan dec_span(const FableDecParams& p, int b, int append) {
+  DecSpan r;
+  r.ctx = cmem(p.ctx_len)[b];
+  r.lo = dec_lo(p, b, r.ctx, 0);
+  if (append) r.lo = max(min(r.lo, r.ctx), 0);
+  r.hi = dec_hi(p, r.ctx, p.nq - 1, append);
+  return r;
+}
+
+// How a call's keys are shared out when the caller sets no split count (p.nsplit 0). The lengths
+// stay on the device, so every workgroup works out the shares by itself, from units of kUnit keys (a
+// sequence has one at least):
+//  * even: `parts` workgroups per (K/V head, row group); each sequence is cut into runs of `per`
+//    units, `per` the least for which the runs fit the parts, so every workgroup has one run at
+//    most. Taken where that is at most a quarter above an even share (few or alike sequences).
+//  * stream: otherwise (many sequences of unequal lengths) the sequences' units follow one another
+//    and each workgroup (two per part when there are more sequences than parts) takes as many, whatever sequences they belong to.
+// A sequence that lies in one workgroup is finished there; of the others each writes a partial record
+// (a stream's workgroup one for a sequence it goes on with, slot 0, and one for a sequence that goes
+// on after it, slot 1). Two equal splits per sequence, the host's choice before, left 48 requests of 64
+// to 8192 keys (Hq 64 / Hk 8, D 128) waiting for the longest: 142 us, 125 as a stream.
+constexpr int kUnit = kDecKeys * kDecWaves;
+__device__ __forceinline__ int dec_units(const DecSpan& r) { return max((r.hi - r.lo + kUnit - 1) / kUnit, 1); }
+// inclusive prefix sum over the wave (row shifts within 16 lanes, then two broadcasts)
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return x;
+}
+__device__ __forceinline__ int wave_sum(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
+// Every wave for itself: lane l holds the span of sequence base + l, read from memory once for
+// batches of up to 64 sequences (a chain of dependent loads ahead of the first row load is what a
+// short segment takes longest for).
+struct DecShare {
+  DecSpan mine;
+  int units;        // of sequence base + lane; 0 past the batch
+  int base;
+  int total, per;   // units of the call, units per run (even) or workgroup (stream)
+  bool even;
+  __device__ __forceinline__ void load(const FableDecParams& p, int append, int b0, int lane) {
+    base = b0;
+    mine = DecSpan{0, 0, 0};
+    units = 0;
+    if (b0 + lane < p.batch) {
+      mine = dec_span(p, b0 + lane, append);
+      units = dec_units(mine);
+    }
+  }
+  // sum over the batch of f(units); sequence 0's lanes are loaded afterwards
+  template <typename F>
+  __device__ __forceinline__ int sum(const FableDecParams& p, int append, int lane, F&& f) {
+    int t = 0;
+#pragma nounroll
+    for (int b0 = (p.batch - 1) & ~63; b0 >= 0; b0 -= 64) {
+      if (b0 != base) load(p, append, b0, lane);
+      t += wave_sum(f(units));
+    }
+    return t;
+  }
+  __device__ __forceinline__ void init(const FableDecParams& p, int append, int parts, int lane) {
+    load(p, append, 0, lane);
+    total = sum(p, append, lane, [](int u) { return u; });
+    const int least = max((int)((unsigned)(total + parts - 1) / (unsigned)parts), kMinUnits);
+    even = false;
+    if (p.batch <= parts) {
+#pragma nounroll
+      for (per = least; 4 * per <= 5 * least; per += max(per >> 4, 1)) {
+        if (sum(p, append, lane, [=](int u) { return (int)((unsigned)(u + per - 1) / (unsigned)per); }) <= parts) {
+          even = true;
+          break;
+        }
+      }
+    }
+    if (!even) per = p.batch <= parts ? least : max((least + 1) / 2, kMinUnits);
+  }
+  // items: runs (even) or units (stream) of a sequence
+  __device__ __forceinline__ int items(int u) const { return even ? (int)((unsigned)(u + per - 1) / (unsigned)per) : u; }
+  __device__ __forceinline__ DecSpan span(int b) const {
+    const int l = b - base;
+    return DecSpan{__builtin_amdgcn_readlane(mine.ctx, l), __builtin_amdgcn_readlane(mine.lo, l), __builtin_amdgcn_readlane(mine.hi, l)};
+  }
+  // the sequence that holds item `at`, and its first item (p.batch: no such item); after init
+  __device__ __forceinline__ int seek(const FableDecParams& p, int append, int at, int lane, int& first) {
+    first = 0;
+#pragma nounroll
+    for (;;) {
+      const int inc = wave_scan(items(units)), sum = __builtin_amdgcn_readlane(inc, 63);
+      if (at >= first + sum) {
+        first += sum;
+        if (base + 64 >= p.batch) return p.batch;
+        load(p, append, base + 64, lane);
+        continue;
+      }
+      const int n = __popcll(__builtin_amdgcn_ballot_w64(first + inc <= at));   // sequences that end before `at`
+      if (n > 0) first += __builtin_amdgcn_readlane(inc, n - 1);
+      return base + n;
+    }
+  }
+  static constexpr int kMinUnits = 4;
 };
 
-__device__ __forceinline__ DecRange dec_range(const FableDecParams& p, int b, int tk, int sp, int append) {
-  DecRange r;
-  const int ctx = p.ctx_len[b];
-  r.qpos = ctx + tk;
-  r.hi = min(ctx + (append ? tk + 1 : 0), p.max_blocks * p.page);
-  int lo = p.leftpad ? p.leftpad[b] : 0;
-  if (p.window >= 0) lo = max(lo, r.qpos - p.window + 1);
-  r.lo = max(lo, 0);
-  const int n = max(r.hi - r.lo, 0);
-  const int chunk = (((n + p.nsplit - 1) / p.nsplit) + kDecChunk - 1) / kDecChunk * kDecChunk;
-  r.start = r.lo + sp * chunk;
-  r.end = min(r.start + chunk, r.hi);
-  return r;
+// floats ahead of the records: two ints per sequence, for the combine
+__host__ __device__ inline long long dec_meta_floats(const FableDecParams& p) { return (2ll * p.batch + 63) / 64 * 64; }
+
+// The partial kernel's argument. The phases that only some workgroups run (the shares, the append)
+// read it again from the kernel argument segment: the phases together use most of the 40 fields,
+// and held for the whole kernel they spilled some 80 scalar registers.
+struct DecArgs : FableDecParams {
+  const void *nk, *nv;                  // the new key and value of each sequence, or null
+  // block table: entry i of sequence b is table[b * max_blocks + i] (tmask -1), or b * max_blocks + i
+  // for a dense cache without one (tmask 0: table is any readable address, its value masked off; no
+  // branch, which would wait for the load at once)
+  const int* table;
+  int tmask;
+  int page_shift, ngrp, flags, parts, pad;
+};
+__device__ __forceinline__ DecArgs dec_reload() {
+  auto k = (const __attribute__((address_space(4))) uint64_t*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  struct {
+    uint64_t w[sizeof(DecArgs) / 8];
+  } raw;
+  static_assert(sizeof(raw) == sizeof(DecArgs), "whole words");
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(DecArgs) / 8); i++) raw.w[i] = k[i];
+  return __builtin_bit_cast(DecArgs, raw);
 }
 
 // SPT (page >= 16): the block-table entries of a chunk are fetched by scalar loads. A chunk of
@@ -69,9 +208,9 @@ __device__ __forceinline__ DecRange dec_range(const FableDecParams& p, int b, in
 // flags: bit 0 new keys were appended (kDecAppend), bit 1 the kernel writes the final output and
 // LSE itself (kDecFinal: one split, no combine launch)
 constexpr int kDecAppend = 1, kDecFinal = 2;
-template <typename T, int HD, bool FEAT, bool SPT>
-__global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int page_shift, int ngrp, int flags) {
-  const int append = flags & kDecAppend;
+template <typename T, int HD, bool FEAT, bool SPT, bool SHARE>
+__global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
+  const int append = p.flags & kDecAppend, page_shift = p.page_shift;
   using V8 = typename Dt<T>::V8;
   constexpr int NDS = HD / 32;  // S^T contraction steps
   constexpr int NDB = HD / 16;  // 16-row blocks of O^T
@@ -88,25 +227,119 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lg = lane >> 4, lh = lane & 15;  // lane group (0..3), lane in group
-  // grid x = (kv head, head group) fastest: the workgroups reading the interleaved heads of the
-  // same cache pages are dispatched together
-  const int b = blockIdx.y / p.nq, tk = blockIdx.y % p.nq;
-  const int kvh = blockIdx.x / ngrp, hgi = blockIdx.x % ngrp;
-  const int h0 = kvh * p.gqa + 16 * hgi, hg = min(16, p.gqa - 16 * hgi);
-  const int sp = blockIdx.z;
-  const int NKV = p.NH / p.gqa;
-  const DecRange rg = dec_range(p, b, tk, sp, append);
+  // (kv head, row group) fastest: the workgroups reading the interleaved heads of the same cache
+  // pages are dispatched together, the row groups of one head to the same XCD where the heads
+  // are a multiple of 8
+  const int NKV = p.NH / p.gqa, HDr = p.HD, nq = p.nq, gqa = p.gqa, NH = p.NH;
+  const int X = NKV * p.ngrp, hgl = blockIdx.x % X, kvh = hgl % NKV, grp = hgl / NKV;
+  const int r0 = 16 * grp, hg = min(16, nq * gqa - r0);  // rows of this group
+  // row g: token, q head and index in q, o and lse
+  auto row_tok = [&](int g) { return (r0 + g) / gqa; };
+  auto row_of = [&](int b, int g) {
+    const int tok = row_tok(g);
+    return (long long)(b * nq + tok) * NH + kvh * gqa + (r0 + g - tok * gqa);
+  };
+  // segments: a stream part's (sequence, run of keys), or the one split of the grid
+  DecShare str;
+  int at = 0, at_end = 0, sq = 0, first = 0;  // (units; sq: the sequence that holds `at`, first: its first)
+  if constexpr (SHARE) {
+    const DecArgs p = dec_reload();
+    str.init(p, append, p.parts, lane);
+    const int part = blockIdx.x / X;
+    if (str.even) {
+      sq = str.seek(p, append, part, lane, first);
+      if (sq >= p.batch) return;
+      at = (part - first) * str.per;   // (this sequence's units from 0 on)
+      at_end = at + str.per;
+      first = 0;
+    } else {
+      at = part * str.per;
+      at_end = min(at + str.per, str.total);
+      if (at >= at_end) return;
+      sq = str.seek(p, append, at, lane, first);
+    }
+  }
+  for (bool more = true; more;) {
+  const int b = SHARE ? sq : (int)blockIdx.y;
+  DecSpan sp;
+  if constexpr (!SHARE) sp = dec_span(p, b, append);
+  int start, end;
+  float* rec = nullptr;  // record of row 0 (rows rec_step apart); null: the final output
+  long long rec_step = HDr + 2;
+  if constexpr (SHARE) {
+    const DecArgs p = dec_reload();
+    if (b >= str.base + 64) str.load(p, append, b, lane);
+    sp = str.span(b);
+    const int units = dec_units(sp), stop = min(at_end, first + units);
+    start = sp.lo + (at - first) * kUnit;
+    end = min(sp.lo + (stop - first) * kUnit, sp.hi);
+    const bool begins = at == first;
+    const int part = blockIdx.x / X;
+    // where the combine finds this sequence's records: the first one's index, and their count
+    // (negative for a stream, whose later ones are in slot 0)
+    if (begins && hgl == 0 && tid == 0) {
+      const int n = str.even ? str.items(units) : (int)((unsigned)(first + units - 1) / (unsigned)str.per) - part + 1;
+      ((int*)p.scratch)[2 * b] = 2 * part + (str.even ? 0 : 1);
+      ((int*)p.scratch)[2 * b + 1] = str.even ? n : -n;
+    }
+    if (!(begins && stop == first + units))
+      rec = p.scratch + dec_meta_floats(p) + ((2ll * part + (begins && !str.even ? 1 : 0)) * X + hgl) * 16 * (HDr + 2);
+    at = stop;
+    first += units;
+    sq++;
+    more = !str.even && at < at_end;
+  } else {
+    const int n = max(sp.hi - sp.lo, 0);
+    const int chunk = (((n + p.nsplit - 1) / p.nsplit) + kDecChunk - 1) / kDecChunk * kDecChunk;
+    start = sp.lo + (int)blockIdx.z * chunk;
+    end = min(start + chunk, sp.hi);
+    if (!(p.flags & kDecFinal)) {
+      rec = p.scratch + (long long)blockIdx.z * (HDr + 2);
+      rec_step = (long long)p.nsplit * (HDr + 2);   // rows are indexed as in q
+    }
+    more = false;
+  }
+  const int ctx = sp.ctx;
+  start = __builtin_amdgcn_readfirstlane(start);
+  end = __builtin_amdgcn_readfirstlane(end);
 
-  // ---- q rows of this head group -> LDS (fp32): one 16-byte load per thread and chunk,
-  // head index clamped (rows past the group are zeroed after the load)
+  // ---- a single new key (nk) -> the cache (rotated k, v), by the workgroups that read it next: an
+  // append kernel of its own cost 3 us ahead of a 9 us decode. (Row groups of one head write the
+  // same bytes. Several tokens keep the kernel: written here one after another they cost more.)
+  if (append && ctx >= start && ctx < end) {
+    const DecArgs p = dec_reload();
+    if (p.nk) {
+      const int j = ctx >> page_shift, rdim = p.rotary ? (p.rotary_dim > 0 ? p.rotary_dim : HDr) : 0, half = rdim / 2;
+      const int blk = p.block_table ? p.block_table[(long long)b * p.max_blocks + j] : b * p.max_blocks + j;
+      const long long dst = (((long long)blk * p.page + (ctx & (p.page - 1))) * NKV + kvh) * HDr, src = ((long long)b * NKV + kvh) * HDr;
+      T* kd = (T*)p.Kc + dst;
+      const int vc = 8 * (tid - 224);   // (at most 128 pairs of k; the last 32 threads carry v)
+      if (vc >= 0 && vc < HDr) *(u32x4*)((T*)p.Vc + dst + vc) = *(const u32x4*)((const T*)p.nv + src + vc);
+      if (tid >= rdim && tid < HDr) kd[tid] = ((const T*)p.nk)[src + tid];
+      if (tid < half) {
+        const long long at = (long long)(p.rotary_pos ? p.rotary_pos[b] : ctx) * half + tid;
+        const float c = p.cos[at], sn = p.sin[at];
+        const int ia = p.rotary == 1 ? tid : 2 * tid, ib = p.rotary == 1 ? tid + half : 2 * tid + 1;
+        const float x = (float)((const T*)p.nk)[src + ia], y = (float)((const T*)p.nk)[src + ib];
+        kd[ia] = (T)(x * c - y * sn);
+        kd[ib] = (T)(y * c + x * sn);
+      }
+      __syncthreads();  // in the cache (this CU's view of it) before the rows are read below
+    }
+  }
+
+  // ---- q rows of this group -> LDS (fp32): one 16-byte load per thread and chunk,
+  // row index clamped (rows past the group are zeroed after the load)
   // A head dim HDr = p.HD below the kernel width HD (a multiple of 8) runs with zero columns
   // HDr..HD-1 in q, K and V (rows in memory are HDr long); only HDr output columns are kept.
-  const int HDr = p.HD;
-  const T* qg = (const T*)p.q + ((long long)(b * p.nq + tk) * p.NH + h0) * HDr;
+  bool qsplit;
+  {
+  const DecArgs p = dec_reload();
+  qsplit = p.rotary != 0;
   for (int i = tid; i < 16 * RCH; i += 256) {
     const int g = i / RCH, c = i % RCH;
     const bool cok = 8 * c < HDr;
-    const u32x4 raw = *(const u32x4*)(qg + (long long)min(g, hg - 1) * HDr + (cok ? 8 * c : 0));
+    const u32x4 raw = *(const u32x4*)((const T*)p.q + row_of(b, min(g, hg - 1)) * HDr + (cok ? 8 * c : 0));
     const V8 v = bitcast<V8>(raw);
 #pragma unroll
     for (int e = 0; e < 8; e++) qsh[g][8 * c + e] = g < hg && cok ? (float)v[e] : 0.0f;
@@ -114,9 +347,9 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
   __syncthreads();
   if (p.rotary) {
     const int rdim = p.rotary_dim > 0 ? p.rotary_dim : HDr, half = rdim / 2;
-    const int rp = (p.rotary_pos ? p.rotary_pos[b] : p.ctx_len[b]) + tk;
+    const int rbase = p.rotary_pos ? p.rotary_pos[b] : ctx;
     for (int i = tid; i < hg * half; i += 256) {
-      const int g = i / half, j = i % half;
+      const int g = i / half, j = i % half, rp = rbase + row_tok(g);
       const float c = p.cos[(long long)rp * half + j], s = p.sin[(long long)rp * half + j];
       const int ia = p.rotary == 1 ? j : 2 * j, ib = p.rotary == 1 ? j + half : 2 * j + 1;
       const float x = qsh[g][ia], y = qsh[g][ib];
@@ -125,10 +358,10 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
     }
     __syncthreads();
   }
+  }
   // Q^T as the B operand: lane holds head lh, head-dim 32*ds + 8*lg + e. A rotated q is not
   // representable in T; it is carried as hi + lo (two MFMAs per step) so rotation costs no
   // precision beyond fp32.
-  const bool qsplit = p.rotary != 0;
   V8 qb[NDS], ql[NDS];
 #pragma unroll
   for (int ds = 0; ds < NDS; ds++)
@@ -146,10 +379,14 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
   for (int db = 0; db < NDB; db++) oacc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.0f;
   const float c_log2 = p.scale * kLog2e;
-  const float slope = (FEAT && p.alibi && lh < hg) ? p.alibi[h0 + lh] : 0.0f;
+  const int tok = row_tok(min(lh, hg - 1)), qpos = ctx + tok;  // this lane's row (lh)
+  const int rlo = max(dec_lo(p, b, ctx, tok), start), rhi = min(dec_hi(p, ctx, tok, append), end);
+  const float slope = (FEAT && p.alibi && lh < hg) ? p.alibi[kvh * p.gqa + (r0 + lh - tok * p.gqa)] : 0.0f;
   const T* Kc = (const T*)p.Kc;
   const T* Vc = (const T*)p.Vc;
-  const int* bt = p.block_table + (long long)b * p.max_blocks;
+  const cint_ptr bt = cmem(p.table) + (long long)b * (p.max_blocks & p.tmask);
+  const int blk0 = b * p.max_blocks, tmask = p.tmask;
+  auto entry = [&](int raw, int i) { return (raw & tmask) | ((blk0 + i) & ~tmask); };
   const int pmask = p.page - 1;
   T* vb = (T*)vraw + wave * kDecKeys * HD;
   T* kbuf = (T*)kraw + wave * kDecKeys * HD;
@@ -158,17 +395,23 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
   // unconditional. Block-table entries are fetched ahead of the row loads that use them, so the
   // K/V row loads of a chunk issue back to back instead of behind their table lookups.
   constexpr int NVI = kDecKeys * RCH / 64;  // K (and V) row loads per lane per chunk
-  const int last = rg.end - 1;
+  const int last = end - 1;
   auto vkey = [&](int kc0, int i) { return min(kc0 + (64 * i + lane) / RCH, last); };
-  int vblk[SPT ? 1 : NVI], sblk[2];
+  int vblk[SPT ? 1 : NVI], sblk[2], sidx[2];  // (sblk: as read; sidx: their indices)
   auto table = [&](int kc0) {
     if constexpr (SPT) {
       const int b0 = kc0 >> page_shift, bl = last >> page_shift;  // wave-uniform
 #pragma unroll
-      for (int j = 0; j < 2; j++) sblk[j] = bt[min(b0 + j, bl)];
+      for (int j = 0; j < 2; j++) {
+        sidx[j] = min(b0 + j, bl);
+        sblk[j] = bt[sidx[j] & tmask];
+      }
     } else {
 #pragma unroll
-      for (int i = 0; i < NVI; i++) vblk[i] = bt[vkey(kc0, i) >> page_shift];
+      for (int i = 0; i < NVI; i++) {
+        const int e = vkey(kc0, i) >> page_shift;
+        vblk[i] = entry(bt[e & tmask], e);
+      }
     }
   };
   // entry of load i's row: page (key >> page_shift) - (kc0 >> page_shift) of the chunk's two
@@ -176,7 +419,7 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
   auto blk_of = [&](int kc0, int i) {
     if constexpr (SPT) {
       const int j = (vkey(kc0, i) >> page_shift) - (kc0 >> page_shift);
-      return j <= 0 ? sblk[0] : sblk[1];
+      return j <= 0 ? entry(sblk[0], sidx[0]) : entry(sblk[1], sidx[1]);
     } else {
       return vblk[i];
     }
@@ -232,14 +475,14 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
   // streamed fastest with about 8 KiB of rows in flight per wave (16 keys of K and V at
   // D=128); 32-key chunks with a second register set in flight read ~6% slower there.
   constexpr int kStep = kDecKeys * kDecWaves;
-  const int kfirst = rg.start + kDecKeys * wave;
+  const int kfirst = start + kDecKeys * wave;
   u32x4 kreg[NVI], vreg[NVI];
-  if (kfirst < rg.end) {
+  if (kfirst < end) {
     table(kfirst);
     load(kfirst, kreg, vreg);
     table(kfirst + kStep);
   }
-  for (int kc0 = kfirst; kc0 < rg.end; kc0 += kStep) {
+  for (int kc0 = kfirst; kc0 < end; kc0 += kStep) {
     zero_pad(kreg, vreg);
     // K and V -> this wave's LDS slices; the slices are the wave's own, and LDS operations of
     // one wave complete in order, so no barrier orders these writes against the reads below or
@@ -251,7 +494,7 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
       *(u32x4*)(vb + row * HD + 8 * (ch ^ vswz(row))) = vreg[i];
     }
     // the next chunk's rows are in flight during this chunk's products
-    if (kc0 + kStep < rg.end) {
+    if (kc0 + kStep < end) {
       load(kc0 + kStep, kreg, vreg);
       table(kc0 + 2 * kStep);
     }
@@ -277,12 +520,12 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
       if (FEAT) {
         float x = s[r] * p.scale;
         if (p.softcap > 0.0f) x = p.softcap * tanh_exp(x / p.softcap);
-        x += slope * (float)(key - rg.qpos);
+        x += slope * (float)(key - qpos);
         t = x * kLog2e;
       } else {
         t = s[r] * c_log2;
       }
-      t = key < rg.end ? t : -INFINITY;
+      t = ((key >= rlo) & (key < rhi)) ? t : -INFINITY;
       s[r] = t;
       mx = fmaxf(mx, t);
     }
@@ -329,7 +572,7 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
 #pragma unroll
     for (int r = 0; r < 4; r++) red_o[(wave * 16 + lh) * HD + 16 * db + 4 * lg + r] = oacc[db][r];
   __syncthreads();
-  const bool final_out = (flags & kDecFinal) != 0;
+  const DecArgs pe = dec_reload();
   for (int i = tid; i < hg * HDr; i += 256) {
     const int g = i / HDr, d = i % HDr;
     float gm = -INFINITY;
@@ -344,20 +587,22 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(FableDecParams p, int 
         acc += f * red_o[(w * 16 + g) * HD + d];
       }
     }
-    if (final_out) {
+    const long long row = row_of(b, g);
+    if (!rec) {
       // what the combine kernel computes from one split (its weight exp2(0) is exactly 1)
-      const long long row = (long long)(b * p.nq + tk) * p.NH + h0 + g;
       const bool ok = gm != -INFINITY && l > 0.0f;
-      ((T*)p.o)[row * HDr + d] = (T)(ok ? acc / l : 0.0f);
-      if (p.lse_out && d == 0) p.lse_out[row] = ok ? gm * kLn2 + __logf(l) : -INFINITY;
+      ((T*)pe.o)[row * HDr + d] = (T)(ok ? acc / l : 0.0f);
+      if (pe.lse_out && d == 0) pe.lse_out[row] = ok ? gm * kLn2 + __logf(l) : -INFINITY;
       continue;
     }
-    float* out = p.scratch + (((long long)(b * p.nq + tk) * p.NH + h0 + g) * p.nsplit + sp) * (HDr + 2);
+    float* out = rec + (SHARE ? g : row) * rec_step;
     if (d == 0) {
       out[0] = gm;
       out[1] = l;
     }
     out[2 + d] = acc;
+  }
+  if (more) __syncthreads();  // the merge has read the LDS regions before the next segment fills them
   }
 }
 
@@ -391,7 +636,16 @@ __global__ __launch_bounds__(256) void dec_partial_f32_kernel(FableDecParams p, 
   const int h0 = kvh * p.gqa + 16 * hgi, hg = min(16, p.gqa - 16 * hgi);
   const int sp = blockIdx.z;
   const int NKV = p.NH / p.gqa, HDr = p.HD;
-  const DecRange rg = dec_range(p, b, tk, sp, append);
+  struct {
+    int qpos, start, end;
+  } rg;
+  {
+    const int ctx = p.ctx_len[b], lo = dec_lo(p, b, ctx, tk), hi = dec_hi(p, ctx, tk, append), n = max(hi - lo, 0);
+    const int chunk = (((n + p.nsplit - 1) / p.nsplit) + kDecChunk - 1) / kDecChunk * kDecChunk;
+    rg.qpos = ctx + tk;
+    rg.start = lo + sp * chunk;
+    rg.end = min(rg.start + chunk, hi);
+  }
 
   const float* qg = (const float*)p.q + ((long long)(b * p.nq + tk) * p.NH + h0) * HDr;
   for (int i = tid; i < 16 * NQ; i += 256) {
@@ -534,30 +788,37 @@ __global__ __launch_bounds__(256) void dec_partial_f32_kernel(FableDecParams p, 
 }
 
 // merge nsplit partials of one (token, head): grid (batch*nq, NH), block HD
-template <typename T, int HD, int NC>
-__global__ __launch_bounds__(256) void dec_combine_kernel(FableDecParams p) {
+template <typename T, int HD, int NC, bool STREAM = false>
+__global__ __launch_bounds__(256) void dec_combine_kernel(FableDecParams p, int ngrp) {
   // one thread per column of the kernel width HD; the head dim p.HD <= HD sets the strides
   const int row = blockIdx.x, h = blockIdx.y, d = threadIdx.x, HDr = p.HD;
   const int dc = min(d, HDr - 1);  // threads past the head dim read a valid column, store nothing
   const float* base = p.scratch + ((long long)row * p.NH + h) * p.nsplit * (HDr + 2);
-  // the splits in chunks of NC (2, 4 or 8, at least the split count up to 8) whose loads are all
-  // issued before any is used (indices past the last split repeat it and are not used): a few
-  // memory latencies instead of one per split (a batch-1 decode of 21 splits took 12 us here
-  // with one load per step); sums in split order
-  constexpr int kC = NC;
-  const int ns = p.nsplit;
-  auto rec = [&](int s) { return base + (long long)min(s, ns - 1) * (HDr + 2); };
-  float gm = -INFINITY;
-  for (int s0 = 0; s0 < ns; s0 += kC) {
-    float m[kC];
-#pragma unroll
-    for (int u = 0; u < kC; u++) m[u] = rec(s0 + u)[0];
-#pragma unroll
-    for (int u = 0; u < kC; u++)
-      if (s0 + u < ns) gm = fmaxf(gm, m[u]);
+  // STREAM: the records of this row's sequence, one per part its units lie in; one part alone has
+  // written the output already
+  int ns = p.nsplit;
+  long long rest = 0, step = HDr + 2;  // record s > 0 is at base + rest + s * step
+  if constexpr (STREAM) {
+    const int b = row / p.nq, tk = row - b * p.nq, slot0 = ((const int*)p.scratch)[2 * b], n = ((const int*)p.scratch)[2 * b + 1];
+    const int NKV = p.NH / p.gqa, kvh = h / p.gqa, r = tk * p.gqa + h - kvh * p.gqa, X = NKV * ngrp;
+    ns = n < 0 ? -n : n;
+    if (ns < 2) return;
+    const long long slot = (long long)X * 16 * (HDr + 2);
+    base = p.scratch + dec_meta_floats(p) + ((long long)slot0 * X + (r >> 4) * NKV + kvh) * 16 * (HDr + 2) + (r & 15) * (HDr + 2);
+    rest = n < 0 ? -slot : 0;
+    step = 2 * slot;
   }
-  float l = 0.0f, acc = 0.0f;
-  if (gm != -INFINITY) {
+  // the splits in chunks of NC (2, 4 or 8, at least the split count up to 8) whose loads are all
+  // issued before any is used (indices past the last split repeat it and are not used): one
+  // memory latency per chunk (a batch-1 decode of 21 splits took 12 us here with one load per step);
+  // the sums run in split order, scaled where a chunk raises the maximum
+  auto rec = [&](int s) {
+    s = min(s, ns - 1);
+    return base + s * step + (STREAM && s > 0 ? rest : 0);
+  };
+  float gm = -INFINITY, l = 0.0f, acc = 0.0f;
+  auto merge = [&](auto chunk) {
+    constexpr int kC = decltype(chunk)::value;
     for (int s0 = 0; s0 < ns; s0 += kC) {
       float m[kC], ls[kC], a[kC];
 #pragma unroll
@@ -567,6 +828,15 @@ __global__ __launch_bounds__(256) void dec_combine_kernel(FableDecParams p) {
         ls[u] = ps[1];
         a[u] = ps[2 + dc];
       }
+      float nm = gm;
+#pragma unroll
+      for (int u = 0; u < kC; u++)
+        if (s0 + u < ns) nm = fmaxf(nm, m[u]);
+      if (nm == -INFINITY) continue;   // no key so far
+      const float keep = exp2_fast(gm - nm);
+      l *= keep;
+      acc *= keep;
+      gm = nm;
 #pragma unroll
       for (int u = 0; u < kC; u++) {
         if (s0 + u < ns) {
@@ -576,7 +846,11 @@ __global__ __launch_bounds__(256) void dec_combine_kernel(FableDecParams p) {
         }
       }
     }
-  }
+  };
+  if (STREAM && ns == 2)
+    merge(std::integral_constant<int, 2>{});
+  else
+    merge(std::integral_constant<int, NC>{});
   const bool ok = gm != -INFINITY && l > 0.0f;
   if (d < HDr) ((T*)p.o)[((long long)row * p.NH + h) * HDr + d] = (T)(ok ? acc / l : 0.0f);
   if (p.lse_out && d == 0) p.lse_out[(long long)row * p.NH + h] = ok ? gm * kLn2 + __logf(l) : -INFINITY;
@@ -614,10 +888,72 @@ __global__ __launch_bounds__(256) void dec_append_kernel(FableDecParams p, const
     __syncthreads();
   }
   if (!ok) return;
-  const int blk = p.block_table[(long long)b * p.max_blocks + (pos >> page_shift)];
+  const int j = pos >> page_shift, blk = p.block_table ? p.block_table[(long long)b * p.max_blocks + j] : b * p.max_blocks + j;
   const long long dst = (((long long)blk * p.page + (pos & (p.page - 1))) * NKV + kvh) * HDr + d;
   ((T*)p.Kc)[dst] = (T)ks[d];
   ((T*)p.Vc)[dst] = nv[src + d];
+}
+
+// row groups of 16 per (sequence, K/V head)
+static int dec_groups(const FableDecParams& p) { return (int)(((long long)p.nq * p.gqa + 15) / 16); }
+
+// Parts of a call (DecShare): one workgroup per CU (more in flight per CU read a batch of alike
+// sequences slower: C4 0.96x with two, 0.86x with three), or two where the (K/V head, row group) count
+// leaves more than an eighth of the CUs out of a round of one.
+static int dec_parts(const FableDecParams& p) {
+  const long long X = (long long)(p.NH / p.gqa) * dec_groups(p);
+  long long parts = 256 / X;
+  if (parts * X < 224) parts = (512 + X - 1) / X;
+  const long long units = (long long)p.batch * (((long long)p.max_blocks * p.page + kUnit - 1) / kUnit + 1);
+  parts = parts < units ? parts : units;
+  return parts > 1 ? (int)parts : 1;
+}
+// workgroups per (K/V head, row group) (DecShare::init)
+static int dec_share_wgs(const FableDecParams& p) { return p.batch <= dec_parts(p) ? dec_parts(p) : 2 * dec_parts(p); }
+// scratch: two records of 16 rows per workgroup
+static long long dec_share_bytes(const FableDecParams& p) {
+  return (dec_meta_floats(p) + (long long)dec_share_wgs(p) * 2 * (p.NH / p.gqa) * dec_groups(p) * 16 * (p.HD + 2)) * 4;
+}
+
+template <typename T, int HD>
+static int launch_dec_partial(const FableDecParams& p, dim3 grid, int page_shift, int flags, int parts, hipStream_t st, const void* nk,
+                              const void* nv) {
+  const bool feat = p.softcap > 0.0f || p.alibi != nullptr, spt = p.page >= 16;
+  auto go = [&](auto ft, auto sp, auto sh) {
+    DecArgs a;
+    (FableDecParams&)a = p;
+    a.nk = nk;
+    a.nv = nv;
+    a.table = p.block_table ? p.block_table : p.ctx_len;
+    a.tmask = p.block_table ? -1 : 0;
+    a.page_shift = page_shift;
+    a.ngrp = dec_groups(p);
+    a.flags = flags;
+    a.parts = parts;
+    a.pad = 0;
+    hipLaunchKernelGGL((dec_partial_kernel<T, HD, decltype(ft)::value, decltype(sp)::value, decltype(sh)::value>), grid, dim3(256), 0, st, a);
+  };
+  using Y = std::integral_constant<bool, true>;
+  using N = std::integral_constant<bool, false>;
+  if (parts > 0)   // (pages of at least 16 rows: dec_shares)
+    feat ? go(Y{}, Y{}, Y{}) : go(N{}, Y{}, Y{});
+  else if (feat)
+    spt ? go(Y{}, Y{}, N{}) : go(Y{}, N{}, N{});
+  else
+    spt ? go(N{}, Y{}, N{}) : go(N{}, N{}, N{});
+  return launch_status("fable_attn_dec (partial)");
+}
+
+template <typename T, int HD>
+static int launch_dec_append(const FableDecParams& p, hipStream_t st, const void* nk, const void* nv) {
+  hipLaunchKernelGGL((dec_append_kernel<T, HD>), dim3(p.batch * p.nq, p.NH / p.gqa), dim3(HD), 0, st, p, (const T*)nk, (const T*)nv,
+                     __builtin_ctz((unsigned)p.page));
+  return launch_status("fable_attn_dec (append)");
+}
+// whether the partial kernel writes the new key itself: one token per sequence
+template <typename T>
+static bool dec_fuses_append(const FableDecParams& p) {
+  return !std::is_same<T, float>::value && p.nq == 1;
 }
 
 template <typename T, int HD>
@@ -625,41 +961,44 @@ static int launch_dec(const FableDecParams& p, hipStream_t st, const void* nk, c
   const int page_shift = __builtin_ctz((unsigned)p.page);
   const int NKV = p.NH / p.gqa;
   const int ngrp = (p.gqa + 15) / 16;
-  if (nk) {
-    hipLaunchKernelGGL((dec_append_kernel<T, HD>), dim3(p.batch * p.nq, NKV), dim3(HD), 0, st, p,
-                       (const T*)nk, (const T*)nv, page_shift);
-    if (int rc = launch_status("fable_attn_dec (append)")) return rc;
-  }
+  const bool fuse = dec_fuses_append<T>(p);
+  if (nk && !fuse)
+    if (int rc = launch_dec_append<T, HD>(p, st, nk, nv)) return rc;
   const bool feat = p.softcap > 0.0f || p.alibi != nullptr;
-  dim3 grid(NKV * ngrp, p.batch * p.nq, p.nsplit);
   if constexpr (std::is_same<T, float>::value) {
+    const dim3 grid(NKV * ngrp, p.batch * p.nq, p.nsplit);
     if (feat)
       hipLaunchKernelGGL((dec_partial_f32_kernel<HD, true>), grid, dim3(256), 0, st, p, page_shift, ngrp, nk ? 1 : 0);
     else
       hipLaunchKernelGGL((dec_partial_f32_kernel<HD, false>), grid, dim3(256), 0, st, p, page_shift, ngrp, nk ? 1 : 0);
   } else {
-    const bool spt = p.page >= 16;
     // one split: the partial kernel writes the output and LSE, and no combine is launched
     const int flags = (nk ? kDecAppend : 0) | (p.nsplit == 1 ? kDecFinal : 0);
-    if (feat && spt)
-      hipLaunchKernelGGL((dec_partial_kernel<T, HD, true, true>), grid, dim3(256), 0, st, p, page_shift, ngrp, flags);
-    else if (feat)
-      hipLaunchKernelGGL((dec_partial_kernel<T, HD, true, false>), grid, dim3(256), 0, st, p, page_shift, ngrp, flags);
-    else if (spt)
-      hipLaunchKernelGGL((dec_partial_kernel<T, HD, false, true>), grid, dim3(256), 0, st, p, page_shift, ngrp, flags);
-    else
-      hipLaunchKernelGGL((dec_partial_kernel<T, HD, false, false>), grid, dim3(256), 0, st, p, page_shift, ngrp, flags);
-    if (int rc = launch_status("fable_attn_dec (partial)")) return rc;
+    if (int rc = launch_dec_partial<T, HD>(p, dim3(NKV * dec_groups(p), p.batch, p.nsplit), page_shift, flags, 0, st, fuse ? nk : nullptr, nv)) return rc;
     if (p.nsplit == 1) return FA_OK;
   }
   if (int rc = launch_status("fable_attn_dec (partial)")) return rc;
   const dim3 cg(p.batch * p.nq, p.NH);
   if (p.nsplit <= 2)
-    hipLaunchKernelGGL((dec_combine_kernel<T, HD, 2>), cg, dim3(HD), 0, st, p);
+    hipLaunchKernelGGL((dec_combine_kernel<T, HD, 2>), cg, dim3(HD), 0, st, p, 0);
   else if (p.nsplit <= 4)
-    hipLaunchKernelGGL((dec_combine_kernel<T, HD, 4>), cg, dim3(HD), 0, st, p);
+    hipLaunchKernelGGL((dec_combine_kernel<T, HD, 4>), cg, dim3(HD), 0, st, p, 0);
   else
-    hipLaunchKernelGGL((dec_combine_kernel<T, HD, 8>), cg, dim3(HD), 0, st, p);
+    hipLaunchKernelGGL((dec_combine_kernel<T, HD, 8>), cg, dim3(HD), 0, st, p, 0);
+  return launch_status("fable_attn_dec (combine)");
+}
+
+// the call with its shares worked out on the device (p.nsplit 0)
+template <typename T, int HD>
+static int launch_dec_share(const FableDecParams& p, hipStream_t st, const void* nk, const void* nv) {
+  const int ngrp = dec_groups(p), X = p.NH / p.gqa * ngrp, parts = dec_parts(p);
+  const bool fuse = dec_fuses_append<T>(p);
+  if (nk && !fuse)
+    if (int rc = launch_dec_append<T, HD>(p, st, nk, nv)) return rc;
+  if (int rc = launch_dec_partial<T, HD>(p, dim3((unsigned)(X * dec_share_wgs(p))), __builtin_ctz((unsigned)p.page), nk ? kDecAppend : 0, parts,
+                                         st, fuse ? nk : nullptr, nv))
+    return rc;
+  hipLaunchKernelGGL((dec_combine_kernel<T, HD, 8, true>), dim3(p.batch * p.nq, p.NH), dim3(HD), 0, st, p, ngrp);
   return launch_status("fable_attn_dec (combine)");
 }
 
@@ -667,24 +1006,30 @@ static int launch_dec(const FableDecParams& p, hipStream_t st, const void* nk, c
 // multiple of 32 (64 at least: the K slice swizzle needs 8 chunks per row) with zero columns
 // past it. The loads skip those columns' bytes, so HBM traffic is that of the real head dim.
 // fp32 runs in kernels of width 64, 128 and 256, the same way.
+template <typename T, int HD>
+static int launch_dec_any(const FableDecParams& p, hipStream_t st, const void* nk, const void* nv) {
+  if constexpr (!std::is_same<T, float>::value)
+    if (p.nsplit == 0) return launch_dec_share<T, HD>(p, st, nk, nv);
+  return launch_dec<T, HD>(p, st, nk, nv);
+}
 template <typename T>
 static int dec_dispatch(const FableDecParams& p, hipStream_t st, const void* nk, const void* nv) {
   constexpr bool f32 = std::is_same<T, float>::value;
   if (p.HD <= 0 || p.HD > 256 || p.HD % 8)
     return fail(FA_ERR_HEADDIM, "fable_attn_dec: head_dim=%d has no kernel (multiples of 8 up to 256)", p.HD);
   if constexpr (f32) {
-    if (p.HD <= 64) return launch_dec<T, 64>(p, st, nk, nv);
-    if (p.HD <= 128) return launch_dec<T, 128>(p, st, nk, nv);
-    return launch_dec<T, 256>(p, st, nk, nv);
+    if (p.HD <= 64) return launch_dec_any<T, 64>(p, st, nk, nv);
+    if (p.HD <= 128) return launch_dec_any<T, 128>(p, st, nk, nv);
+    return launch_dec_any<T, 256>(p, st, nk, nv);
   } else {
     switch (p.HD <= 64 ? 2 : (p.HD + 31) / 32) {
-      case 2: return launch_dec<T, 64>(p, st, nk, nv);
-      case 3: return launch_dec<T, 96>(p, st, nk, nv);
-      case 4: return launch_dec<T, 128>(p, st, nk, nv);
-      case 5: return launch_dec<T, 160>(p, st, nk, nv);
-      case 6: return launch_dec<T, 192>(p, st, nk, nv);
-      case 7: return launch_dec<T, 224>(p, st, nk, nv);
-      default: return launch_dec<T, 256>(p, st, nk, nv);
+      case 2: return launch_dec_any<T, 64>(p, st, nk, nv);
+      case 3: return launch_dec_any<T, 96>(p, st, nk, nv);
+      case 4: return launch_dec_any<T, 128>(p, st, nk, nv);
+      case 5: return launch_dec_any<T, 160>(p, st, nk, nv);
+      case 6: return launch_dec_any<T, 192>(p, st, nk, nv);
+      case 7: return launch_dec_any<T, 224>(p, st, nk, nv);
+      default: return launch_dec_any<T, 256>(p, st, nk, nv);
     }
   }
 }
@@ -838,7 +1183,7 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(FableDecParams p, const T
   const bool ok = nk && pos >= 0 && (pos >> page_shift) < p.max_blocks;
   long long dst = 0;
   if (ok) {
-    const int blk = p.block_table[(long long)b * p.max_blocks + (pos >> page_shift)];
+    const int j = pos >> page_shift, blk = p.block_table ? p.block_table[(long long)b * p.max_blocks + j] : b * p.max_blocks + j;
     dst = ((long long)blk * p.page + (pos & (p.page - 1))) * NKV * HDr;
   }
   const long long tok = (long long)b * p.nq + tk;
@@ -908,7 +1253,7 @@ static void dec_tile_params(const FableDecParams& p, bool append, FableFwdParams
   f.batch = p.batch;
   f.lse_sb = (int64_t)p.nq * p.NH;
   f.lse_sh = 1;
-  pg = FwdPaged{p.block_table, p.max_blocks, __builtin_ctz((unsigned)p.page), p.page * NKV * D, p.page * NKV * D, p.ctx_len,
+  pg = FwdPaged{p.block_table ? p.block_table : p.ctx_len, p.block_table ? -1 : 0, p.max_blocks, __builtin_ctz((unsigned)p.page), p.page * NKV * D, p.page * NKV * D, p.ctx_len,
                 append ? 1 : 0, p.leftpad, nullptr, p.NH};
 }
 
@@ -970,6 +1315,29 @@ static int dec_checked(FableDecParams p, int dtype, void* stream, const void* ne
 
 // fable_attn_dec with one workspace for whatever the call needs. p.nsplit: the caller's hint (0:
 // the library's choice), which the many-token path does not take.
+// Whether the shares are worked out on the device: fp16/bf16, no count of the caller's, pages of at
+// least 16 rows, a table that can hold kShareBytes of keys and values, and a batch that equal
+// splits would not spread evenly over the parts (more sequences than parts, or a count that
+// does not divide them). The shares take 2-3 us (in the partial kernel, and a combine that is always
+// launched), which batches of short sequences do not win back (32 x 500 keys, Hq 32 / Hk 8: 15.9 us
+// with one workgroup per sequence and head, 18.9 with shares; 7 x 769-12319 keys of two heads 20.7
+// and 20.9; 16 x 100-3000 keys of 16 D-64 heads 35.5 and 31.8; 48 x 64-8192 keys, Hq 64 / Hk 8,
+// 155 and 135). Where equal splits fill the parts they stay: sequences of one length are then
+// shared evenly without (16 x 32768 keys 311 and 314 us; eight of 1000 to 16000 keys 68 and 53).
+constexpr long long kShareBytes = 128LL << 20;
+static bool dec_shares(const FableDecParams& p, int dtype) {
+  if (dtype == FA_F32 || p.nsplit > 0 || p.batch < 2 || p.gqa <= 0 || p.page < 16) return false;
+  if ((long long)p.batch * p.max_blocks * p.page * (p.NH / p.gqa) * p.HD * 4 < kShareBytes) return false;
+  const int parts = fa::dec_parts(p);
+  return p.batch > parts || parts % p.batch != 0;
+}
+// splits per sequence otherwise: its rows are packed into dec_groups groups
+static int dec_fixed_splits(const FableDecParams& p, int dtype) {
+  const int64_t bound = (int64_t)p.max_blocks * p.page;
+  return dtype == FA_F32 ? fa_decode_num_splits(p.batch, p.nq, p.NH, p.gqa, bound, p.nsplit)
+                         : fa_decode_num_splits(p.batch, fa::dec_groups(p), p.NH / p.gqa, 1, bound, p.nsplit);
+}
+
 extern "C" int64_t fable_attn_dec_ws_bytes(FableDecParams p, int dtype, int append) {
   using namespace fa;
   if (p.nq < 1) p.nq = 1;
@@ -982,29 +1350,41 @@ extern "C" int64_t fable_attn_dec_ws_bytes(FableDecParams p, int dtype, int appe
     if (launch_fwd_paged(f, pg, dtype, p.rotary != 0, nullptr, fw) != FA_OK) return -1;
     return 2 * dec_q_bytes(p) + fw.need;
   }
-  p.nsplit = fa_decode_num_splits(p.batch, p.nq, p.NH, p.gqa, (int64_t)p.max_blocks * p.page, p.nsplit);
+  if (dec_shares(p, dtype)) return dec_share_bytes(p);
+  p.nsplit = dec_fixed_splits(p, dtype);
   return dec_uses_scratch(p, dtype) ? (int64_t)p.batch * p.nq * p.NH * p.nsplit * (p.HD + 2) * 4 : 0;
 }
 
-extern "C" int fable_attn_dec_ws(FableDecParams p, int dtype, void* ws, int64_t ws_bytes, void* stream, const void* new_k,
+extern "C" int fable_attn_dec_ws(FableDecParams p, int dtype, void* ws, int64_t ws_bytes, void* stream_, const void* new_k,
                                  const void* new_v) {
   using namespace fa;
-  if (!p.q || !p.Kc || !p.Vc || !p.block_table || !p.o || !p.ctx_len)
-    return fail(FA_ERR_ARG, "fable_attn_dec_ws: null pointer");
+  if (!p.q || !p.Kc || !p.Vc || !p.o || !p.ctx_len) return fail(FA_ERR_ARG, "fable_attn_dec_ws: null pointer");
   if (p.nq < 1) p.nq = 1;
-  const bool tiles = dec_uses_tiles(p, dtype);
-  if (!tiles && p.NH > 0 && p.gqa > 0 && p.NH % p.gqa == 0)
-    p.nsplit = fa_decode_num_splits(p.batch, p.nq, p.NH, p.gqa, (int64_t)p.max_blocks * p.page, p.nsplit);
-  else if (p.nsplit < 1)
-    p.nsplit = 1;
+  const bool tiles = dec_uses_tiles(p, dtype), share = !tiles && dec_shares(p, dtype);
+  if (!p.block_table && dtype == FA_F32) return fail(FA_ERR_ARG, "fable_attn_dec_ws: null block_table (fp32)");
+  const int hint = p.nsplit;
+  p.nsplit = 1;
   if (int rc = dec_check(p, new_k, new_v)) return rc;
   if (p.batch <= 0) return FA_OK;
   if (tiles)
-    return dtype == FA_F16 ? launch_dec_tiles<_Float16>(p, dtype, (char*)ws, ws_bytes, (hipStream_t)stream, new_k, new_v)
-                           : launch_dec_tiles<__bf16>(p, dtype, (char*)ws, ws_bytes, (hipStream_t)stream, new_k, new_v);
-  const long long need = (long long)p.batch * p.nq * p.NH * p.nsplit * (p.HD + 2) * 4;
-  if (dec_uses_scratch(p, dtype) && (!ws || ws_bytes < need))
+    return dtype == FA_F16 ? launch_dec_tiles<_Float16>(p, dtype, (char*)ws, ws_bytes, (hipStream_t)stream_, new_k, new_v)
+                           : launch_dec_tiles<__bf16>(p, dtype, (char*)ws, ws_bytes, (hipStream_t)stream_, new_k, new_v);
+  long long need;
+  if (share) {
+    need = dec_share_bytes(p);
+  } else {
+    p.nsplit = hint;
+    p.nsplit = dec_fixed_splits(p, dtype);
+    need = dec_uses_scratch(p, dtype) ? (long long)p.batch * p.nq * p.NH * p.nsplit * (p.HD + 2) * 4 : 0;
+  }
+  if (need > 0 && (!ws || ws_bytes < need))
     return fail(FA_ERR_ARG, "fable_attn_dec_ws: workspace of %lld bytes, %lld needed", (long long)ws_bytes, need);
   p.scratch = (float*)ws;
-  return dec_checked(p, dtype, stream, new_k, new_v);
+  if (!share) return dec_checked(p, dtype, stream_, new_k, new_v);
+  p.nsplit = 0;
+  switch (dtype) {
+    case FA_F16: return dec_dispatch<_Float16>(p, (hipStream_t)stream_, new_k, new_v);
+    case FA_BF16: return dec_dispatch<__bf16>(p, (hipStream_t)stream_, new_k, new_v);
+    default: return fail(FA_ERR_DTYPE, "fable_attn_dec_ws: dtype %d not implemented (fp16/bf16/fp32)", dtype);
+  }
 }

@@ -196,7 +196,7 @@ static int paged_run(FableFwdParams p, FablePagedKV kv, int dtype, FwdWs& ws, hi
   int rc;
   if (fwd_check(p, dtype, ws.query, rc)) return rc;
   if (!paged_served(p, kv, dtype)) return fail(FA_ERR_ARG, "fable_attn_fwd_paged: head_dim=%d page=%d dtype=%d is not served", p.HD, kv.page, dtype);
-  const FwdPaged pg{kv.block_table, kv.max_blocks, __builtin_ctz((unsigned)kv.page), kv.k_page_stride, kv.v_page_stride,
+  const FwdPaged pg{kv.block_table, -1, kv.max_blocks, __builtin_ctz((unsigned)kv.page), kv.k_page_stride, kv.v_page_stride,
                     nullptr, 0, nullptr, nullptr, 1};
   return launch_fwd_paged(p, pg, dtype, false, st, ws);
 }

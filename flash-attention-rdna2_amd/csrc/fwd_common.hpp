@@ -101,6 +101,8 @@ struct FwdSplit {
 //    ctx[z] keys, and the new tokens' own when `append` (then p.causal is set).
 struct FwdPaged {
   const int* table;      // [batch][max_blocks]
+  int tmask;             // -1; 0: a dense cache, page i of sequence z is z * max_blocks + i and the table's
+                         // value (any readable address) is masked off
   int max_blocks, page_shift;
   long long kpg, vpg;    // elements
   const int* ctx;        // cached keys per sequence, or null

@@ -293,11 +293,16 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
   static_assert(!PG || (kRowStep && 64 % C::DCH == 0 && 64 / C::DCH <= 16), "paged loads");
   int ent[NE], ekey = kstart, pg_cur[NE], pg_prev[NE];  // next K tile's entries and first key
   const int wrow = tid / 64 * (64 / C::DCH);            // first row of the wave's first load
+  auto pg_index = [&](int j) {
+    if constexpr (PG)
+      return z * pg.max_blocks + (min(ekey + wrow + j * RSTEP, kvalid - 1) >> pg.page_shift);
+    else
+      return 0;
+  };
   auto pg_fetch = [&]() {
     if constexpr (PG) {
 #pragma unroll
-      for (int j = 0; j < NE; j++)
-        ent[j] = pg.table[(long long)z * pg.max_blocks + (min(ekey + wrow + j * RSTEP, kvalid - 1) >> pg.page_shift)];
+      for (int j = 0; j < NE; j++) ent[j] = pg.table[pg_index(j) & pg.tmask];
     }
   };
   auto pg_load = [&](u32x4 (&ld)[C::KJ], const T* base, int key0, const int (&page)[NE], long long spg, long long srow,
@@ -327,7 +332,7 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
 #pragma unroll
       for (int j = 0; j < NE; j++) {
         pg_prev[j] = pg_cur[j];
-        pg_cur[j] = __builtin_amdgcn_readfirstlane(ent[j]);
+        pg_cur[j] = __builtin_amdgcn_readfirstlane((ent[j] & pg.tmask) | (pg_index(j) & ~pg.tmask));
       }
       pg_load(ldk, Kg, ekey, pg_cur, pg.kpg, p.sK.s, koff);
       ekey += C::BC;

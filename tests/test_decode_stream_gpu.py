@@ -1,0 +1,118 @@
+"""Decode calls whose keys are shared out by the kernels from the lengths on the device (a table that
+can hold many keys), and the same calls with equal splits per sequence (a narrow table), against
+the fp64 decode oracle with the bounds of the decode tests: batches of unequal lengths whose sequences
+end inside a workgroup's share, span several of them, or are empty; more sequences than a wave has
+lanes; several tokens and heads packed into groups of 16 rows (with the last group partly filled);
+K/V head counts that do not divide the CUs; every kernel width; the append written by the
+workgroups that read the new keys, with a left pad past them, both rotary forms and a partial
+width; a dense cache read without a block table; and the same call replayed as a graph."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+from tests.helpers import to_np
+from tests.test_decode_gpu import check, make_case, run_kernel, run_oracle
+
+pytestmark = pytest.mark.gpu
+RAGGED = [3000, 1, 0, 700, 64, 65, 2047]   # (7: divides no power of two)
+
+# name, HD, NH, gqa, ctx(list per batch), window, rotary, append, leftpad, nq, softcap, alibi, page
+CASES = [
+    ("ragged", 128, 8, 4, RAGGED, -1, 0, False, 0, 1, 0.0, False, 16),
+    ("ragged append rotary", 128, 8, 4, RAGGED, -1, 1, True, 0, 1, 0.0, False, 16),
+    ("ragged mha 5 heads", 64, 5, 1, RAGGED, -1, 2, True, 0, 1, 0.0, False, 64),
+    ("96 kv heads", 64, 96, 1, [500, 3, 200], -1, 0, True, 0, 1, 0.0, False, 16),
+    ("300 kv heads", 64, 300, 1, [130, 3, 64], -1, 0, False, 0, 1, 0.0, False, 16),
+    ("130 sequences", 64, 4, 4, [(37 * i) % 400 for i in range(130)], -1, 1, True, 0, 1, 0.0, False, 16),
+    ("4 tokens x 4 heads", 128, 8, 4, RAGGED, -1, 1, True, 0, 4, 0.0, False, 16),
+    ("5 tokens x 4 heads", 128, 8, 4, RAGGED, -1, 1, True, 0, 5, 0.0, False, 16),
+    ("3 tokens x 8 heads no append", 128, 16, 8, RAGGED, -1, 0, False, 0, 3, 0.0, False, 16),
+    ("21 tokens x 3 heads window", 128, 6, 3, [900, 40, 0], 50, 1, True, 0, 21, 0.0, False, 16),
+    ("20 heads in a group", 128, 40, 20, [900, 40], -1, 0, True, 0, 2, 0.0, False, 16),
+    ("window", 128, 8, 4, RAGGED, 100, 0, True, 0, 2, 0.0, False, 16),
+    ("leftpad past the new keys", 128, 8, 4, [300, 5, 0], -1, 1, True, 40, 2, 0.0, False, 16),
+    ("softcap", 128, 8, 4, RAGGED, -1, 1, True, 0, 3, 20.0, False, 16),
+    ("alibi", 128, 8, 4, RAGGED, -1, 0, True, 0, 3, 0.0, True, 16),
+    ("page 1", 128, 8, 4, [90, 1, 0, 130], -1, 1, True, 0, 2, 0.0, False, 1),
+    ("page 8", 64, 8, 4, [90, 1, 0, 1300], -1, 1, True, 0, 2, 0.0, False, 8),
+    ("D40", 40, 8, 4, RAGGED, -1, 1, True, 0, 2, 0.0, False, 16),
+    ("D96", 96, 8, 4, RAGGED, -1, 1, True, 0, 2, 0.0, False, 16),
+    ("D160 alibi", 160, 4, 2, RAGGED, -1, 0, True, 0, 2, 0.0, True, 16),
+    ("D192", 192, 4, 2, RAGGED, -1, 2, True, 0, 2, 0.0, False, 16),
+    ("D224 softcap", 224, 4, 2, RAGGED, -1, 1, True, 0, 2, 15.0, False, 16),
+    ("D256", 256, 4, 2, RAGGED, -1, 1, True, 0, 2, 0.0, False, 32),
+    ("D256 alibi", 256, 4, 2, RAGGED, -1, 0, False, 0, 2, 0.0, True, 32),
+]
+
+
+def widen(c, bytes_held=1 << 28):
+    """The case with block-table columns (out-of-range entries, never read) up to a table that can
+    hold `bytes_held` of keys and values."""
+    nblk, page, Hk, D = c["kc"].shape
+    B, nb = c["bt"].shape
+    cols = -(-bytes_held // (B * page * Hk * D * 4))
+    c["bt"] = np.concatenate([c["bt"], np.full((B, max(cols - nb, 0)), 10 ** 6, np.int32)], 1)
+    return c
+
+
+@pytest.mark.parametrize("wide", [True, False], ids=["shared", "fixed"])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_stream_parity(case, dt, wide):
+    print(f"[stream] {case[0]} {dt} {'shared' if wide else 'fixed'}", flush=True)
+    c = make_case(case, dt)
+    c = widen(c) if wide else c
+    o, l, kc, vc = run_kernel(c, dt)
+    o_ref, l_ref = run_oracle(c, dt)
+    check(o, l, o_ref, l_ref, dt, case[0])
+    if c["nk"] is not None:
+        kcn, vcn, page = to_np(kc), to_np(vc), c["kc"].shape[1]
+        for b, cx in enumerate(c["ctx"]):
+            for t in range(c["q"].shape[1]):
+                blk, row = c["bt"][b, (cx + t) // page], (cx + t) % page
+                assert np.array_equal(vcn[blk, row], c["nv"][b, t])
+                if not c["rotary"]:
+                    assert np.array_equal(kcn[blk, row], c["nk"][b, t])
+
+
+def test_stream_equals_fixed_splits():
+    """The split count of the caller's choice takes the grid of fixed splits: same result to the
+    rounding of the output (both paths round the same probabilities relative to maxima of their
+    own: see test_decode_tiles_gpu.test_tiles_partial_rotary for the bound)."""
+    c = widen(make_case(("fixed", 128, 8, 4, RAGGED, -1, 1, True, 0, 3, 0.0, False, 16), "bf16"))
+    a, la, _, _ = run_kernel(c, "bf16")
+    for n in (1, 3):
+        b, lb, _, _ = run_kernel(c, "bf16", num_splits=n)
+        assert orc.rel_rms(a, b) <= 2.0 ** -8
+        fin = np.isfinite(la)
+        assert np.array_equal(fin, np.isfinite(lb)) and np.abs(la[fin] - lb[fin]).max() <= 1e-4
+
+
+@pytest.mark.parametrize("nq", [1, 3, 40])
+def test_dense_cache_without_table(nq):
+    """A dense cache read and appended to without a block table (the kernels form sequence b's page
+    as b) against the same cache with the table spelt out, bit for bit; nq 40 runs on the tiles."""
+    import torch
+
+    from fable_attn import _lib
+    L = _lib.load()
+    B, H, Hk, D, cap = 5, 8, 2, 128, 1024
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=torch.bfloat16)
+    q, nk, nv, kc0, vc0 = rnd(B, nq, H, D), rnd(B, nq, Hk, D), rnd(B, nq, Hk, D), rnd(B, cap, Hk, D), rnd(B, cap, Hk, D)
+    lens = torch.tensor([900, 0, 1, 64, 333], dtype=torch.int32, device="cuda")
+    res = []
+    for table in (None, torch.arange(B, dtype=torch.int32, device="cuda").view(B, 1)):
+        kc, vc, out = kc0.clone(), vc0.clone(), torch.empty_like(q)
+        p = _lib.FableDecParams()
+        p.q, p.Kc, p.Vc, p.o, p.ctx_len = q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), lens.data_ptr()
+        p.block_table = table.data_ptr() if table is not None else None
+        p.batch, p.NH, p.gqa, p.HD, p.page, p.max_blocks, p.nq, p.window, p.scale = B, H, H // Hk, D, cap, 1, nq, -1, D ** -0.5
+        n = L.fable_attn_dec_ws_bytes(p, _lib.FA_BF16, 1)
+        ws = torch.empty(max(n, 256), dtype=torch.uint8, device="cuda")
+        st = torch.cuda.current_stream().cuda_stream
+        _lib.check(L.fable_attn_dec_ws(p, _lib.FA_BF16, ws.data_ptr(), n, st, nk.data_ptr(), nv.data_ptr()), "dec")
+        torch.cuda.synchronize()
+        res.append((out, kc, vc))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
