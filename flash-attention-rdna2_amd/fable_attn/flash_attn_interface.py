@@ -349,6 +349,17 @@ def _infer_plan(q, k, v, softmax_scale, causal, window_size, softcap):
     return p, dt, (B, SQ, Hq, D), int(_C._L.fable_attn_fwd_ws_bytes(p, dt))
 
 
+def _plain_call(dropout_p, alibi_slopes, qv, attention_chunk, return_attn_probs, q_descale, k_descale,
+                v_descale, num_splits, pack_gqa, sm_margin):
+    """Whether a dense call's options are those _infer_fast serves (hints of a wrong type, and a chunk
+    of one, go to the general path, which raises)."""
+    return (not dropout_p and alibi_slopes is None and qv is None and not attention_chunk
+            and not return_attn_probs and q_descale is None and k_descale is None
+            and v_descale is None and (num_splits is None or type(num_splits) is int)
+            and (pack_gqa is None or type(pack_gqa) is bool)
+            and (sm_margin is None or type(sm_margin) is int))
+
+
 def _infer_fast(q, k, v, softmax_scale, causal, window_size, softcap):
     """flash_attn_func's plain inference call (no gradient, dropout, alibi, qv, chunk or
     probabilities) with the per-call host work cut to what changes between calls of one
@@ -392,11 +403,8 @@ def flash_attn_func(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False,
                     num_splits=1, pack_gqa=None, sm_margin=0):
     """q, k, v: (batch, seqlen, nheads, headdim). Returns out in the same layout (dense), or
     (out, softmax_lse, S_dmask) when return_attn_probs=True."""
-    if (not dropout_p and alibi_slopes is None and qv is None and not attention_chunk
-            and not return_attn_probs and q_descale is None and k_descale is None
-            and v_descale is None and (num_splits is None or type(num_splits) is int)
-            and (pack_gqa is None or type(pack_gqa) is bool)
-            and (sm_margin is None or type(sm_margin) is int)):
+    if _plain_call(dropout_p, alibi_slopes, qv, attention_chunk, return_attn_probs, q_descale, k_descale,
+                   v_descale, num_splits, pack_gqa, sm_margin):
         out = _infer_fast(q, k, v, softmax_scale, causal, window_size, softcap)
         if out is not None:
             return out
@@ -413,6 +421,11 @@ def flash_attn_qkvpacked_func(qkv, dropout_p=0.0, softmax_scale=None, causal=Fal
                               num_splits=1, pack_gqa=None, sm_margin=0):
     """qkv: (batch, seqlen, 3, nheads, headdim)."""
     q, k, v = qkv.unbind(2)
+    if _plain_call(dropout_p, alibi_slopes, qv, attention_chunk, return_attn_probs, q_descale, k_descale,
+                   v_descale, num_splits, pack_gqa, sm_margin):
+        out = _infer_fast(q, k, v, softmax_scale, causal, window_size, softcap)
+        if out is not None:
+            return out
     return _dense(q, k, v, dropout_p, softmax_scale, causal, window_size, softcap, alibi_slopes,
                   deterministic, return_attn_probs, qv, attention_chunk, q_descale, k_descale,
                   v_descale, num_splits, pack_gqa, sm_margin)
@@ -426,6 +439,11 @@ def flash_attn_kvpacked_func(q, kv, dropout_p=0.0, softmax_scale=None, causal=Fa
                              num_splits=1, pack_gqa=None, sm_margin=0):
     """q: (batch, sq, nheads, d); kv: (batch, sk, 2, nheads_k, d)."""
     k, v = kv.unbind(2)
+    if _plain_call(dropout_p, alibi_slopes, qv, attention_chunk, return_attn_probs, q_descale, k_descale,
+                   v_descale, num_splits, pack_gqa, sm_margin):
+        out = _infer_fast(q, k, v, softmax_scale, causal, window_size, softcap)
+        if out is not None:
+            return out
     return _dense(q, k, v, dropout_p, softmax_scale, causal, window_size, softcap, alibi_slopes,
                   deterministic, return_attn_probs, qv, attention_chunk, q_descale, k_descale,
                   v_descale, num_splits, pack_gqa, sm_margin)
@@ -613,7 +631,68 @@ def _cache_rows(q, k_cache, cache_seqlens, cache_batch_idx, block_table):
     return table, page, lens
 
 
-@torch.no_grad()
+def _sig(t):
+    """What a plan depends on of a tensor argument (None stays None)."""
+    return None if t is None else (t.shape, t.dtype, t.device, t.is_contiguous())
+
+
+def _decode_key(q, k_cache, v_cache, k, v, cos, sin, lens, leftpad, table, alibi, scale, window, softcap,
+                interleaved, num_splits):
+    return (_sig(q), _sig(k_cache), _sig(v_cache), _sig(k), _sig(v), _sig(cos), _sig(sin), _sig(lens),
+            _sig(leftpad), _sig(table), _sig(alibi), scale, window, softcap, interleaved, num_splits)
+
+
+def _decode_plan(q, k_cache, v_cache, k, v, cos, sin, lens, leftpad, table, alibi, scale, window, softcap,
+                 interleaved, num_splits):
+    """The launch parameters of one decode signature that the general path has just served: every
+    tensor contiguous, on q's device and of the dtype the kernels read (so the general path passed
+    them on as they are). None when some tensor was converted or the call took another shape of the
+    problem (a padded or widened head dim, fp32). The result holds no data pointer."""
+    dev = q.device
+    if dev.index is None or lens is None or q.dtype not in (torch.float16, torch.bfloat16):
+        return None
+    if q.dim() != 4 or k_cache.dim() != 4 or v_cache.shape != k_cache.shape or q.shape[3] % 8:
+        return None
+    if any(t is not None and not (t.is_contiguous() and t.device == dev and t.dtype == dt)
+           for dt, ts in ((q.dtype, (q, k_cache, v_cache, k, v)), (torch.float32, (cos, sin, alibi)),
+                          (torch.int32, (lens, leftpad, table))) for t in ts):
+        return None
+    B, NQ, H, D = q.shape
+    page, Hk = k_cache.shape[1], k_cache.shape[2]
+    if table is None and k_cache.shape[0] < B:
+        return None
+    _, wl, _ = _map_window(True, window)
+    p = _lib.FableDecParams()
+    p.batch, p.NH, p.gqa, p.HD, p.page = B, H, H // Hk, D, page
+    p.max_blocks = table.shape[1] if table is not None else 1
+    p.nsplit, p.window = int(num_splits or 0), int(wl + 1 if 0 <= wl < 2 ** 31 - 1 else -1)
+    p.rotary = (2 if interleaved else 1) if cos is not None else 0
+    p.scale = float(scale if scale is not None else D ** -0.5)
+    p.softcap, p.nq = float(softcap or 0.0), NQ
+    p.rotary_dim = int(cos.shape[-1] * 2) if cos is not None else 0
+    dt = _C._dt(q)
+    need = int(_C._L.fable_attn_dec_ws_bytes(p, dt, 1 if k is not None else 0))
+    return None if need < 0 else (p, dt, need)
+
+
+def _decode_fast(plan, q, k_cache, v_cache, k, v, cos, sin, lens, leftpad, table, alibi):
+    """One call of a planned signature: outputs and workspace allocated, pointers filled, launched.
+    None when an address is not aligned or the device is not current (the general path serves it)."""
+    p, dt, need = plan
+    dev = q.device.index
+    ptr = lambda t: t.data_ptr() if t is not None else None
+    qp, kp, vp, nkp, nvp = q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), ptr(k), ptr(v)
+    if (qp | kp | vp | (nkp or 0) | (nvp or 0)) & 15 or dev != torch._C._cuda_getDevice():
+        return None
+    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need > 0 else None
+    p.q, p.Kc, p.Vc, p.o, p.ctx_len = qp, kp, vp, out.data_ptr(), lens.data_ptr()
+    p.block_table, p.cos, p.sin, p.leftpad, p.alibi = ptr(table), ptr(cos), ptr(sin), ptr(leftpad), ptr(alibi)
+    _lib.check(_C._L.fable_attn_dec_ws(p, dt, ptr(ws), need, torch._C._cuda_getCurrentRawStream(dev), nkp, nvp),
+               "fable_attn_dec")
+    return out
+
+
 def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, qv=None,
                             rotary_cos=None, rotary_sin=None,
                             cache_seqlens=None, cache_batch_idx=None, cache_leftpad=None,
@@ -625,6 +704,57 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, qv=None,
                             pack_gqa=None, sm_margin=0, scheduler_metadata=None,
                             cu_seqlens_q=None, cu_seqlens_k_new=None, max_seqlen_q=None,
                             rotary_seqlens=None):
+    """Decode against a paged or dense KV cache (arguments and results: _with_kvcache). A step of a
+    serving loop repeats one signature (shapes, dtypes, options) with new tensors: the first call
+    of a signature goes through all checks, and the launch parameters it came to are kept per
+    thread (without any pointer), so later calls only fill in addresses and launch."""
+    key = None
+    if (qv is None and cache_batch_idx is None and not attention_chunk and not return_softmax_lse
+            and q_descale is None and k_descale is None and v_descale is None and cu_seqlens_q is None
+            and cu_seqlens_k_new is None and rotary_seqlens is None and (page_table is None or block_table is None)
+            and (num_splits is None or type(num_splits) is int) and (pack_gqa is None or type(pack_gqa) is bool)
+            and (sm_margin is None or type(sm_margin) is int)):
+        table = block_table if block_table is not None else page_table
+        args = (q, k_cache, v_cache, k, v, rotary_cos, rotary_sin, cache_seqlens, cache_leftpad, table, alibi_slopes)
+        plans = getattr(_tls, "decode_plans", None)
+        if plans is None:
+            plans = _tls.decode_plans = {}
+        try:
+            key = _decode_key(*args, softmax_scale, window_size, softcap, rotary_interleaved, num_splits)
+            plan = plans.get(key)
+        except (AttributeError, TypeError):   # not tensors, or an unhashable argument
+            key = plan = None
+        if plan is not None:
+            out = _decode_fast(plan, *args)
+            if out is not None:
+                return out
+    res = _with_kvcache(q, k_cache, v_cache, k, v, qv, rotary_cos, rotary_sin, cache_seqlens, cache_batch_idx,
+                        cache_leftpad, block_table, softmax_scale, causal, window_size, softcap,
+                        rotary_interleaved, alibi_slopes, num_splits, return_softmax_lse,
+                        page_table=page_table, attention_chunk=attention_chunk, q_descale=q_descale,
+                        k_descale=k_descale, v_descale=v_descale, pack_gqa=pack_gqa, sm_margin=sm_margin,
+                        scheduler_metadata=scheduler_metadata, cu_seqlens_q=cu_seqlens_q,
+                        cu_seqlens_k_new=cu_seqlens_k_new, max_seqlen_q=max_seqlen_q,
+                        rotary_seqlens=rotary_seqlens)
+    if key is not None and key not in plans:
+        if len(plans) >= _MAX_PLANS:
+            plans.clear()
+        plans[key] = _decode_plan(*args, softmax_scale, window_size, softcap, rotary_interleaved, num_splits)
+    return res
+
+
+@torch.no_grad()
+def _with_kvcache(q, k_cache, v_cache, k=None, v=None, qv=None,
+                  rotary_cos=None, rotary_sin=None,
+                  cache_seqlens=None, cache_batch_idx=None, cache_leftpad=None,
+                  block_table=None, softmax_scale=None, causal=False,
+                  window_size=(-1, -1), softcap=0.0, rotary_interleaved=True,
+                  alibi_slopes=None, num_splits=0, return_softmax_lse=False, *,
+                  page_table=None, attention_chunk=0,
+                  q_descale=None, k_descale=None, v_descale=None,
+                  pack_gqa=None, sm_margin=0, scheduler_metadata=None,
+                  cu_seqlens_q=None, cu_seqlens_k_new=None, max_seqlen_q=None,
+                  rotary_seqlens=None):
     """Decode against a paged (k_cache/v_cache (num_blocks, page, nheads_k, d) + block_table)
     or dense ((batch, seqlen, nheads_k, d)) KV cache; split-KV kernels with an LSE combine.
     q: (batch, seqlen_q, nheads, d), or packed (total_q, nheads, d) with cu_seqlens_q; new
@@ -749,7 +879,7 @@ def _kvcache_packed_q(q, k_cache, v_cache, k, qv, cu_seqlens_q, max_seqlen_q, re
         qvb = qv.new_zeros((nseq * width,) + tuple(qv.shape[1:]))
         qvb[slot] = qv
         qvb = qvb.view(nseq, width, qv.shape[1], qv.shape[2])
-    r = flash_attn_with_kvcache(qb, k_cache, v_cache, qv=qvb, return_softmax_lse=return_lse,
+    r = _with_kvcache(qb, k_cache, v_cache, qv=qvb, return_softmax_lse=return_lse,
                                 **kw)
     ob = r[0] if return_lse else r                               # (batch, width, nheads, dv)
     out = ob.reshape(nseq * width, ob.shape[2], ob.shape[3])[slot]
