@@ -32,14 +32,14 @@ __device__ __forceinline__ float quad_sum_b(float x) {
   return x + __shfl_xor(x, 32);
 }
 
-// log2-domain logit of one score and d(logit)/d(scale*q.k)
-template <bool FEAT>
+// log2-domain logit of one score and d(logit)/d(scale*q.k) (MODE: bwd_with_mode)
+template <int MODE>
 __device__ __forceinline__ float logit2_f32(const FableBwdParams& p, float s, float c_log2, float slope, float inv_cap,
                                             int q, int key, float& deriv) {
   deriv = 1.0f;
-  if (!FEAT) return s * c_log2;
+  if constexpr (MODE == kBwdPlain) return s * c_log2;
   float x = s * p.scale;
-  if (p.softcap > 0.0f) {
+  if constexpr (MODE == kBwdCap) {
     const float t = tanhf(x * inv_cap);
     x = p.softcap * t;
     deriv = 1.0f - t * t;
@@ -183,23 +183,25 @@ bwd_dq_f32_kernel(FableBwdParams p, int nqt) {
           }
         }
       // s[bb][j]: key kb + 16bb + 4g + j, query qi
-      const bool edge = FEAT || (CAUSAL && kb + C::BC - 1 > qw + delta) || kb + C::BC > SK;
+      const bool edge = edge_tile_b<CAUSAL, FEAT>(p, qw, 16, kb, C::BC, delta, SQ, SK);
       uint32_t keep = 0u;  // bit 4*bb + j: score s[bb][j] is kept
       if constexpr (DROP)
         keep = dropout_bits<4 * C::NKB>(p.drop_seed, ((uint64_t)h * SQ + qi) * SK + kb + 4 * g, C::BC, drop_bound,
                                         [](int i) { return (uint64_t)(16 * (i >> 2) + (i & 3)); });
+      bwd_with_mode<FEAT>(p, [&](auto mode) {
 #pragma unroll
-      for (int bb = 0; bb < C::NKB; bb++)
+        for (int bb = 0; bb < C::NKB; bb++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int key = kb + 16 * bb + 4 * g + j;
-          float deriv;
-          const float x = logit2_f32<FEAT>(p, s[bb][j], c_log2, slope, inv_cap, qi, key, deriv);
-          float pr = exp2_fast(x - lse2);
-          if (edge && !visible_b<CAUSAL, FEAT>(p, qi, key, delta, SQ, SK)) pr = 0.0f;
-          const float z = DROP ? dropout_keep(p.keep_scale, keep, 4 * bb + j) : 1.0f;
-          s[bb][j] = pr * (z * dp[bb][j] - Di) * deriv;  // dS^T (backward.hip:170-176)
-        }
+          for (int j = 0; j < 4; j++) {
+            const int key = kb + 16 * bb + 4 * g + j;
+            float deriv;
+            const float x = logit2_f32<decltype(mode)::value>(p, s[bb][j], c_log2, slope, inv_cap, qi, key, deriv);
+            float pr = exp2_fast(x - lse2);
+            if (edge && !visible_b<CAUSAL, FEAT>(p, qi, key, delta, SQ, SK)) pr = 0.0f;
+            const float z = DROP ? dropout_keep(p.keep_scale, keep, 4 * bb + j) : 1.0f;
+            s[bb][j] = pr * (z * dp[bb][j] - Di) * deriv;  // dS^T (backward.hip:170-176)
+          }
+      });
       // dQ^T += K^T . dS^T over key pairs 16bb + 4g + j
       const float* kp = kl + st * C::TILE + 4 * g * C::STR + c16;
 #pragma unroll
@@ -368,27 +370,29 @@ bwd_dkdv_f32_kernel(FableBwdParams p, int nkt) {
           // keep the scheduler from hoisting every LDS read of the loop (register pressure)
           if ((u & 3) == 3) __builtin_amdgcn_sched_barrier(0);
         }
-      const bool edge = FEAT || (CAUSAL && kw + 15 > qt0 + delta) || qt0 + C::BQ > SQ || kw + 16 > SK;
+      const bool edge = edge_tile_b<CAUSAL, FEAT>(p, qt0, C::BQ, kw, 16, delta, SQ, SK);
       uint32_t keep = 0u;  // bit 4*qb + j: score s[qb][j] is kept
       if constexpr (DROP)
         keep = dropout_bits<4 * C::NQB>(p.drop_seed, ((uint64_t)h * SQ + qt0 + 4 * g) * SK + key, (uint64_t)C::BQ * SK, drop_bound,
                                         [&](int i) { return (uint64_t)(16 * (i >> 2) + (i & 3)) * SK; });
+      bwd_with_mode<FEAT>(p, [&](auto mode) {
 #pragma unroll
-      for (int qb = 0; qb < C::NQB; qb++) {
-        const f32x4 l4 = *(const f32x4*)&rowv[stage][0][16 * qb + 4 * g];
-        const f32x4 d4 = *(const f32x4*)&rowv[stage][1][16 * qb + 4 * g];
+        for (int qb = 0; qb < C::NQB; qb++) {
+          const f32x4 l4 = *(const f32x4*)&rowv[stage][0][16 * qb + 4 * g];
+          const f32x4 d4 = *(const f32x4*)&rowv[stage][1][16 * qb + 4 * g];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int q = qt0 + 16 * qb + 4 * g + j;
-          float deriv;
-          const float x = logit2_f32<FEAT>(p, s[qb][j], c_log2, slope, inv_cap, q, key, deriv);
-          float pr = exp2_fast(x - l4[j]);
-          if (edge && !visible_b<CAUSAL, FEAT>(p, q, key, delta, SQ, SK)) pr = 0.0f;
-          const float z = DROP ? dropout_keep(p.keep_scale, keep, 4 * qb + j) : 1.0f;
-          s[qb][j] = z * pr;                               // P (dropped)
-          dp[qb][j] = pr * (z * dp[qb][j] - d4[j]) * deriv;  // dS
+          for (int j = 0; j < 4; j++) {
+            const int q = qt0 + 16 * qb + 4 * g + j;
+            float deriv;
+            const float x = logit2_f32<decltype(mode)::value>(p, s[qb][j], c_log2, slope, inv_cap, q, key, deriv);
+            float pr = exp2_fast(x - l4[j]);
+            if (edge && !visible_b<CAUSAL, FEAT>(p, q, key, delta, SQ, SK)) pr = 0.0f;
+            const float z = DROP ? dropout_keep(p.keep_scale, keep, 4 * qb + j) : 1.0f;
+            s[qb][j] = z * pr;                               // P (dropped)
+            dp[qb][j] = pr * (z * dp[qb][j] - d4[j]) * deriv;  // dS
+          }
         }
-      }
+      });
       // dV^T += dO^T . P, dK^T += Q^T . dS over query pairs 16qb + 4g + j
 #pragma unroll
       for (int qb = 0; qb < C::NQB; qb++)
@@ -450,8 +454,14 @@ static int launch_bwd_f32_1(const FableBwdParams& p, hipStream_t st) {
 int launch_bwd_f32(const FableBwdParams& p, hipStream_t st) {
   if (p.D <= 0 || p.D > 256 || p.D % 8)
     return fail(FA_ERR_HEADDIM, "fable_attn_bwd: head_dim=%d has no fp32 kernel (multiples of 8 up to 256)", p.D);
-  if (p.D <= 64) return launch_bwd_f32_1<F32BwdQCfg<64, 64, 8, 2>, F32BwdKVCfg<64, 64, 8, 2>>(p, st);
-  if (p.D <= 128) return launch_bwd_f32_1<F32BwdQCfg<128, 64, 8, 2>, F32BwdKVCfg<128, 32, 8, 2>>(p, st);
+  // the forward's shapes for the same reasons (launch_fwd_f32): width 64 B2 S1000 H12 causal 285 ->
+  // 226 us, B2 S2000 H12 1029 -> 815 (B1 S2000 H32 causal: 552 with 8 waves, 595 with 4); width 128
+  // B2 S1000 H8 causal 477 -> 306, B4 S1500 H16 2288 -> 2217
+  if (p.D <= 64) {
+    if ((long long)((p.SQ + 127) / 128) * p.Hq * p.B < 512) return launch_bwd_f32_1<F32BwdQCfg<64, 64, 4, 2>, F32BwdKVCfg<64, 64, 4, 2>>(p, st);
+    return launch_bwd_f32_1<F32BwdQCfg<64, 64, 8, 2>, F32BwdKVCfg<64, 64, 8, 2>>(p, st);
+  }
+  if (p.D <= 128) return launch_bwd_f32_1<F32BwdQCfg<128, 32, 4, 2>, F32BwdKVCfg<128, 32, 4, 2>>(p, st);
   return launch_bwd_f32_1<F32BwdQCfg<256, 32, 4, 1>, F32BwdKVCfg<256, 32, 4, 1, 2>>(p, st);
 }
 

@@ -158,7 +158,12 @@ fwd_f32_kernel(FableFwdParams p, int nqt) {
           for (int e = 0; e < 4; e++) s[b] = mma16f32(a[e], qreg[4 * u + e], s[b]);
         }
       // softmax (log2 domain)
-      const bool masked = FEAT || kb + C::BC > SK || (CAUSAL && kb + C::BC - 1 > qw + delta) || qw + 16 > SQ;
+      // (only tiles that some row does not see in full run the mask: with windows, chunk and alibi
+      // tested for every score, a causal alibi layer of 1000 keys spent a third of its VALU work here)
+      bool masked = kb + C::BC > SK || (CAUSAL && kb + C::BC - 1 > qw + delta) || qw + 16 > SQ;
+      if (FEAT)
+        masked = masked || p.attn_chunk > 0 || (p.win_left >= 0 && kb < qw + 15 + delta - p.win_left) ||
+                 (p.win_right >= 0 && kb + C::BC - 1 > qw + delta + p.win_right);
       float mx = -INFINITY;
 #pragma unroll
       for (int b = 0; b < C::NKB; b++)
@@ -252,8 +257,16 @@ static int launch_f32(const FableFwdParams& p, hipStream_t st) {
 int launch_fwd_f32(const FableFwdParams& p, hipStream_t st) {
   if (p.HD <= 0 || p.HD > 256 || p.HD % 8)
     return fail(FA_ERR_HEADDIM, "fable_attn_fwd: head_dim=%d has no fp32 kernel (multiples of 8 up to 256)", p.HD);
-  if (p.HD <= 64) return launch_f32<F32Cfg<64, 64, 8, 2>>(p, st);
-  if (p.HD <= 128) return launch_f32<F32Cfg<128, 64, 8, 2>>(p, st);
+  // Width 64: workgroups of 8 waves while they fill two rounds of the CUs, else of 4 (twice as
+  // many, two per CU): B2 S1000 H12 causal 110 -> 94 us, B2 S2000 H12 340 -> 265; at 512 and 1024
+  // workgroups the 8-wave shape is the faster one (B1 S2000 H32 causal 174 and 185, B8 S1000 H16 202 and
+  // 250). Width 128: 4 waves and 32-key tiles, three workgroups' tiles per CU where the 8-wave
+  // shape with 64 keys held one (B2 S1000 H8 causal 147 -> 107 us, B4 S1500 H16 696 -> 694).
+  if (p.HD <= 64) {
+    if ((long long)((p.SQ + 127) / 128) * p.NH * p.batch < 512) return launch_f32<F32Cfg<64, 64, 4, 2>>(p, st);
+    return launch_f32<F32Cfg<64, 64, 8, 2>>(p, st);
+  }
+  if (p.HD <= 128) return launch_f32<F32Cfg<128, 32, 4, 2>>(p, st);
   return launch_f32<F32Cfg<256, 32, 8, 2>>(p, st);
 }
 

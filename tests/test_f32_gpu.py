@@ -212,3 +212,14 @@ def test_f32_reference_launcher_head_dim_80():
     assert orc.rel_rms(to_np(out), ro) <= FTOL
     le, inf_ok = lse_err(to_np(lse)[None], rl[:1])
     assert inf_ok and le <= LTOL
+
+
+# grids of 512 workgroups of 128 rows at width 64: the 8-wave shape (the cases above take the 4-wave one)
+LARGE = [("D64 causal 512 workgroups", 4, 64, 64, 130, 130, 64, True, -1, -1, 0.0, False, 0, 0.0),
+         ("D64 window gqa 512 workgroups", 4, 64, 32, 130, 140, 64, False, 70, 30, 0.0, False, 0, 0.0)]
+
+
+@pytest.mark.parametrize("case", LARGE, ids=[c[0] for c in LARGE])
+def test_f32_large_grid(case):
+    test_f32_forward_vs_oracle(case)
+    test_f32_backward_vs_oracle(case)
