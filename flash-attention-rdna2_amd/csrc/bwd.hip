@@ -66,3 +66,49 @@ extern "C" int fable_attn_bwd(FableBwdParams p, int dtype, void* stream) {
     default: return fail(FA_ERR_DTYPE, "fable_attn_bwd: dtype %d not implemented (fp16/bf16/fp32)", dtype);
   }
 }
+
+// ------------------------------------------------------------------ rows outside every sequence
+namespace fa {
+
+// Zeros in the rows of a packed tensor that no sequence uses: before cu[0], between a sequence's used
+// rows and the next one's first, and from the last one's used rows to the end. The backward kernels
+// write every row a sequence uses, so filling whole gradients first (three passes over them: 48 us for
+// 25k rows of 32 + 2 x 8 heads, D 128) wrote nearly all of it twice. One launch for dQ, dK and dV:
+// grid (gaps, tensors, slices of a gap), 16-byte stores.
+struct GapTensor {
+  uint4* base;
+  long long rows, row16;      // rows of the buffer, 16-byte units per row
+  int most;                   // the longest sequence the caller named (the kernels' grids end there)
+  const int *cu, *used;
+};
+__global__ __launch_bounds__(256) void zero_gaps_kernel(GapTensor a, GapTensor b, GapTensor c, int batch) {
+  const GapTensor t = blockIdx.y == 0 ? a : (blockIdx.y == 1 ? b : c);
+  const int g = blockIdx.x;   // gap g lies before sequence g (g = batch: after the last one)
+  long long r0 = 0, r1 = g < batch ? t.cu[g] : t.rows;
+  if (g > 0) {
+    const int s0 = t.cu[g - 1], len = t.cu[g] - s0;
+    r0 = s0 + max(min(t.used ? min(len, t.used[g - 1]) : len, t.most), 0);
+  }
+  r0 = max(r0, 0ll) * t.row16;
+  r1 = min(r1, t.rows) * t.row16;
+  for (long long i = r0 + blockIdx.z * 256 + threadIdx.x; i < r1; i += 256ll * gridDim.z) t.base[i] = uint4{0u, 0u, 0u, 0u};
+}
+
+}  // namespace fa
+
+extern "C" int fable_attn_bwd_zero_gaps(FableBwdParams p, int dtype, int64_t total_q, int64_t total_k, void* stream) {
+  using namespace fa;
+  const int el = dtype == FA_F32 ? 4 : 2;
+  // (arguments that fable_attn_bwd refuses are left for it to report)
+  if (!p.dQ || !p.dK || !p.dV || !p.cu_q || !p.cu_k || p.D <= 0 || p.D % 8 || p.Hq <= 0 || p.Hk <= 0) return FA_OK;
+  const long long nq = (long long)p.Hq * p.D * el, nk = (long long)p.Hk * p.D * el;
+  if (((uintptr_t)p.dQ | (uintptr_t)p.dK | (uintptr_t)p.dV) & 15)
+    return fail(FA_ERR_ARG, "fable_attn_bwd_zero_gaps: tensors are not 16-byte aligned");
+  if (p.dqs.s != (int64_t)p.Hq * p.D || p.dks.s != (int64_t)p.Hk * p.D || p.dvs.s != (int64_t)p.Hk * p.D)
+    return fail(FA_ERR_ARG, "fable_attn_bwd_zero_gaps: rows are not contiguous");
+  if (p.B < 0) return FA_OK;
+  hipLaunchKernelGGL(zero_gaps_kernel, dim3(p.B + 1, 3, 4), dim3(256), 0, (hipStream_t)stream,
+                     GapTensor{(uint4*)p.dQ, total_q, nq / 16, p.SQ, p.cu_q, p.seqused_q}, GapTensor{(uint4*)p.dK, total_k, nk / 16, p.SK, p.cu_k, p.seqused_k},
+                     GapTensor{(uint4*)p.dV, total_k, nk / 16, p.SK, p.cu_k, p.seqused_k}, p.B);
+  return launch_status("fable_attn_bwd_zero_gaps");
+}

@@ -990,42 +990,47 @@ __global__ __launch_bounds__(256) void bwd_split_merge_kernel(FableBwdParams p, 
 // ------------------------------------------------------------ dQ from a dS workspace
 // D = rowsum(O*dO) for every (b, h, q) row: HD/8 lanes per row, one 16-byte chunk each, and
 // DSUM_RPT rows per lane whose loads are all in flight before the first sum (one row per lane
-// left each workgroup waiting on a single load pair: C3 33 us for 134 MB).
+// left each workgroup waiting on a single load pair: C3 33 us for 134 MB). Consecutive lane groups
+// take consecutive heads of a token, then the next token: in the (B, S, H, D) layouts of the API
+// a workgroup reads one contiguous run. (A workgroup per head read 256-byte pieces H*D apart: packed
+// batches of 25k rows of 32 heads, D 128, 125 us for 420 MB; now DSUM_US.) A packed batch's rows
+// are those of its whole buffer from cu_q[0] to cu_q[B], whatever sequence they belong to (rows past
+// a seqused end get a sum that nothing reads); the grid covers B times the longest sequence.
 constexpr int DSUM_RPT = 4;
 template <typename T, int HD>
-__global__ __launch_bounds__(256) void bwd_dsum_kernel(FableBwdParams p, int rblocks) {
+__global__ __launch_bounds__(256) void bwd_dsum_kernel(FableBwdParams p) {
   constexpr int LPR = HD / 8, RPB = 256 / LPR;
   using V8 = typename Dt<T>::V8;
   const int tid = threadIdx.x;
-  const int rb = blockIdx.x % rblocks, zh = blockIdx.x / rblocks;
-  const int h = zh % p.Hq, b = zh / p.Hq;
   if (blockIdx.x == 0) ds_build_table(p);  // the dS workspace's tile table, for the next kernels
-  const BwdSeq sq = bwd_seq(p, b);
-  // (a packed batch's grid covers its longest sequence: the blocks past a shorter one's end)
-  if (sq.SQ <= 0 || rb * DSUM_RPT * RPB >= sq.SQ) return;
+  const long long q_first = p.cu_q ? p.cu_q[0] : 0;
+  const long long nrows = p.cu_q ? p.cu_q[p.B] - q_first : (long long)p.B * p.SQ, total = nrows * p.Hq;
   const int c = tid % LPR;
   // chunks past a head dim p.D below HD read the row's first chunk and add nothing
   const bool cok = 8 * c < p.D;
-  const T* ob = (const T*)p.O + (long long)b * p.os.b + (long long)h * p.os.h + (cok ? 8 * c : 0);
-  const T* db = (const T*)p.dO + (long long)b * p.dos.b + (long long)h * p.dos.h + (cok ? 8 * c : 0);
+  for (long long i0 = (long long)blockIdx.x * (RPB * DSUM_RPT); i0 < total; i0 += (long long)gridDim.x * (RPB * DSUM_RPT)) {
   V8 o[DSUM_RPT], d[DSUM_RPT];
+  long long at[DSUM_RPT];
 #pragma unroll
   for (int r = 0; r < DSUM_RPT; r++) {
-    // rows past the end load the last row (in bounds) and are not stored
-    const int q = min((rb * DSUM_RPT + r) * RPB + tid / LPR, sq.SQ - 1);
-    o[r] = *(const V8*)(ob + (sq.qo + q) * p.os.s);
-    d[r] = *(const V8*)(db + (sq.qo + q) * p.dos.s);
+    // pairs past the end load the last one (in bounds) and are not stored
+    const long long i = min(i0 + r * RPB + tid / LPR, total - 1), row = i / p.Hq;
+    const int h = (int)(i - row * p.Hq);
+    const long long b = p.cu_q ? 0 : row / p.SQ, q = p.cu_q ? q_first + row : row - b * p.SQ;
+    o[r] = *(const V8*)((const T*)p.O + b * p.os.b + (long long)h * p.os.h + q * p.os.s + (cok ? 8 * c : 0));
+    d[r] = *(const V8*)((const T*)p.dO + b * p.dos.b + (long long)h * p.dos.h + q * p.dos.s + (cok ? 8 * c : 0));
+    at[r] = b * p.lse_sb + (long long)h * p.lse_sh + q;
   }
 #pragma unroll
   for (int r = 0; r < DSUM_RPT; r++) {
-    const int q = (rb * DSUM_RPT + r) * RPB + tid / LPR;
     float acc = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; e++) acc += (float)o[r][e] * (float)d[r][e];
     acc = cok ? acc : 0.0f;
 #pragma unroll
     for (int m = LPR / 2; m > 0; m >>= 1) acc += __shfl_xor(acc, m);
-    if (c == 0 && q < sq.SQ) p.dsum[(long long)b * p.lse_sb + (long long)h * p.lse_sh + sq.qo + q] = acc;
+    if (c == 0 && i0 + r * RPB + tid / LPR < total) p.dsum[at[r]] = acc;
+  }
   }
 }
 
@@ -1318,8 +1323,8 @@ static int launch_bwd_ds(const FableBwdParams& p, hipStream_t st, int nkt) {
   // the D-row kernel reduces over a power-of-two count of lanes per row (chunks past the head
   // dim add zero)
   constexpr int DW = CKV::HD <= 32 ? 32 : (CKV::HD <= 64 ? 64 : (CKV::HD <= 128 ? 128 : 256));
-  constexpr int RPB = 256 / (DW / 8) * DSUM_RPT;  // rows per dsum workgroup
-  const long long gd = (long long)((p.SQ + RPB - 1) / RPB) * p.Hq * p.B;
+  constexpr int RPB = 256 / (DW / 8) * DSUM_RPT;  // (row, head) pairs per dsum workgroup
+  const long long gd = ((long long)p.SQ * p.Hq * p.B + RPB - 1) / RPB;
   // grids of fewer 8-wave workgroups than CUs run 4-wave ones (twice as many, half the rows)
   using CDS = BwdDsQCfg<CKV::HD, 4, CD::WPE, kDsqSets>;
   const int nqt = (p.SQ + CD::BQ - 1) / CD::BQ;
@@ -1328,7 +1333,7 @@ static int launch_bwd_ds(const FableBwdParams& p, hipStream_t st, int nkt) {
   const long long gq = (long long)(small ? nqts : nqt) * p.Hq * p.B;
   const long long gkv = (long long)nkt * p.Hk * p.B * CKV::DSPLIT;
   if (gd > 0x7FFFFFFF || gq > 0x7FFFFFFF || gkv > 0x7FFFFFFF) return fail(FA_ERR_ARG, "fable_attn_bwd: grid too large");
-  hipLaunchKernelGGL((bwd_dsum_kernel<T, DW>), dim3((unsigned)gd), dim3(256), 0, st, p, (p.SQ + RPB - 1) / RPB);
+  hipLaunchKernelGGL((bwd_dsum_kernel<T, DW>), dim3((unsigned)gd), dim3(256), 0, st, p);
   if (int rc = launch_status("fable_attn_bwd (dsum)")) return rc;
   if constexpr (CKV::PAIR) {
     BwdSplit sp{1, nkt, CKV::BK, 0, nullptr};

@@ -350,7 +350,8 @@ def bwd_varlen(dout, q, k, v, out, lse, cu_q, cu_k, max_sq, max_sk, scale, causa
     _req(lse.dtype == torch.float32 and lse.is_contiguous() and tuple(lse.shape) == (Hq, q.shape[0])
          and lse.device == q.device, "lse must be contiguous fp32 [Hq, total_q] on q's device")
     batch = _check_varlen_index(q, cu_q, cu_k, seqused_q, seqused_k)
-    dq, dk, dv = torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v)
+    # dense; the kernels write every row a sequence uses, one launch ahead of them zeroes the others
+    dq, dk, dv = (torch.empty(t.shape, dtype=t.dtype, device=t.device) for t in (q, k, v))
     dsum = torch.empty((Hq, q.shape[0]), dtype=torch.float32, device=q.device)
     al = _alibi(alibi, Hq, q.device)
     row = lambda t: Strides(0, t.stride(1), t.stride(0))
@@ -373,6 +374,7 @@ def bwd_varlen(dout, q, k, v, out, lse, cu_q, cu_k, max_sq, max_sk, scale, causa
     p.lse_sb, p.lse_sh = 0, q.shape[0]
     ws = _ds_workspace(p, _dt(q), q.device, ds_max_bytes)  # noqa: F841  (alive through the launch)
     with _on(q.device):
+        _lib.check(_L.fable_attn_bwd_zero_gaps(p, _dt(q), q.shape[0], k.shape[0], _stream(q)), "fable_attn_bwd (varlen)")
         _lib.check(_L.fable_attn_bwd(p, _dt(q), _stream(q)), "fable_attn_bwd (varlen)")
     return dq, dk, dv
 

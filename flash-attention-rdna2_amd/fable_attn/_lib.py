@@ -125,7 +125,7 @@ STRUCTS = {0: FableFwdParams, 1: FableBwdParams, 2: FableDecParams, 3: CombinePa
 EXPORTS = ("fa_forward_launch", "fable_attn_backward_launch", "fa_decode_launch",
            "fable_attn_fwd", "fable_attn_fwd_ws", "fable_attn_fwd_ws_bytes", "fable_attn_bwd", "fable_attn_dec", "fable_attn_dec_noalloc",
            "fable_attn_dec_noalloc_max_floats", "fable_attn_dec_ws", "fable_attn_dec_ws_bytes",
-           "fable_attn_fwd_paged", "fable_attn_fwd_paged_ws_bytes",
+           "fable_attn_fwd_paged", "fable_attn_fwd_paged_ws_bytes", "fable_attn_bwd_zero_gaps",
            "fa_decode_num_splits", "fa_combine_launch", "fable_attn_bwd_ds_bytes",
            "fable_attn_abi_version", "fable_attn_struct_size", "fable_attn_last_error")
 
@@ -161,7 +161,8 @@ def load():
     lib.fable_attn_fwd_paged.argtypes = [FableFwdParams, FablePagedKV, c_i32, c_ptr, c_i64, c_ptr]
     lib.fable_attn_fwd_paged_ws_bytes.argtypes = [FableFwdParams, FablePagedKV, c_i32]
     lib.fable_attn_fwd_paged_ws_bytes.restype = c_i64
-    for f in ("fable_attn_dec_ws", "fable_attn_fwd_paged", "fable_attn_fwd", "fable_attn_fwd_ws", "fable_attn_bwd", "fable_attn_dec", "fable_attn_dec_noalloc",
+    lib.fable_attn_bwd_zero_gaps.argtypes = [FableBwdParams, c_i32, c_i64, c_i64, c_ptr]
+    for f in ("fable_attn_bwd_zero_gaps", "fable_attn_dec_ws", "fable_attn_fwd_paged", "fable_attn_fwd", "fable_attn_fwd_ws", "fable_attn_bwd", "fable_attn_dec", "fable_attn_dec_noalloc",
               "fa_forward_launch",
               "fable_attn_backward_launch", "fa_decode_launch",
               "fa_decode_num_splits", "fa_combine_launch", "fable_attn_abi_version"):

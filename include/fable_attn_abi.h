@@ -316,6 +316,11 @@ int fable_attn_fwd_paged(FableFwdParams p, FablePagedKV kv, int dtype, void* ws,
 /* the backward (reference launcher kernels/backward.hip:508-521); dense or packed varlen */
 int fable_attn_bwd(FableBwdParams p, int dtype, void* stream);
 
+/* Zeros in the rows of packed dQ (total_q rows), dK and dV (total_k rows) that no sequence uses (outside
+ * cu_q / cu_k, past seqused): fable_attn_bwd writes the others. The gradients are dense [total, H, D]
+ * tensors. No reference counterpart (the reference allocates zeroed gradients per sequence). */
+int fable_attn_bwd_zero_gaps(FableBwdParams p, int dtype, int64_t total_q, int64_t total_k, void* stream);
+
 /* Bytes of FableBwdParams.ds_ws the backward can use for these shapes (fp16/bf16 at every head
  * dim; 0 for fp32, which recomputes, or when no query sees a key). No reference counterpart: the
  * reference backward recomputes dS in its dQ kernel (backward.hip:298-387). A table of

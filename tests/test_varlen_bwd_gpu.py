@@ -21,7 +21,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as orc
-from tests.helpers import check_grads, gen, to_dev, to_np
+from tests.helpers import check_grads, gen, to_dev, to_np, torch_dtype
 
 pytestmark = pytest.mark.gpu
 
@@ -257,3 +257,49 @@ def test_varlen_backward_persistent(case, dt):
         model = orc.bwd(*args, model=dt, stored_o=bhsd(out[a:b]))
         got = [x[a:b].transpose(1, 0, 2)[None] for x in (dq, dk, dv)]
         check_grads("varlen_bwd_persist", f"{name} seq {i} len {lens[i]}", dt, got, ref, model, vanish_ok=True)
+
+
+@pytest.mark.parametrize("dt", [torch_dtype("bf16"), torch_dtype("f32")], ids=["bf16", "f32"])
+@pytest.mark.parametrize("used", [False, True], ids=["whole", "seqused"])
+def test_varlen_backward_rows_of_no_sequence(dt, used):
+    """Rows before the first and after the last sequence, past seqused and of sequences without
+    queries or keys: zero gradients, in buffers that held NaN before; the other rows as in a buffer
+    that holds the sequences alone."""
+    import torch
+
+    from fable_attn import _C
+    lq, lk, H, Hk, D = [40, 0, 130, 7], [64, 33, 0, 90], 4, 2, 64
+    uq, uk = ([30, 0, 130, 2], [64, 20, 0, 50]) if used else (lq, lk)
+    lead, tail = 5, 200
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rnd = lambda n, h: torch.randn(n, h, D, generator=g, device="cuda", dtype=torch.float32).to(dt)
+    cu = lambda n: torch.tensor([lead + sum(n[:i]) for i in range(len(n) + 1)], dtype=torch.int32, device="cuda")
+    nq, nk = lead + sum(lq) + tail, lead + sum(lk) + tail
+    q, do, k, v = rnd(nq, H), rnd(nq, H), rnd(nk, Hk), rnd(nk, Hk)
+    iq, ik = (torch.tensor(u, dtype=torch.int32, device="cuda") if used else None for u in (uq, uk))
+    args = (0.125, True, -1, 0, 0.0, None, 0.0, 0)
+    out, lse = _C.fwd_varlen(q, k, v, cu(lq), cu(lk), max(lq), max(lk), *args, 0, iq, ik, return_lse=True)
+    poison = [torch.full((n, h, D), float("nan"), device="cuda", dtype=dt) for n, h in ((nq, H), (nk, Hk), (nk, Hk))]
+    del poison   # (the allocator hands the same memory out again)
+    got = _C.bwd_varlen(do, q, k, v, out, lse, cu(lq), cu(lk), max(lq), max(lk), *args, iq, ik)
+    torch.cuda.synchronize()
+    for t, lens, use in ((got[0], lq, uq), (got[1], lk, uk), (got[2], lk, uk)):
+        live = torch.zeros(t.shape[0], dtype=torch.bool, device="cuda")
+        at = lead
+        for n, u in zip(lens, use):
+            live[at:at + min(n, u)] = True
+            at += n
+        assert torch.isfinite(t).all()
+        assert (t[~live] == 0).all()
+    for z in range(4):   # each sequence on its own
+        if not uq[z] or not uk[z]:
+            continue
+        a, b = lead + sum(lq[:z]), lead + sum(lk[:z])
+        one = lambda n: torch.tensor([0, n], dtype=torch.int32, device="cuda")
+        s = [x[i:i + n].contiguous() for x, i, n in ((do, a, uq[z]), (q, a, uq[z]), (k, b, uk[z]), (v, b, uk[z]), (out, a, uq[z]))]
+        ref = _C.bwd_varlen(s[0], s[1], s[2], s[3], s[4], lse[:, a:a + uq[z]].contiguous(), one(uq[z]), one(uk[z]), uq[z], uk[z], *args)
+        # the same tiles and sums in the same order (the splits of a small grid may differ: fp32 partials
+        # summed in another order move a result across at most one rounding of the dtype)
+        for x, y in zip((got[0][a:a + uq[z]], got[1][b:b + uk[z]], got[2][b:b + uk[z]]), ref):
+            tol = 2.0 ** -7 if dt is torch.bfloat16 else 1e-5
+            assert (x.float() - y.float()).abs().max() <= tol * y.float().abs().max()
