@@ -349,6 +349,15 @@ def _infer_plan(q, k, v, softmax_scale, causal, window_size, softcap):
     return p, dt, (B, SQ, Hq, D), int(_C._L.fable_attn_fwd_ws_bytes(p, dt))
 
 
+def _option_key(softmax_scale, window_size, softcap):
+    """The options of a signature by value: a tensor hashes by its identity, so a key that held it would
+    still match after its value changed. TypeError (no key, the general path) for a window of tensors."""
+    left, right = window_size
+    if isinstance(left, torch.Tensor) or isinstance(right, torch.Tensor):
+        raise TypeError("no key")
+    return (softmax_scale if softmax_scale is None else float(softmax_scale), window_size, float(softcap or 0.0))
+
+
 def _plain_call(dropout_p, alibi_slopes, qv, attention_chunk, return_attn_probs, q_descale, k_descale,
                 v_descale, num_splits, pack_gqa, sm_margin):
     """Whether a dense call's options are those _infer_fast serves (hints of a wrong type, and a chunk
@@ -373,10 +382,10 @@ def _infer_fast(q, k, v, softmax_scale, causal, window_size, softcap):
     if plans is None:
         plans = _tls.plans = {}
     try:
-        key = (q.shape, k.shape, v.shape, q.stride(), k.stride(), v.stride(), q.dtype, q.device,
-               causal, window_size, softcap, softmax_scale)
+        key = (q.shape, k.shape, v.shape, q.stride(), k.stride(), v.stride(), q.dtype, k.dtype, v.dtype,
+               q.device, k.device, v.device, _option_key(softmax_scale, window_size, softcap), bool(causal))
         plan = plans.get(key, False)
-    except (AttributeError, TypeError):   # not tensors, or an unhashable argument
+    except (AttributeError, TypeError, ValueError, RuntimeError):   # not tensors, or no key
         return None
     if plan is False:
         if len(plans) >= _MAX_PLANS:
@@ -639,7 +648,7 @@ def _sig(t):
 def _decode_key(q, k_cache, v_cache, k, v, cos, sin, lens, leftpad, table, alibi, scale, window, softcap,
                 interleaved, num_splits):
     return (_sig(q), _sig(k_cache), _sig(v_cache), _sig(k), _sig(v), _sig(cos), _sig(sin), _sig(lens),
-            _sig(leftpad), _sig(table), _sig(alibi), scale, window, softcap, interleaved, num_splits)
+            _sig(leftpad), _sig(table), _sig(alibi), _option_key(scale, window, softcap), bool(interleaved), num_splits)
 
 
 def _decode_plan(q, k_cache, v_cache, k, v, cos, sin, lens, leftpad, table, alibi, scale, window, softcap,
@@ -722,7 +731,7 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, qv=None,
         try:
             key = _decode_key(*args, softmax_scale, window_size, softcap, rotary_interleaved, num_splits)
             plan = plans.get(key)
-        except (AttributeError, TypeError):   # not tensors, or an unhashable argument
+        except (AttributeError, TypeError, ValueError, RuntimeError):   # not tensors, or no key
             key = plan = None
         if plan is not None:
             out = _decode_fast(plan, *args)

@@ -108,3 +108,37 @@ def test_packed_inference_equals_separate():
         for _ in range(2):
             assert torch.equal(flash_attn_qkvpacked_func(qkv, **kw), want)
             assert torch.equal(flash_attn_kvpacked_func(qkv[:, :, 0], qkv[:, :, 1:], **kw), want)
+
+
+def test_tensor_options_by_value():
+    """A scale, cap or window given as a tensor counts by the value it has at the call."""
+    import torch
+
+    from fable_attn import flash_attn_kvpacked_func
+    c = _inputs(1, append=False)
+    qkv = torch.randn(2, 77, 3, 4, 64, device="cuda", dtype=torch.float16)
+    x = torch.tensor(2.0)
+    for opt in ({"softmax_scale": x}, {"softcap": x}, {"window_size": (x, 0)}):
+        for value in (2.0, 5.0):
+            x.fill_(value)
+            plain = {n: value if t is x else (int(value), 0) for n, t in opt.items()}
+            for _ in range(2):
+                assert torch.equal(_both(c, **opt), _both(c, **plain))
+                assert torch.equal(flash_attn_kvpacked_func(qkv[:, :, 0], qkv[:, :, 1:], **opt),
+                                   flash_attn_kvpacked_func(qkv[:, :, 0], qkv[:, :, 1:], **plain))
+
+
+def test_packed_inference_mixed_dtypes_refused():
+    """A served (fp16, fp16) signature does not let (fp16 q, bf16 kv) of the same shapes through."""
+    import torch
+
+    from fable_attn import flash_attn_func, flash_attn_kvpacked_func
+    q = torch.randn(1, 32, 4, 64, device="cuda", dtype=torch.float16)
+    kv = torch.randn(1, 32, 2, 4, 64, device="cuda", dtype=torch.float16)
+    flash_attn_kvpacked_func(q, kv)
+    with pytest.raises(RuntimeError):
+        flash_attn_kvpacked_func(q, kv.bfloat16())
+    k, v = kv.unbind(2)
+    for a, b in ((k.bfloat16(), v), (k, v.bfloat16())):
+        with pytest.raises(RuntimeError):
+            flash_attn_func(q, a, b)
