@@ -74,16 +74,20 @@ namespace fa {
 // rows and the next one's first, and from the last one's used rows to the end. The backward kernels
 // write every row a sequence uses, so filling whole gradients first (three passes over them: 48 us for
 // 25k rows of 32 + 2 x 8 heads, D 128) wrote nearly all of it twice. One launch for dQ, dK and dV:
-// grid (gaps, tensors, slices of a gap), 16-byte stores.
+// grid (workgroups, tensors), 16-byte stores. A buffer padded to a fixed size has its padding in the
+// last gap (kTailParts workgroups), sequences cut by seqused in every gap (`slices` each): with 4 workgroups per
+// gap 8 sequences of 512 rows ahead of 28k rows of padding took 15 us longer than the fill, now as long (47 us).
+constexpr int kTailParts = 128, kUsedParts = 1024;
 struct GapTensor {
   uint4* base;
   long long rows, row16;      // rows of the buffer, 16-byte units per row
   int most;                   // the longest sequence the caller named (the kernels' grids end there)
   const int *cu, *used;
 };
-__global__ __launch_bounds__(256) void zero_gaps_kernel(GapTensor a, GapTensor b, GapTensor c, int batch) {
+__global__ __launch_bounds__(256) void zero_gaps_kernel(GapTensor a, GapTensor b, GapTensor c, int batch, int slices) {
   const GapTensor t = blockIdx.y == 0 ? a : (blockIdx.y == 1 ? b : c);
-  const int g = blockIdx.x;   // gap g lies before sequence g (g = batch: after the last one)
+  const int g = min((int)blockIdx.x / slices, batch);   // gap g lies before sequence g (g = batch: after the last one)
+  const long long part = (int)blockIdx.x - g * slices, parts = g < batch ? slices : kTailParts;
   long long r0 = 0, r1 = g < batch ? t.cu[g] : t.rows;
   if (g > 0) {
     const int s0 = t.cu[g - 1], len = t.cu[g] - s0;
@@ -91,7 +95,7 @@ __global__ __launch_bounds__(256) void zero_gaps_kernel(GapTensor a, GapTensor b
   }
   r0 = max(r0, 0ll) * t.row16;
   r1 = min(r1, t.rows) * t.row16;
-  for (long long i = r0 + blockIdx.z * 256 + threadIdx.x; i < r1; i += 256ll * gridDim.z) t.base[i] = uint4{0u, 0u, 0u, 0u};
+  for (long long i = r0 + 256 * part + threadIdx.x; i < r1; i += 256 * parts) t.base[i] = uint4{0u, 0u, 0u, 0u};
 }
 
 }  // namespace fa
@@ -107,8 +111,13 @@ extern "C" int fable_attn_bwd_zero_gaps(FableBwdParams p, int dtype, int64_t tot
   if (p.dqs.s != (int64_t)p.Hq * p.D || p.dks.s != (int64_t)p.Hk * p.D || p.dvs.s != (int64_t)p.Hk * p.D)
     return fail(FA_ERR_ARG, "fable_attn_bwd_zero_gaps: rows are not contiguous");
   if (p.B < 0) return FA_OK;
-  hipLaunchKernelGGL(zero_gaps_kernel, dim3(p.B + 1, 3, 4), dim3(256), 0, (hipStream_t)stream,
-                     GapTensor{(uint4*)p.dQ, total_q, nq / 16, p.SQ, p.cu_q, p.seqused_q}, GapTensor{(uint4*)p.dK, total_k, nk / 16, p.SK, p.cu_k, p.seqused_k},
-                     GapTensor{(uint4*)p.dV, total_k, nk / 16, p.SK, p.cu_k, p.seqused_k}, p.B);
+  // (with a negative length fable_attn_bwd writes nothing)
+  const int mq = p.SQ < 0 || p.SK < 0 ? 0 : p.SQ, mk = p.SQ < 0 || p.SK < 0 ? 0 : p.SK;
+  int slices = 1;
+  if ((p.seqused_q || p.seqused_k) && p.B < kUsedParts) slices = kUsedParts / (p.B > 8 ? p.B : 8);
+  hipLaunchKernelGGL(zero_gaps_kernel, dim3(p.B * slices + kTailParts, 3), dim3(256), 0, (hipStream_t)stream,
+                     GapTensor{(uint4*)p.dQ, total_q, nq / 16, mq, p.cu_q, p.seqused_q},
+                     GapTensor{(uint4*)p.dK, total_k, nk / 16, mk, p.cu_k, p.seqused_k},
+                     GapTensor{(uint4*)p.dV, total_k, nk / 16, mk, p.cu_k, p.seqused_k}, p.B, slices);
   return launch_status("fable_attn_bwd_zero_gaps");
 }

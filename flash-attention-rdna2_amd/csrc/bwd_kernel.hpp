@@ -993,22 +993,24 @@ __global__ __launch_bounds__(256) void bwd_split_merge_kernel(FableBwdParams p, 
 // left each workgroup waiting on a single load pair: C3 33 us for 134 MB). Consecutive lane groups
 // take consecutive heads of a token, then the next token: in the (B, S, H, D) layouts of the API
 // a workgroup reads one contiguous run. (A workgroup per head read 256-byte pieces H*D apart: packed
-// batches of 25k rows of 32 heads, D 128, 125 us for 420 MB; now DSUM_US.) A packed batch's rows
-// are those of its whole buffer from cu_q[0] to cu_q[B], whatever sequence they belong to (rows past
-// a seqused end get a sum that nothing reads); the grid covers B times the longest sequence.
+// batches of 25k rows of 32 heads, D 128, 125 us for 420 MB; now 94.) A packed batch's rows
+// are those of its whole buffer from cu_q[0] to cu_q[B], whatever sequence they belong to; the grid
+// covers B times the longest sequence. With seqused (`per` workgroups for each sequence) they are the
+// used rows of each sequence: most of a buffer of fixed slots may be unused.
 constexpr int DSUM_RPT = 4;
 template <typename T, int HD>
-__global__ __launch_bounds__(256) void bwd_dsum_kernel(FableBwdParams p) {
+__global__ __launch_bounds__(256) void bwd_dsum_kernel(FableBwdParams p, int per) {
   constexpr int LPR = HD / 8, RPB = 256 / LPR;
   using V8 = typename Dt<T>::V8;
   const int tid = threadIdx.x;
   if (blockIdx.x == 0) ds_build_table(p);  // the dS workspace's tile table, for the next kernels
-  const long long q_first = p.cu_q ? p.cu_q[0] : 0;
-  const long long nrows = p.cu_q ? p.cu_q[p.B] - q_first : (long long)p.B * p.SQ, total = nrows * p.Hq;
+  const int z = per ? blockIdx.x / per : 0, nblk = per ? per : gridDim.x;
+  const long long q_first = p.cu_q ? p.cu_q[z] : 0;
+  const long long nrows = per ? bwd_seq(p, z).SQ : p.cu_q ? p.cu_q[p.B] - q_first : (long long)p.B * p.SQ, total = nrows * p.Hq;
   const int c = tid % LPR;
   // chunks past a head dim p.D below HD read the row's first chunk and add nothing
   const bool cok = 8 * c < p.D;
-  for (long long i0 = (long long)blockIdx.x * (RPB * DSUM_RPT); i0 < total; i0 += (long long)gridDim.x * (RPB * DSUM_RPT)) {
+  for (long long i0 = (long long)(blockIdx.x - z * nblk) * (RPB * DSUM_RPT); i0 < total; i0 += (long long)nblk * (RPB * DSUM_RPT)) {
   V8 o[DSUM_RPT], d[DSUM_RPT];
   long long at[DSUM_RPT];
 #pragma unroll
@@ -1324,7 +1326,8 @@ static int launch_bwd_ds(const FableBwdParams& p, hipStream_t st, int nkt) {
   // dim add zero)
   constexpr int DW = CKV::HD <= 32 ? 32 : (CKV::HD <= 64 ? 64 : (CKV::HD <= 128 ? 128 : 256));
   constexpr int RPB = 256 / (DW / 8) * DSUM_RPT;  // (row, head) pairs per dsum workgroup
-  const long long gd = ((long long)p.SQ * p.Hq * p.B + RPB - 1) / RPB;
+  const long long per = p.cu_q && p.seqused_q ? ((long long)p.SQ * p.Hq + RPB - 1) / RPB : 0;
+  const long long gd = per ? per * p.B : ((long long)p.SQ * p.Hq * p.B + RPB - 1) / RPB;
   // grids of fewer 8-wave workgroups than CUs run 4-wave ones (twice as many, half the rows)
   using CDS = BwdDsQCfg<CKV::HD, 4, CD::WPE, kDsqSets>;
   const int nqt = (p.SQ + CD::BQ - 1) / CD::BQ;
@@ -1333,7 +1336,7 @@ static int launch_bwd_ds(const FableBwdParams& p, hipStream_t st, int nkt) {
   const long long gq = (long long)(small ? nqts : nqt) * p.Hq * p.B;
   const long long gkv = (long long)nkt * p.Hk * p.B * CKV::DSPLIT;
   if (gd > 0x7FFFFFFF || gq > 0x7FFFFFFF || gkv > 0x7FFFFFFF) return fail(FA_ERR_ARG, "fable_attn_bwd: grid too large");
-  hipLaunchKernelGGL((bwd_dsum_kernel<T, DW>), dim3((unsigned)gd), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((bwd_dsum_kernel<T, DW>), dim3((unsigned)gd), dim3(256), 0, st, p, (int)per);
   if (int rc = launch_status("fable_attn_bwd (dsum)")) return rc;
   if constexpr (CKV::PAIR) {
     BwdSplit sp{1, nkt, CKV::BK, 0, nullptr};

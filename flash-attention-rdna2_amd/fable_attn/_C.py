@@ -372,9 +372,9 @@ def bwd_varlen(dout, q, k, v, out, lse, cu_q, cu_k, max_sq, max_sk, scale, causa
     p.seqused_q = seqused_q.data_ptr() if seqused_q is not None else None
     p.seqused_k = seqused_k.data_ptr() if seqused_k is not None else None
     p.lse_sb, p.lse_sh = 0, q.shape[0]
-    ws = _ds_workspace(p, _dt(q), q.device, ds_max_bytes)  # noqa: F841  (alive through the launch)
     with _on(q.device):
         _lib.check(_L.fable_attn_bwd_zero_gaps(p, _dt(q), q.shape[0], k.shape[0], _stream(q)), "fable_attn_bwd (varlen)")
+        ws = _ds_workspace(p, _dt(q), q.device, ds_max_bytes)  # noqa: F841  (alive through the launch)
         _lib.check(_L.fable_attn_bwd(p, _dt(q), _stream(q)), "fable_attn_bwd (varlen)")
     return dq, dk, dv
 

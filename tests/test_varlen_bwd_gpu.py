@@ -261,7 +261,8 @@ def test_varlen_backward_persistent(case, dt):
 
 @pytest.mark.parametrize("dt", [torch_dtype("bf16"), torch_dtype("f32")], ids=["bf16", "f32"])
 @pytest.mark.parametrize("used", [False, True], ids=["whole", "seqused"])
-def test_varlen_backward_rows_of_no_sequence(dt, used):
+@pytest.mark.parametrize("tail", [200, 6000])
+def test_varlen_backward_rows_of_no_sequence(dt, used, tail):
     """Rows before the first and after the last sequence, past seqused and of sequences without
     queries or keys: zero gradients, in buffers that held NaN before; the other rows as in a buffer
     that holds the sequences alone."""
@@ -270,7 +271,7 @@ def test_varlen_backward_rows_of_no_sequence(dt, used):
     from fable_attn import _C
     lq, lk, H, Hk, D = [40, 0, 130, 7], [64, 33, 0, 90], 4, 2, 64
     uq, uk = ([30, 0, 130, 2], [64, 20, 0, 50]) if used else (lq, lk)
-    lead, tail = 5, 200
+    lead = 5
     g = torch.Generator(device="cuda").manual_seed(1)
     rnd = lambda n, h: torch.randn(n, h, D, generator=g, device="cuda", dtype=torch.float32).to(dt)
     cu = lambda n: torch.tensor([lead + sum(n[:i]) for i in range(len(n) + 1)], dtype=torch.int32, device="cuda")
