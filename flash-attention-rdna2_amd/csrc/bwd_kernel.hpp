@@ -917,9 +917,43 @@ constexpr int kBwdPersistWG = 256, kBwdXcd = 8;
 // matter) keep the dispatched grid.
 constexpr long long kBwdPersistMinItems = 512;
 constexpr long long kBwdPersistMaxSteps = 16;
+// Work item of workgroup L of a packed batch's dispatched grid (at most kBwdSortMax sequences, one
+// lane each). Whole K/V groups go to the XCDs round-robin as in xcd_group_remap, the longest
+// sequences first; an XCD runs its groups in chunks of kBwdChunkKeys keys (by the longest sequence),
+// a chunk's first key blocks before its second ones. All groups of an XCD side by side (the rule for
+// dense batches, whose key blocks are alike) left each workgroup streaming Q and dO alone: a few key
+// blocks of a long sequence have to run together to share them in L2. One group after another
+// shares most but ends on whatever sequence comes last. bf16 backward, D 128, before -> now: 24
+// samples of 64-2048 rows, 32 / 8 heads 1720 -> 1480 us (one group at a time 1600, so with the longest
+// first 1518), not causal 3233 -> 2500; 8 of 1000-8000 rows, 16 / 4 heads 4959 -> 3459; 60 of 16-700
+// rows 544 -> 530; 64 of 20-200 rows 158 -> 160; 8 of 2048 rows 1048 -> 1052.
+constexpr int kBwdChunkKeys = 8192, kBwdSortMax = 64;
+__device__ __forceinline__ int bwd_packed_item(const FableBwdParams& p, int nkt, int L) {
+  const int groups = p.Hk * p.B, R = groups / kBwdXcd, M = R * kBwdXcd * nkt;
+  int group, u;
+  if (L >= M) {  // the groups past the last full round, as in xcd_group_remap
+    const int w = M + xcd_remap(L - M, groups * nkt - M);
+    group = w / nkt;
+    u = w - group * nkt;
+  } else {
+    const int x = L % kBwdXcd, k = L / kBwdXcd, cg = max(kBwdChunkKeys / p.SK, 1);
+    const int c = k / (cg * nkt), kk = k - c * cg * nkt, n = min(cg, R - c * cg);
+    u = kk / n;
+    group = x + kBwdXcd * (c * cg + kk - u * n);
+  }
+  const int r = group / p.Hk, kvh = group - r * p.Hk, lane = threadIdx.x & 63;
+  const int len = lane < p.B ? bwd_seq(p, lane).SQ : 0;
+  int rank = 0;  // of sequence `lane`; ties in their order
+  for (int i = 0; i < p.B; i++) {
+    const int li = __builtin_amdgcn_readlane(len, i);
+    rank += li > len || (li == len && i < lane);
+  }
+  const int b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < p.B && rank == r));
+  return (b * p.Hk + kvh) * nkt + u;
+}
 // The pair kernel. Dispatched (PERSIST false): one work item per workgroup, the grid
 // share-major (every key block's first share, then the second, ...) and mapped to items by
-// xcd_group_remap. Persistent (PERSIST true, no query split): a fixed grid of kBwdPersistWG
+// xcd_group_remap (packed batches without a split: bwd_packed_item). Persistent (PERSIST true, no query split): a fixed grid of kBwdPersistWG
 // workgroups per CU slot, each running a fixed list of items. Workgroup L of the dispatched
 // grid runs on XCD L % 8 (round-robin dispatch), so XCD x's share of the work is the items of
 // L = x + 8 j, j = 0, 1, ..., in that order; the R persistent workgroups of XCD x (blockIdx % 8
@@ -934,8 +968,9 @@ bwd_dkdv_pair_kernel(FableBwdParams p, int nkt, BwdSplit sp) {
   if constexpr (!PERSIST) {
     const int nitems = gridDim.x / sp.n;
     const int share = blockIdx.x / nitems;
-    bwd_pair_item<T, C, CAUSAL, FEAT, DROP, DSW, false>(p, nkt, sp, xcd_group_remap(blockIdx.x - share * nitems, nitems, nkt, 1, kBwdUMajor),
-                                                        share);
+    const int w = p.cu_q && sp.n == 1 && p.B <= kBwdSortMax ? bwd_packed_item(p, nkt, blockIdx.x)
+                                                            : xcd_group_remap(blockIdx.x - share * nitems, nitems, nkt, 1, kBwdUMajor);
+    bwd_pair_item<T, C, CAUSAL, FEAT, DROP, DSW, false>(p, nkt, sp, w, share);
   } else {
     const int x = blockIdx.x % kBwdXcd, r = blockIdx.x / kBwdXcd, R = gridDim.x / kBwdXcd;
     const long long nitems = (long long)nkt * p.Hk * p.B;

@@ -304,3 +304,36 @@ def test_varlen_backward_rows_of_no_sequence(dt, used, tail):
         for x, y in zip((got[0][a:a + uq[z]], got[1][b:b + uk[z]], got[2][b:b + uk[z]]), ref):
             tol = 2.0 ** -7 if dt is torch.bfloat16 else 1e-5
             assert (x.float() - y.float()).abs().max() <= tol * y.float().abs().max()
+
+
+@pytest.mark.parametrize("batch,Hk,longest,D,causal", [(2, 1, 300, 128, True), (5, 3, 300, 128, False), (5, 3, 5000, 128, True),
+                                                       (64, 2, 300, 64, True), (65, 1, 300, 64, True), (9, 8, 1100, 96, True)])
+def test_varlen_backward_work_order(batch, Hk, longest, D, causal):
+    """The order of a packed batch's work items (longest sequences first, in chunks of groups; more
+    than 64 sequences: as they come): every key block of every sequence exactly once, whatever the
+    lengths (equal ones, empty ones, a max_seqlen above them) and the count of K/V groups."""
+    import torch
+
+    from fable_attn import _C
+    H = 2 * Hk
+    r = np.random.default_rng(batch)
+    lens = [int(x) for x in r.integers(0, min(longest, 1100), batch)]
+    lens[0], lens[-1], lens[batch // 2] = 0, lens[1], min(longest, 1100)
+    at = [sum(lens[:i]) for i in range(batch + 1)]
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    rnd = lambda h: torch.randn(at[-1], h, D, generator=g, device="cuda", dtype=torch.bfloat16)
+    cu = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    q, do, k, v = rnd(H), rnd(H), rnd(Hk), rnd(Hk)
+    args = (D ** -0.5, causal, -1, -1, 0.0, None, 0.0, 0)
+    out, lse = _C.fwd_varlen(q, k, v, cu(at), cu(at), longest, longest, *args, 0, None, None, return_lse=True)
+    poison = [torch.full_like(x, float("nan")) for x in (q, k, v)]
+    del poison   # (the allocator hands the same memory out again)
+    got = _C.bwd_varlen(do, q, k, v, out, lse, cu(at), cu(at), longest, longest, *args)
+    for z in range(batch):
+        if not lens[z]:
+            continue
+        s = slice(at[z], at[z + 1])
+        ref = _C.bwd_varlen(*(x[s].contiguous() for x in (do, q, k, v, out)), lse[:, s].contiguous(), cu([0, lens[z]]),
+                            cu([0, lens[z]]), lens[z], lens[z], *args)
+        for x, y in zip(got, ref):   # (a split of the small grid moves a sum across at most one rounding)
+            assert (x[s].float() - y.float()).abs().max() <= 2.0 ** -7 * y.float().abs().max()
