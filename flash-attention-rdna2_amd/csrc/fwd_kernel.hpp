@@ -289,13 +289,17 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
   // each load of the next K tile is fetched a tile ahead by a vector load (a scalar one would
   // share its counter with the LDS reads), and made uniform when the K tile is loaded; the V
   // tile, one behind, takes the entries its K tile used.
+  // The caller's range starts at bk0, the first key a row of the workgroup sees: ahead of it (a left
+  // pad, keys that left the window) table entries may name no page and rows may hold anything. The
+  // first tile starts at bk0 rounded down, so entries are looked up from bk0 on, and that tile's rows
+  // before it read as zeros (masked, they would still meet P = 0 as 0 * NaN).
   constexpr int NE = PG ? C::KJ : 1;
   static_assert(!PG || (kRowStep && 64 % C::DCH == 0 && 64 / C::DCH <= 16), "paged loads");
   int ent[NE], ekey = kstart, pg_cur[NE], pg_prev[NE];  // next K tile's entries and first key
   const int wrow = tid / 64 * (64 / C::DCH);            // first row of the wave's first load
   auto pg_index = [&](int j) {
     if constexpr (PG)
-      return z * pg.max_blocks + (min(ekey + wrow + j * RSTEP, kvalid - 1) >> pg.page_shift);
+      return z * pg.max_blocks + (min(max(ekey + wrow + j * RSTEP, FEAT ? bk0 : 0), kvalid - 1) >> pg.page_shift);
     else
       return 0;
   };
@@ -305,15 +309,15 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
       for (int j = 0; j < NE; j++) ent[j] = pg.table[pg_index(j) & pg.tmask];
     }
   };
-  auto pg_load = [&](u32x4 (&ld)[C::KJ], const T* base, int key0, const int (&page)[NE], long long spg, long long srow,
-                     const int (&off)[C::KJ]) {
+  auto pg_load = [&](bool first, u32x4 (&ld)[C::KJ], const T* base, int key0, const int (&page)[NE], long long spg,
+                     long long srow, const int (&off)[C::KJ]) {
     if constexpr (PG) {
 #pragma unroll
       for (int j = 0; j < NE; j++) {
         const int key = __builtin_amdgcn_readfirstlane(key0 + wrow + j * RSTEP);
         const int in = key & ((1 << pg.page_shift) - 1);
         const auto r = buf_rsrc(base + page[j] * spg + in * srow, (long long)(kvalid - key) * srow * 2);
-        ld[j] = buf_load16(r, off[j]);
+        ld[j] = buf_load16(r, FEAT && first && key + lane / C::DCH < bk0 ? kBufZero : off[j]);
       }
     }
   };
@@ -327,14 +331,14 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
     }
     if (ntiles > 0) pg_fetch();
   }
-  auto gload_k = [&]() {
+  auto gload_k = [&](bool first = false) {
     if constexpr (PG) {
 #pragma unroll
       for (int j = 0; j < NE; j++) {
         pg_prev[j] = pg_cur[j];
         pg_cur[j] = __builtin_amdgcn_readfirstlane((ent[j] & pg.tmask) | (pg_index(j) & ~pg.tmask));
       }
-      pg_load(ldk, Kg, ekey, pg_cur, pg.kpg, p.sK.s, koff);
+      pg_load(first, ldk, Kg, ekey, pg_cur, pg.kpg, p.sK.s, koff);
       ekey += C::BC;
       pg_fetch();
       return;
@@ -346,9 +350,9 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
     k_left -= 2 * k_step;
   };
   // (PG: `ahead` K tiles have been loaded past this V tile, 0 or 1)
-  auto gload_v = [&](int ahead = 1) {
+  auto gload_v = [&](int ahead = 1, bool first = false) {
     if constexpr (PG) {
-      pg_load(ldv, Vg, ekey - (1 + ahead) * C::BC, ahead ? pg_prev : pg_cur, pg.vpg, p.sV.s, voff);
+      pg_load(first, ldv, Vg, ekey - (1 + ahead) * C::BC, ahead ? pg_prev : pg_cur, pg.vpg, p.sV.s, voff);
       return;
     }
     const auto r = buf_rsrc(v_cur, v_left);
@@ -633,8 +637,8 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
   if (ntiles > 0) {
 #pragma unroll
     for (int j = 0; j < BP; j++) {
-      gload_k();   // tile j
-      gload_v(0);  // tile j
+      gload_k(j == 0);     // tile j
+      gload_v(0, j == 0);  // tile j
       lstore_k(j);
       lstore_v(j);
     }

@@ -91,3 +91,44 @@ def test_tiles_partial_rotary():
         # to bf16: four independent roundings of at most 2^-9, rms 2^-9 / sqrt(3) each, so
         # 2.3e-3 is expected; the bound is 2^-8
         assert orc.rel_rms(a.cpu().numpy(), b.cpu().numpy()) <= 2.0 ** -8
+
+
+def hide(c):
+    """The case with NaN in every K and V row below the first key a token sees, and with the table entries
+    of whole pages below it naming one page of NaN (a read there shows as a wrong value)."""
+    kc, vc = (np.concatenate([c[n], np.full_like(c[n][:1], np.nan)]) for n in ("kc", "vc"))
+    bt, page = c["bt"].copy(), c["kc"].shape[1]
+    for b, cx in enumerate(c["ctx"]):
+        lo = max(c["lp"][b] if c["lp"] is not None else 0, cx - c["window"] + 1 if c["window"] >= 0 else 0)
+        lo = min(lo, cx)             # (the new keys are written, whatever the pad)
+        for x in (kc, vc):
+            if lo // page < bt.shape[1]:
+                x[bt[b, lo // page], :lo % page] = np.nan
+        bt[b, :lo // page] = len(kc) - 1
+    return dict(c, kc=kc, vc=vc, bt=bt)
+
+
+# name, HD, NH, gqa, ctx(list per batch), window, rotary, append, leftpad, nq, softcap, alibi, page
+HIDDEN = [
+    ("window", 128, 4, 2, [1200, 90, 333], 100, 0, True, 0, 70, 0.0, False, 16),
+    ("window no append rotary", 128, 8, 8, [1200, 90], 101, 1, False, 0, 12, 0.0, False, 16),
+    ("window split", 128, 8, 8, [5003], 2000, 0, True, 0, 12, 0.0, False, 16),
+    ("leftpad", 128, 4, 2, [600, 80], -1, 0, True, 37, 70, 0.0, False, 16),
+    ("leftpad one page", 128, 4, 2, [600, 80], -1, 1, True, 37, 70, 0.0, False, 1024),
+    ("leftpad past the keys", 128, 4, 2, [600, 20], -1, 0, False, 63, 70, 0.0, False, 16),
+    ("D64 window", 64, 8, 4, [777, 5], 201, 0, True, 0, 33, 25.0, False, 64),
+    ("D40 leftpad", 40, 4, 2, [300], -1, 1, True, 49, 50, 0.0, False, 16),
+    ("D256 window leftpad", 256, 4, 4, [520, 64], 128, 0, True, 33, 40, 0.0, False, 16),
+    ("D256 alibi leftpad", 256, 4, 4, [520, 64], -1, 0, True, 31, 40, 0.0, True, 32),
+    ("below the tiles", 128, 4, 2, [600, 80], 99, 1, True, 37, 5, 0.0, False, 16),
+]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("case", HIDDEN, ids=[c[0] for c in HIDDEN])
+def test_nothing_below_the_first_visible_key_is_read(case, dt):
+    print(f"[tiles] hidden {case[0]} {dt}", flush=True)
+    c = make_case(case, dt)
+    o, l, _, _ = run_kernel(hide(c), dt)
+    o_ref, l_ref = run_oracle(c, dt)
+    check(o, l, o_ref, l_ref, dt, "hidden " + case[0])

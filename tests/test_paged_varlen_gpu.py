@@ -87,3 +87,30 @@ def test_paged_equals_gathered(case, dt):
         # both are within TOL of the exact result
         assert orc.rel_rms(a, b) <= 2 * TOL[dt], kw
         assert np.array_equal(a == 0, b == 0), kw   # rows without a key
+
+
+@pytest.mark.parametrize("D,page,window", [(128, 16, 100), (64, 64, 77), (256, 16, 33), (40, 32, 5)])
+def test_pages_before_the_window_are_not_read(D, page, window):
+    """NaN in the rows that no query's window reaches, and in the page that their table entries name."""
+    import torch
+
+    from fable_attn import flash_attn_varlen_func
+    lq, lk, Hk = [70, 9, 130], [700, 300, 130], 2
+    g = torch.Generator(device="cuda").manual_seed(4)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=torch.bfloat16)
+    nb = -(-max(lk) // page)
+    kc, vc = rnd(3 * nb + 1, page, Hk, D), rnd(3 * nb + 1, page, Hk, D)
+    bt = torch.randperm(3 * nb, generator=torch.Generator().manual_seed(5)).view(3, nb).int()
+    q = rnd(sum(lq), 4, D)
+    cu = lambda n: torch.tensor([0] + list(np.cumsum(n)), dtype=torch.int32, device="cuda")
+    f = lambda table: flash_attn_varlen_func(q, kc, vc, cu(lq), cu(lk), max(lq), max(lk), block_table=table.cuda(),
+                                             causal=True, window_size=(window, 0))
+    want = f(bt)
+    kc[-1], vc[-1] = float("nan"), float("nan")
+    hidden = bt.clone()
+    for z in range(3):
+        lo = max(lk[z] - lq[z] - window, 0)
+        kc[bt[z, lo // page].item(), :lo % page] = float("nan")
+        vc[bt[z, lo // page].item(), :lo % page] = float("nan")
+        hidden[z, :lo // page] = 3 * nb
+    assert torch.equal(f(hidden), want)
