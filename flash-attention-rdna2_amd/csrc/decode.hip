@@ -1166,9 +1166,11 @@ namespace fa {
 // to 32, 500 to 32000 keys, D 64 to 256; 16 tokens of 4 heads over 32000 keys 227 -> 51 us), at
 // 512 rows 0.07-0.39x.
 constexpr int kTileRows = 64;
+// (A window of 0 keys, which leaves no key visible, has no form in the forward's bounds: the decode
+// kernel serves it.)
 static bool dec_uses_tiles(const FableDecParams& p, int dtype) {
   return (dtype == FA_F16 || dtype == FA_BF16) && p.gqa > 0 && (long long)p.nq * p.gqa >= kTileRows && p.page >= 16 &&
-         p.HD > 0 && p.HD <= 256 && p.HD % 8 == 0;
+         p.window != 0 && p.HD > 0 && p.HD <= 256 && p.HD % 8 == 0;
 }
 
 // One workgroup per new token, before the tile kernel: the token's k (rotated) and v rows go to

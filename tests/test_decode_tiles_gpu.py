@@ -132,3 +132,13 @@ def test_nothing_below_the_first_visible_key_is_read(case, dt):
     o, l, _, _ = run_kernel(hide(c), dt)
     o_ref, l_ref = run_oracle(c, dt)
     check(o, l, o_ref, l_ref, dt, "hidden " + case[0])
+
+
+@pytest.mark.parametrize("append", [False, True])
+@pytest.mark.parametrize("nq", [3, 31, 32, 70])
+def test_window_of_no_keys(nq, append):
+    """window 0 hides every key (a token sees keys from its position + 1 on) on both sides of the row count
+    at which the tile kernel starts (64: 32 tokens of 2 heads)."""
+    c = make_case(("window 0", 128, 4, 2, [300, 0], 0, 0, append, 0, nq, 0.0, False, 16), "bf16")
+    o, l, _, _ = run_kernel(c, "bf16")
+    assert not o.any() and np.isneginf(l).all()
