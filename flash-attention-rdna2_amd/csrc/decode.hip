@@ -1267,7 +1267,8 @@ static long long dec_q_bytes(const FableDecParams& p) {
 }
 
 template <typename T>
-static int launch_dec_tiles(const FableDecParams& p, int dtype, char* ws, long long ws_bytes, hipStream_t st, const void* nk, const void* nv) {
+static int launch_dec_tiles(const FableDecParams& p, int dtype, int nsplit, char* ws, long long ws_bytes, hipStream_t st, const void* nk,
+                            const void* nv) {
   FableFwdParams f;
   FwdPaged pg;
   dec_tile_params(p, nk != nullptr, f, pg);
@@ -1284,7 +1285,7 @@ static int launch_dec_tiles(const FableDecParams& p, int dtype, char* ws, long l
       pg.qlo = qlo;
     }
   }
-  FwdWs fw{ws ? ws + 2 * qb : nullptr, ws_bytes - 2 * qb, false, 0};
+  FwdWs fw{ws ? ws + 2 * qb : nullptr, ws_bytes - 2 * qb, false, 0, nsplit};
   return launch_fwd_paged(f, pg, dtype, p.rotary != 0, st, fw);
 }
 
@@ -1315,8 +1316,8 @@ static int dec_checked(FableDecParams p, int dtype, void* stream, const void* ne
 
 }  // namespace fa
 
-// fable_attn_dec with one workspace for whatever the call needs. p.nsplit: the caller's hint (0:
-// the library's choice), which the many-token path does not take.
+// fable_attn_dec with one workspace for whatever the call needs. p.nsplit: the caller's count (0:
+// the library's choice).
 // Whether the shares are worked out on the device: fp16/bf16, no count of the caller's, pages of at
 // least 16 rows, a table that can hold kShareBytes of keys and values, and a batch that equal
 // splits would not spread evenly over the parts (more sequences than parts, or a count that
@@ -1348,7 +1349,7 @@ extern "C" int64_t fable_attn_dec_ws_bytes(FableDecParams p, int dtype, int appe
     FableFwdParams f;
     FwdPaged pg;
     dec_tile_params(p, append != 0, f, pg);
-    FwdWs fw{nullptr, 0, true, 0};
+    FwdWs fw{nullptr, 0, true, 0, p.nsplit};
     if (launch_fwd_paged(f, pg, dtype, p.rotary != 0, nullptr, fw) != FA_OK) return -1;
     return 2 * dec_q_bytes(p) + fw.need;
   }
@@ -1369,8 +1370,8 @@ extern "C" int fable_attn_dec_ws(FableDecParams p, int dtype, void* ws, int64_t 
   if (int rc = dec_check(p, new_k, new_v)) return rc;
   if (p.batch <= 0) return FA_OK;
   if (tiles)
-    return dtype == FA_F16 ? launch_dec_tiles<_Float16>(p, dtype, (char*)ws, ws_bytes, (hipStream_t)stream_, new_k, new_v)
-                           : launch_dec_tiles<__bf16>(p, dtype, (char*)ws, ws_bytes, (hipStream_t)stream_, new_k, new_v);
+    return dtype == FA_F16 ? launch_dec_tiles<_Float16>(p, dtype, hint, (char*)ws, ws_bytes, (hipStream_t)stream_, new_k, new_v)
+                           : launch_dec_tiles<__bf16>(p, dtype, hint, (char*)ws, ws_bytes, (hipStream_t)stream_, new_k, new_v);
   long long need;
   if (share) {
     need = dec_share_bytes(p);

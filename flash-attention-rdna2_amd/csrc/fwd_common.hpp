@@ -152,6 +152,7 @@ struct FwdWs {
   long long bytes;
   bool query;
   long long need;  // out: workspace bytes of the split this call takes (0: none)
+  int nsplit = 0;  // paged instances: the caller's split count (0: the launcher's choice)
 };
 
 // the fp16/bf16 forward per kernel width (fwd_d32 ... fwd_d256.hip: head dims up to the width,

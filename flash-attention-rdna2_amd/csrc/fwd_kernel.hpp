@@ -897,7 +897,8 @@ struct CfgTag {
 
 // Launcher of the paged instances: C for the plain masks, CF for the feature masks and for a
 // rotated q. A grid that leaves CUs idle splits the keys of each tile (as fwd_split_count, up
-// to kPagedSplitMax shares of at least kPagedSplitTiles tiles of the longest cache the table holds).
+// to kPagedSplitMax shares of at least kPagedSplitTiles tiles of the longest cache the table holds); a
+// split count of the caller's is taken as it is, up to kPagedSplitMax.
 constexpr int kPagedSplitMax = 32, kPagedSplitTiles = 4;
 template <typename T, class C, class CF>
 static int launch_fwd_pg(const FableFwdParams& p, const FwdPaged& pg, bool rot, hipStream_t st, FwdWs& ws) {
@@ -914,6 +915,7 @@ static int launch_fwd_pg(const FableFwdParams& p, const FwdPaged& pg, bool rot, 
     const long long tiles = ((long long)p.SK + K::BC - 1) / K::BC;
     long long n = kSlots / nblk;
     n = n < tiles / kPagedSplitTiles ? n : tiles / kPagedSplitTiles;
+    if (ws.nsplit > 0) n = ws.nsplit < 0x7FFFFFFF / nblk ? ws.nsplit : 0x7FFFFFFF / nblk;
     n = n < kPagedSplitMax ? n : kPagedSplitMax;
     FwdSplit sp{1, nqt, K::BR, 0, nullptr, nullptr};
     ws.need = 0;

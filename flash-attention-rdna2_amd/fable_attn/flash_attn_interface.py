@@ -59,7 +59,8 @@ def _reject_fp8(q_descale, k_descale, v_descale):
 
 def _accept_hints(num_splits=None, pack_gqa=None, sm_margin=None):
     """Scheduling hints change the schedule, never the result; only their types are checked
-    (reference :110-128). num_splits is honoured by decode."""
+    (reference :110-128). num_splits is honoured by decode
+    (up to 32 splits where 64 or more rows share a K/V head, up to 512 below that)."""
     for name, val, ok in (("num_splits", num_splits, int), ("pack_gqa", pack_gqa, bool),
                           ("sm_margin", sm_margin, int)):
         if val is not None and not isinstance(val, ok):

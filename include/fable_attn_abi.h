@@ -336,9 +336,9 @@ int fable_attn_dec(FableDecParams p, int dtype, void* stream, const void* new_k,
 /* fable_attn_dec with one workspace for whatever the call needs (p.scratch is ignored), and the
  * choice of path left to the library: calls with many new tokens run on the forward's tile kernel
  * (each K/V row read once per query tile instead of once per new token). p.nsplit is the caller's
- * hint, 0 for the library's choice; the tile path does not take it. p.block_table may be NULL in
- * fp16/bf16: sequence b's pages are then b*max_blocks, b*max_blocks+1, ... (a dense cache). fable_attn_dec_ws_bytes gives
- * the bytes to pass (256-byte aligned device memory, scratch per call); `append` tells whether
+ * split count, 0 for the library's choice (at most 32 splits on the tile path, 512 elsewhere).
+ * p.block_table may be NULL in fp16/bf16: sequence b's pages are then b*max_blocks, b*max_blocks+1,
+ * ... (a dense cache). fable_attn_dec_ws_bytes gives the bytes to pass (256-byte aligned device memory, scratch per call); `append` tells whether
  * new_k/new_v will be passed. Same results as fable_attn_dec up to fp32 summation order. */
 int64_t fable_attn_dec_ws_bytes(FableDecParams p, int dtype, int append);
 int fable_attn_dec_ws(FableDecParams p, int dtype, void* ws, int64_t ws_bytes, void* stream, const void* new_k,

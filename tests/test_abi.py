@@ -282,3 +282,20 @@ def test_forward_key_split_workspace_query():
     assert q(B=1, H=8, SQ=256, SK=256, D=64) == 0                          # too few key tiles
     assert q(B=1, H=8, SQ=1024, SK=1024, D=60) == -1                       # no kernel for D=60
     assert b"head_dim=60" in lib.fable_attn_last_error()
+
+
+def test_decode_split_count_of_many_tokens():
+    """The caller's split count holds for calls of 64 or more rows per K/V head too: one split needs no
+    workspace, n splits n partials (O in fp32 and the LSE) of every query tile, up to 32."""
+    from fable_attn import _lib
+    L = _lib.load()
+
+    def need(n):
+        p = _lib.FableDecParams()
+        p.batch, p.NH, p.gqa, p.HD, p.page, p.max_blocks, p.nq, p.window, p.scale = 1, 8, 8, 128, 16, 512, 16, -1, 0.1
+        p.nsplit = n
+        return L.fable_attn_dec_ws_bytes(p, _lib.FA_BF16, 1)
+    assert need(0) > 0 and need(1) == 0
+    rows = need(2) // 2 // (128 * 4 + 4)
+    assert rows >= 128 and all(need(n) == n * rows * (128 * 4 + 4) for n in (2, 3, 8, 32))
+    assert need(100) == need(32)

@@ -142,3 +142,11 @@ def test_window_of_no_keys(nq, append):
     c = make_case(("window 0", 128, 4, 2, [300, 0], 0, 0, append, 0, nq, 0.0, False, 16), "bf16")
     o, l, _, _ = run_kernel(c, "bf16")
     assert not o.any() and np.isneginf(l).all()
+
+
+@pytest.mark.parametrize("splits", [1, 2, 5, 32, 100])
+def test_split_counts(splits):
+    c = make_case(("splits", 128, 16, 8, [3000, 70, 0], -1, 1, True, 0, 17, 0.0, False, 16), "f16")
+    o, l, _, _ = run_kernel(c, "f16", num_splits=splits)
+    o_ref, l_ref = run_oracle(c, "f16")
+    check(o, l, o_ref, l_ref, "f16", f"tiles in {splits} splits")
