@@ -20,8 +20,9 @@
 //    split;
 //  * the combine kernel merges the splits (natural-log LSE optional);
 //  * appending new_k/new_v (with rotary on k) needs no synchronisation of the device (the
-//    reference's hipDeviceSynchronize(), fa_decode.hip:348-351): one new token is written by the
-//    workgroups that read it, several by a kernel earlier in the same stream.
+//    reference's hipDeviceSynchronize(), fa_decode.hip:348-351): one new token of a single sequence or
+//    of a dense cache is written by the workgroups that read it, all others by a kernel earlier in
+//    the same stream.
 // Scores are handled in the log2 domain; partial maxima are stored in log2 units.
 #include <mutex>
 #include <type_traits>
@@ -305,7 +306,8 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
 
   // ---- a single new key (nk) -> the cache (rotated k, v), by the workgroups that read it next: an
   // append kernel of its own cost 3 us ahead of a 9 us decode. (Row groups of one head write the
-  // same bytes. Several tokens keep the kernel: written here one after another they cost more.)
+  // same bytes. Which calls come here: dec_fuses_append. Several tokens keep the kernel: written here
+  // one after another they cost more.)
   if (append && ctx >= start && ctx < end) {
     const DecArgs p = dec_reload();
     if (p.nk) {
@@ -950,10 +952,13 @@ static int launch_dec_append(const FableDecParams& p, hipStream_t st, const void
                      __builtin_ctz((unsigned)p.page));
   return launch_status("fable_attn_dec (append)");
 }
-// whether the partial kernel writes the new key itself: one token per sequence
+// Whether the partial kernel writes the new key itself: one token per sequence, whose row no other
+// sequence can read. With a block table two sequences may name one page (drafted tokens laid out as
+// batch rows of successive lengths, a cache row given twice), and then a workgroup that reads the row
+// must find it written: by a kernel ahead, as for several tokens. (v is copied in 16-byte pieces.)
 template <typename T>
-static bool dec_fuses_append(const FableDecParams& p) {
-  return !std::is_same<T, float>::value && p.nq == 1;
+static bool dec_fuses_append(const FableDecParams& p, const void* nv) {
+  return !std::is_same<T, float>::value && p.nq == 1 && (!p.block_table || p.batch == 1) && ((uintptr_t)nv & 15) == 0;
 }
 
 template <typename T, int HD>
@@ -961,7 +966,7 @@ static int launch_dec(const FableDecParams& p, hipStream_t st, const void* nk, c
   const int page_shift = __builtin_ctz((unsigned)p.page);
   const int NKV = p.NH / p.gqa;
   const int ngrp = (p.gqa + 15) / 16;
-  const bool fuse = dec_fuses_append<T>(p);
+  const bool fuse = dec_fuses_append<T>(p, nv);
   if (nk && !fuse)
     if (int rc = launch_dec_append<T, HD>(p, st, nk, nv)) return rc;
   const bool feat = p.softcap > 0.0f || p.alibi != nullptr;
@@ -992,7 +997,7 @@ static int launch_dec(const FableDecParams& p, hipStream_t st, const void* nk, c
 template <typename T, int HD>
 static int launch_dec_share(const FableDecParams& p, hipStream_t st, const void* nk, const void* nv) {
   const int ngrp = dec_groups(p), X = p.NH / p.gqa * ngrp, parts = dec_parts(p);
-  const bool fuse = dec_fuses_append<T>(p);
+  const bool fuse = dec_fuses_append<T>(p, nv);
   if (nk && !fuse)
     if (int rc = launch_dec_append<T, HD>(p, st, nk, nv)) return rc;
   if (int rc = launch_dec_partial<T, HD>(p, dim3((unsigned)(X * dec_share_wgs(p))), __builtin_ctz((unsigned)p.page), nk ? kDecAppend : 0, parts,

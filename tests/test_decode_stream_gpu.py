@@ -116,3 +116,60 @@ def test_dense_cache_without_table(nq):
         res.append((out, kc, vc))
     for a, b in zip(*res):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("rotary", [False, True])
+@pytest.mark.parametrize("paged", [True, False], ids=["paged", "dense"])
+def test_appends_to_a_shared_cache_row(paged, rotary):
+    """Tokens of one sequence laid out as batch rows of successive lengths (one block table, or one
+    cache row by cache_batch_idx): each row sees the keys that the rows before it append in the same
+    call, as the same tokens of one batch row do. Called twice, as a serving loop does."""
+    import torch
+
+    from fable_attn import flash_attn_with_kvcache
+    n, H, Hk, D, L, cap, page = 8, 8, 2, 128, 1500, 4096, 16
+    g = torch.Generator(device="cuda").manual_seed(2)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=torch.bfloat16)
+    q, k, v = rnd(1, n, H, D), rnd(1, n, Hk, D), rnd(1, n, Hk, D)
+    kc0, vc0 = (rnd(cap // page, page, Hk, D) if paged else rnd(2, cap, Hk, D) for _ in range(2))
+    table = torch.randperm(cap // page, generator=torch.Generator().manual_seed(3)).view(1, -1).int().cuda()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    ang = torch.rand(cap, D // 2, generator=g, device="cuda") * 6.28
+    opt = dict(rotary_cos=ang.cos(), rotary_sin=ang.sin()) if rotary else {}
+    where = lambda b: dict(block_table=table.expand(b, -1).contiguous()) if paged else dict(cache_batch_idx=i32([1] * b))
+    rows = lambda t: t.view(n, 1, *t.shape[2:]).contiguous()
+    res = []
+    for b, args in ((1, (q, k, v)), (n, tuple(rows(t) for t in (q, k, v)))):
+        lens = i32([L] if b == 1 else [L + i for i in range(n)])
+        for _ in range(2):
+            kc, vc = kc0.clone(), vc0.clone()
+            out = flash_attn_with_kvcache(args[0], kc, vc, args[1], args[2], cache_seqlens=lens, **where(b), **opt)
+        res.append((out.reshape(n, H, D).float(), kc, vc))
+    torch.cuda.synchronize()
+    (a, ka, va), (b, kb, vb) = res
+    assert torch.equal(ka, kb) and torch.equal(va, vb)
+    # both round their probabilities (to running maxima of their own) and results to bf16, as in
+    # test_decode_tiles_gpu.test_tiles_partial_rotary
+    assert orc.rel_rms(a.cpu().numpy(), b.cpu().numpy()) <= 2.0 ** -8
+
+
+def test_append_of_a_misaligned_new_token():
+    """new_v needs no alignment at the C-ABI entry points of the decode kernel."""
+    import torch
+
+    from fable_attn import _lib
+    L = _lib.load()
+    B, H, Hk, D, cap = 1, 8, 2, 128, 256
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=torch.bfloat16)
+    q, nk, kc, vc = rnd(B, 1, H, D), rnd(B, 1, Hk, D), rnd(B, cap, Hk, D), rnd(B, cap, Hk, D)
+    nv = rnd(B * Hk * D + 1)[1:].view(B, 1, Hk, D)
+    lens, table = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([100], [[0]]))
+    out = torch.empty_like(q)
+    p = _lib.FableDecParams()
+    p.q, p.Kc, p.Vc, p.o, p.ctx_len = q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), lens.data_ptr()
+    p.block_table, p.nsplit = table.data_ptr(), 1
+    p.batch, p.NH, p.gqa, p.HD, p.page, p.max_blocks, p.nq, p.window, p.scale = B, H, H // Hk, D, cap, 1, 1, -1, D ** -0.5
+    _lib.check(L.fable_attn_dec(p, _lib.FA_BF16, torch.cuda.current_stream().cuda_stream, nk.data_ptr(), nv.data_ptr()), "dec")
+    torch.cuda.synchronize()
+    assert torch.equal(vc[0, 100], nv[0, 0]) and torch.equal(kc[0, 100], nk[0, 0])
