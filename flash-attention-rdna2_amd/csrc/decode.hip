@@ -1172,10 +1172,10 @@ namespace fa {
 // 512 rows 0.07-0.39x.
 constexpr int kTileRows = 64;
 // (A window of 0 keys, which leaves no key visible, has no form in the forward's bounds: the decode
-// kernel serves it.)
+// kernel serves it; so does it tables of 2^31 entries and more.)
 static bool dec_uses_tiles(const FableDecParams& p, int dtype) {
   return (dtype == FA_F16 || dtype == FA_BF16) && p.gqa > 0 && (long long)p.nq * p.gqa >= kTileRows && p.page >= 16 &&
-         p.window != 0 && p.HD > 0 && p.HD <= 256 && p.HD % 8 == 0;
+         (long long)p.batch * p.max_blocks <= 0x7FFFFFFF && p.window != 0 && p.HD > 0 && p.HD <= 256 && p.HD % 8 == 0;
 }
 
 // One workgroup per new token, before the tile kernel: the token's k (rotated) and v rows go to

@@ -299,3 +299,20 @@ def test_decode_split_count_of_many_tokens():
     rows = need(2) // 2 // (128 * 4 + 4)
     assert rows >= 128 and all(need(n) == n * rows * (128 * 4 + 4) for n in (2, 3, 8, 32))
     assert need(100) == need(32)
+
+
+def test_paged_prompts_served():
+    """What the paged prompt kernel takes: a row stride of which 16 rows pass 2^31 bytes is left to the
+    gather (the kernel's offsets within a load are 32 bits wide), as are other widths and small pages."""
+    from fable_attn import _lib
+    L = _lib.load()
+
+    def served(D=128, page=16, row=None, vrow=None, blocks=64, batch=3):
+        p = _fwd_params(B=batch, H=8, SQ=64, SK=64, D=D, varlen=True)
+        p.sK.s, p.sV.s = row or 4 * D, vrow or row or 4 * D
+        return L.fable_attn_fwd_paged_ws_bytes(p, _lib.FablePagedKV(0, blocks, page, 16 * 4 * D, 16 * 4 * D), _lib.FA_BF16) >= 0
+    assert served() and served(D=64) and served(D=256) and served(page=256)
+    assert not served(D=96) and not served(page=8) and not served(page=24)
+    most = (2 ** 31 - 1) // 32
+    assert served(row=most // 8 * 8) and not served(row=most // 8 * 8 + 8) and not served(vrow=1 << 27)
+    assert not served(row=1 << 31) and not served(blocks=1 << 26, batch=32)
