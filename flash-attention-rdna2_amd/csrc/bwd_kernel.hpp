@@ -1025,38 +1025,22 @@ __global__ __launch_bounds__(256) void bwd_split_merge_kernel(FableBwdParams p, 
 // ------------------------------------------------------------ dQ from a dS workspace
 // D = rowsum(O*dO) for every (b, h, q) row: HD/8 lanes per row, one 16-byte chunk each, and
 // DSUM_RPT rows per lane whose loads are all in flight before the first sum (one row per lane
-// left each workgroup waiting on a single load pair: C3 33 us for 134 MB). Consecutive lane groups
-// take consecutive heads of a token, then the next token: in the (B, S, H, D) layouts of the API
-// a workgroup reads one contiguous run. (A workgroup per head read 256-byte pieces H*D apart: packed
-// batches of 25k rows of 32 heads, D 128, 125 us for 420 MB; now 94.) A packed batch's rows
-// are those of its whole buffer from cu_q[0] to cu_q[B], whatever sequence they belong to; the grid
-// covers B times the longest sequence. With seqused (`per` workgroups for each sequence) they are the
-// used rows of each sequence: most of a buffer of fixed slots may be unused.
+// left each workgroup waiting on a single load pair: C3 33 us for 134 MB).
 constexpr int DSUM_RPT = 4;
-template <typename T, int HD>
-__global__ __launch_bounds__(256) void bwd_dsum_kernel(FableBwdParams p, int per) {
-  constexpr int LPR = HD / 8, RPB = 256 / LPR;
+// loads of DSUM_RPT rows at o(r), d(r) (elements), then their sums to dsum[at(r)] where ok(r)
+template <typename T, int HD, class FO, class FD, class FA, class FK>
+__device__ __forceinline__ void bwd_dsum_rows(const FableBwdParams& p, FO&& at_o, FD&& at_d, FA&& at, FK&& ok) {
   using V8 = typename Dt<T>::V8;
-  const int tid = threadIdx.x;
-  if (blockIdx.x == 0) ds_build_table(p);  // the dS workspace's tile table, for the next kernels
-  const int z = per ? blockIdx.x / per : 0, nblk = per ? per : gridDim.x;
-  const long long q_first = p.cu_q ? p.cu_q[z] : 0;
-  const long long nrows = per ? bwd_seq(p, z).SQ : p.cu_q ? p.cu_q[p.B] - q_first : (long long)p.B * p.SQ, total = nrows * p.Hq;
-  const int c = tid % LPR;
+  constexpr int LPR = HD / 8;
+  const int c = threadIdx.x % LPR;
   // chunks past a head dim p.D below HD read the row's first chunk and add nothing
   const bool cok = 8 * c < p.D;
-  for (long long i0 = (long long)(blockIdx.x - z * nblk) * (RPB * DSUM_RPT); i0 < total; i0 += (long long)nblk * (RPB * DSUM_RPT)) {
+  const int c8 = cok ? 8 * c : 0;
   V8 o[DSUM_RPT], d[DSUM_RPT];
-  long long at[DSUM_RPT];
 #pragma unroll
   for (int r = 0; r < DSUM_RPT; r++) {
-    // pairs past the end load the last one (in bounds) and are not stored
-    const long long i = min(i0 + r * RPB + tid / LPR, total - 1), row = i / p.Hq;
-    const int h = (int)(i - row * p.Hq);
-    const long long b = p.cu_q ? 0 : row / p.SQ, q = p.cu_q ? q_first + row : row - b * p.SQ;
-    o[r] = *(const V8*)((const T*)p.O + b * p.os.b + (long long)h * p.os.h + q * p.os.s + (cok ? 8 * c : 0));
-    d[r] = *(const V8*)((const T*)p.dO + b * p.dos.b + (long long)h * p.dos.h + q * p.dos.s + (cok ? 8 * c : 0));
-    at[r] = b * p.lse_sb + (long long)h * p.lse_sh + q;
+    o[r] = *(const V8*)((const T*)p.O + at_o(r) + c8);
+    d[r] = *(const V8*)((const T*)p.dO + at_d(r) + c8);
   }
 #pragma unroll
   for (int r = 0; r < DSUM_RPT; r++) {
@@ -1066,8 +1050,52 @@ __global__ __launch_bounds__(256) void bwd_dsum_kernel(FableBwdParams p, int per
     acc = cok ? acc : 0.0f;
 #pragma unroll
     for (int m = LPR / 2; m > 0; m >>= 1) acc += __shfl_xor(acc, m);
-    if (c == 0 && i0 + r * RPB + tid / LPR < total) p.dsum[at[r]] = acc;
+    if (c == 0 && ok(r)) p.dsum[at(r)] = acc;
   }
+}
+// Dense batches: a workgroup per run of rows of one (b, h). (The packed kernel's walk over (row, head)
+// pairs takes two 64-bit divisions per row ahead of the loads: as the dense kernel it added 1 us to a
+// backward on the device, B4 S128 H16 D64 20.3 us and with this kernel 19.3, B4 S333 H12 D64 26.9 and 25.8.)
+template <typename T, int HD>
+__global__ __launch_bounds__(256) void bwd_dsum_kernel(FableBwdParams p, int rblocks) {
+  constexpr int LPR = HD / 8, RPB = 256 / LPR;
+  const int rb = blockIdx.x % rblocks, zh = blockIdx.x / rblocks;
+  const int h = zh % p.Hq, b = zh / p.Hq;
+  if (blockIdx.x == 0) ds_build_table(p);  // the dS workspace's tile table, for the next kernels
+  const long long ob = (long long)b * p.os.b + (long long)h * p.os.h, db = (long long)b * p.dos.b + (long long)h * p.dos.h;
+  const long long lb = (long long)b * p.lse_sb + (long long)h * p.lse_sh;
+  auto row = [&](int r) { return (rb * DSUM_RPT + r) * RPB + (int)threadIdx.x / LPR; };
+  // rows past the end load the last row (in bounds) and are not stored
+  bwd_dsum_rows<T, HD>(
+      p, [&](int r) { return ob + min(row(r), p.SQ - 1) * p.os.s; }, [&](int r) { return db + min(row(r), p.SQ - 1) * p.dos.s; },
+      [&](int r) { return lb + row(r); }, [&](int r) { return row(r) < p.SQ; });
+}
+// Packed batches: consecutive lane groups take consecutive heads of a token, then the next token: a
+// workgroup reads one contiguous run of the (total, H, D) buffer. (A workgroup per head read 256-byte
+// pieces H*D apart: 25k rows of 32 heads, D 128, 125 us for 420 MB; now 94.) The rows are those of the
+// whole buffer from cu_q[0] to cu_q[B], whatever sequence they belong to; the grid covers B times
+// the longest sequence. With seqused (`per` workgroups for each sequence) they are the used rows of
+// each sequence: most of a buffer of fixed slots may be unused.
+template <typename T, int HD>
+__global__ __launch_bounds__(256) void bwd_dsum_packed_kernel(FableBwdParams p, int per) {
+  constexpr int LPR = HD / 8, RPB = 256 / LPR;
+  if (blockIdx.x == 0) ds_build_table(p);
+  const int z = per ? blockIdx.x / per : 0, nblk = per ? per : gridDim.x;
+  const long long q_first = p.cu_q[z];
+  const long long total = (per ? bwd_seq(p, z).SQ : p.cu_q[p.B] - q_first) * p.Hq;
+  for (long long i0 = (long long)(blockIdx.x - z * nblk) * (RPB * DSUM_RPT); i0 < total; i0 += (long long)nblk * (RPB * DSUM_RPT)) {
+    long long q[DSUM_RPT];
+    int h[DSUM_RPT];
+#pragma unroll
+    for (int r = 0; r < DSUM_RPT; r++) {
+      // pairs past the end load the last one (in bounds) and are not stored
+      const long long i = min(i0 + r * RPB + threadIdx.x / LPR, total - 1), row = i / p.Hq;
+      h[r] = (int)(i - row * p.Hq);
+      q[r] = q_first + row;
+    }
+    bwd_dsum_rows<T, HD>(
+        p, [&](int r) { return (long long)h[r] * p.os.h + q[r] * p.os.s; }, [&](int r) { return (long long)h[r] * p.dos.h + q[r] * p.dos.s; },
+        [&](int r) { return (long long)h[r] * p.lse_sh + q[r]; }, [&](int r) { return i0 + r * RPB + threadIdx.x / LPR < total; });
   }
 }
 
@@ -1360,9 +1388,10 @@ static int launch_bwd_ds(const FableBwdParams& p, hipStream_t st, int nkt) {
   // the D-row kernel reduces over a power-of-two count of lanes per row (chunks past the head
   // dim add zero)
   constexpr int DW = CKV::HD <= 32 ? 32 : (CKV::HD <= 64 ? 64 : (CKV::HD <= 128 ? 128 : 256));
-  constexpr int RPB = 256 / (DW / 8) * DSUM_RPT;  // (row, head) pairs per dsum workgroup
+  constexpr int RPB = 256 / (DW / 8) * DSUM_RPT;  // rows, packed (row, head) pairs, per dsum workgroup
+  const int rblocks = (p.SQ + RPB - 1) / RPB;
   const long long per = p.cu_q && p.seqused_q ? ((long long)p.SQ * p.Hq + RPB - 1) / RPB : 0;
-  const long long gd = per ? per * p.B : ((long long)p.SQ * p.Hq * p.B + RPB - 1) / RPB;
+  const long long gd = per ? per * p.B : p.cu_q ? ((long long)p.SQ * p.Hq * p.B + RPB - 1) / RPB : (long long)rblocks * p.Hq * p.B;
   // grids of fewer 8-wave workgroups than CUs run 4-wave ones (twice as many, half the rows)
   using CDS = BwdDsQCfg<CKV::HD, 4, CD::WPE, kDsqSets>;
   const int nqt = (p.SQ + CD::BQ - 1) / CD::BQ;
@@ -1371,7 +1400,10 @@ static int launch_bwd_ds(const FableBwdParams& p, hipStream_t st, int nkt) {
   const long long gq = (long long)(small ? nqts : nqt) * p.Hq * p.B;
   const long long gkv = (long long)nkt * p.Hk * p.B * CKV::DSPLIT;
   if (gd > 0x7FFFFFFF || gq > 0x7FFFFFFF || gkv > 0x7FFFFFFF) return fail(FA_ERR_ARG, "fable_attn_bwd: grid too large");
-  hipLaunchKernelGGL((bwd_dsum_kernel<T, DW>), dim3((unsigned)gd), dim3(256), 0, st, p, (int)per);
+  if (p.cu_q)
+    hipLaunchKernelGGL((bwd_dsum_packed_kernel<T, DW>), dim3((unsigned)gd), dim3(256), 0, st, p, (int)per);
+  else
+    hipLaunchKernelGGL((bwd_dsum_kernel<T, DW>), dim3((unsigned)gd), dim3(256), 0, st, p, rblocks);
   if (int rc = launch_status("fable_attn_bwd (dsum)")) return rc;
   if constexpr (CKV::PAIR) {
     BwdSplit sp{1, nkt, CKV::BK, 0, nullptr};
