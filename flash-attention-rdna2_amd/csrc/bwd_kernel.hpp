@@ -927,7 +927,16 @@ constexpr long long kBwdPersistMaxSteps = 16;
 // samples of 64-2048 rows, 32 / 8 heads 1720 -> 1480 us (one group at a time 1600, so with the longest
 // first 1518), not causal 3233 -> 2500; 8 of 1000-8000 rows, 16 / 4 heads 4959 -> 3459; 60 of 16-700
 // rows 544 -> 530; 64 of 20-200 rows 158 -> 160; 8 of 2048 rows 1048 -> 1052.
-constexpr int kBwdChunkKeys = 8192, kBwdSortMax = 64;
+// Groups that make no two full chunks leave a last chunk too small for the XCD: causal ones then run side
+// by side (4000 + 2500 + 100 rows, 32 / 8 heads, D 96: 741 us in chunks of two groups and one, 649 as
+// one, 659 without the order; 24 of 64-2048 rows, 8 / 2 heads 509, 430, 509), others, whose key blocks are
+// alike, one after another (the latter 829 us in chunks of four, 705 so, 950 without the order). Ranking the sequences takes every
+// workgroup about a microsecond, which key blocks of under kBwdSortSteps tiles of 32 rows do not win back:
+// 60 of 16-700 rows, 16 / 16 heads, D 64 249 -> 273 with the order, D 96 326 -> 357.
+constexpr int kBwdChunkKeys = 8192, kBwdSortMax = 64, kBwdSortSteps = 32;
+__device__ __forceinline__ bool bwd_packed_order(const FableBwdParams& p) {
+  return p.cu_q && p.B <= kBwdSortMax && (long long)((p.SQ + 31) >> 5) * p.gqa >= kBwdSortSteps;
+}
 __device__ __forceinline__ int bwd_packed_item(const FableBwdParams& p, int nkt, int L) {
   const int groups = p.Hk * p.B, R = groups / kBwdXcd, M = R * kBwdXcd * nkt;
   int group, u;
@@ -936,7 +945,7 @@ __device__ __forceinline__ int bwd_packed_item(const FableBwdParams& p, int nkt,
     group = w / nkt;
     u = w - group * nkt;
   } else {
-    const int x = L % kBwdXcd, k = L / kBwdXcd, cg = max(kBwdChunkKeys / p.SK, 1);
+    const int x = L % kBwdXcd, k = L / kBwdXcd, c0 = max(kBwdChunkKeys / p.SK, 1), cg = R >= 2 * c0 ? c0 : p.causal ? R : 1;
     const int c = k / (cg * nkt), kk = k - c * cg * nkt, n = min(cg, R - c * cg);
     u = kk / n;
     group = x + kBwdXcd * (c * cg + kk - u * n);
@@ -968,7 +977,7 @@ bwd_dkdv_pair_kernel(FableBwdParams p, int nkt, BwdSplit sp) {
   if constexpr (!PERSIST) {
     const int nitems = gridDim.x / sp.n;
     const int share = blockIdx.x / nitems;
-    const int w = p.cu_q && sp.n == 1 && p.B <= kBwdSortMax ? bwd_packed_item(p, nkt, blockIdx.x)
+    const int w = sp.n == 1 && bwd_packed_order(p) ? bwd_packed_item(p, nkt, blockIdx.x)
                                                             : xcd_group_remap(blockIdx.x - share * nitems, nitems, nkt, 1, kBwdUMajor);
     bwd_pair_item<T, C, CAUSAL, FEAT, DROP, DSW, false>(p, nkt, sp, w, share);
   } else {

@@ -337,3 +337,12 @@ def test_varlen_backward_work_order(batch, Hk, longest, D, causal):
                             cu([0, lens[z]]), lens[z], lens[z], *args)
         for x, y in zip(got, ref):   # (a split of the small grid moves a sum across at most one rounding)
             assert (x[s].float() - y.float()).abs().max() <= 2.0 ** -7 * y.float().abs().max()
+
+
+@pytest.mark.parametrize("batch,Hk,longest,D,causal", [(5, 3, 600, 128, True), (5, 3, 600, 128, False), (64, 2, 600, 64, True),
+                                                       (64, 2, 600, 64, False), (9, 8, 600, 96, False), (20, 2, 2100, 64, True),
+                                                       (24, 2, 2100, 64, True), (3, 8, 500, 64, True), (3, 8, 520, 64, False)])
+def test_varlen_backward_work_order_rules(batch, Hk, longest, D, causal):
+    """As above on both sides of the order's rules: key blocks of 32 row tiles and more (512 rows of two
+    heads), groups of an XCD that make one chunk (side by side if causal, else one by one) or several."""
+    test_varlen_backward_work_order(batch, Hk, longest, D, causal)
