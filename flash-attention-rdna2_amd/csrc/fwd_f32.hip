@@ -260,13 +260,13 @@ int launch_fwd_f32(const FableFwdParams& p, hipStream_t st) {
   // Width 64: workgroups of 8 waves while they fill two rounds of the CUs, else of 4 (twice as
   // many, two per CU): B2 S1000 H12 causal 110 -> 94 us, B2 S2000 H12 340 -> 265; at 512 and 1024
   // workgroups the 8-wave shape is the faster one (B1 S2000 H32 causal 174 and 185, B8 S1000 H16 202 and
-  // 250). Width 128: 4 waves and 32-key tiles, three workgroups' tiles per CU where the 8-wave
-  // shape with 64 keys held one (B2 S1000 H8 causal 147 -> 107 us, B4 S1500 H16 696 -> 694).
-  if (p.HD <= 64) {
-    if ((long long)((p.SQ + 127) / 128) * p.NH * p.batch < 512) return launch_f32<F32Cfg<64, 64, 4, 2>>(p, st);
-    return launch_f32<F32Cfg<64, 64, 8, 2>>(p, st);
-  }
-  if (p.HD <= 128) return launch_f32<F32Cfg<128, 32, 4, 2>>(p, st);
+  // 250). Width 128: below the same grid 4 waves and 32-key tiles, three workgroups' tiles per CU
+  // where the 8-wave shape with 64 keys holds one (B2 S1000 H8 causal 147 -> 107 us); at 512
+  // workgroups the two are alike (B8 S512 H16 109 us each), past it the 8-wave shape, which reads K and V
+  // half as often, is the faster one (B1 S3000 H32/8 causal 734 and 781, B4 S2048 H16/4 causal 637 and 811).
+  const bool small = (long long)((p.SQ + 127) / 128) * p.NH * p.batch < 512;
+  if (p.HD <= 64) return small ? launch_f32<F32Cfg<64, 64, 4, 2>>(p, st) : launch_f32<F32Cfg<64, 64, 8, 2>>(p, st);
+  if (p.HD <= 128) return small ? launch_f32<F32Cfg<128, 32, 4, 2>>(p, st) : launch_f32<F32Cfg<128, 64, 8, 2>>(p, st);
   return launch_f32<F32Cfg<256, 32, 8, 2>>(p, st);
 }
 

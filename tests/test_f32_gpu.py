@@ -223,3 +223,14 @@ LARGE = [("D64 causal 512 workgroups", 4, 64, 64, 130, 130, 64, True, -1, -1, 0.
 def test_f32_large_grid(case):
     test_f32_forward_vs_oracle(case)
     test_f32_backward_vs_oracle(case)
+
+
+# the same grids at width 128: below 512 workgroups of 128 rows the 4-wave shape, from there the 8-wave one
+LARGE_128 = [("D128 causal 510 workgroups", 5, 51, 51, 130, 130, 128, True, -1, -1, 0.0, False, 0, 0.0),
+             ("D128 causal 512 workgroups", 4, 64, 64, 130, 130, 128, True, -1, -1, 0.0, False, 0, 0.0),
+             ("D104 window gqa 512 workgroups", 4, 64, 32, 130, 140, 104, False, 70, 30, 0.0, False, 0, 0.0)]
+
+
+@pytest.mark.parametrize("case", LARGE_128, ids=[c[0] for c in LARGE_128])
+def test_f32_large_grid_width_128(case):
+    test_f32_forward_vs_oracle(case)
