@@ -186,7 +186,7 @@ struct DecArgs : FableDecParams {
   // branch, which would wait for the load at once)
   const int* table;
   int tmask;
-  int page_shift, ngrp, flags, parts, pad;
+  int page_shift, ngrp, flags, parts, nkv;
 };
 __device__ __forceinline__ DecArgs dec_reload() {
   auto k = (const __attribute__((address_space(4))) uint64_t*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -231,14 +231,24 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
   // (kv head, row group) fastest: the workgroups reading the interleaved heads of the same cache
   // pages are dispatched together, the row groups of one head to the same XCD where the heads
   // are a multiple of 8
-  const int NKV = p.NH / p.gqa, HDr = p.HD, nq = p.nq, gqa = p.gqa, NH = p.NH;
-  const int X = NKV * p.ngrp, hgl = blockIdx.x % X, kvh = hgl % NKV, grp = hgl / NKV;
+  // (scalar divisions stand in a chain of some hundred cycles each ahead of the first load: the grid's
+  // axes and the host's K/V head count leave none for calls of up to 16 rows)
+  const int NKV = p.nkv, HDr = p.HD, nq = p.nq, gqa = p.gqa, NH = p.NH;
+  const int X = gridDim.x, hgl = blockIdx.x, grp = p.ngrp > 1 ? hgl / NKV : 0, kvh = hgl - grp * NKV;
   const int r0 = 16 * grp, hg = min(16, nq * gqa - r0);  // rows of this group
   // row g: token, q head and index in q, o and lse
-  auto row_tok = [&](int g) { return (r0 + g) / gqa; };
+  auto row_tok = [&](int g) {
+    int t = 0;
+    if (nq > 1) t = (int)((unsigned)(r0 + g) / (unsigned)gqa);   // (a division per row: not for one token)
+    return t;
+  };
   auto row_of = [&](int b, int g) {
     const int tok = row_tok(g);
     return (long long)(b * nq + tok) * NH + kvh * gqa + (r0 + g - tok * gqa);
+  };
+  auto args = [&]() -> DecArgs {   // (the fixed grid's instances hold them)
+    if constexpr (SHARE) return dec_reload();
+    return p;
   };
   // segments: a stream part's (sequence, run of keys), or the one split of the grid
   DecShare str;
@@ -246,7 +256,7 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
   if constexpr (SHARE) {
     const DecArgs p = dec_reload();
     str.init(p, append, p.parts, lane);
-    const int part = blockIdx.x / X;
+    const int part = blockIdx.y;
     if (str.even) {
       sq = str.seek(p, append, part, lane, first);
       if (sq >= p.batch) return;
@@ -262,6 +272,18 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
   }
   for (bool more = true; more;) {
   const int b = SHARE ? sq : (int)blockIdx.y;
+  // q rows of this group, loaded while the lengths are on their way: one 16-byte load per thread and
+  // chunk, row index clamped (rows past the group are zeroed after the load)
+  constexpr int NQI = (16 * RCH + 255) / 256;
+  u32x4 qraw[NQI];
+  {
+    const DecArgs p = args();
+#pragma unroll
+    for (int u = 0; u < NQI; u++) {
+      const int i = min(tid + 256 * u, 16 * RCH - 1), g = i / RCH, c = i % RCH;
+      qraw[u] = *(const u32x4*)((const T*)p.q + row_of(b, min(g, hg - 1)) * HDr + (8 * c < HDr ? 8 * c : 0));
+    }
+  }
   DecSpan sp;
   if constexpr (!SHARE) sp = dec_span(p, b, append);
   int start, end;
@@ -275,7 +297,7 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
     start = sp.lo + (at - first) * kUnit;
     end = min(sp.lo + (stop - first) * kUnit, sp.hi);
     const bool begins = at == first;
-    const int part = blockIdx.x / X;
+    const int part = blockIdx.y;
     // where the combine finds this sequence's records: the first one's index, and their count
     // (negative for a stream, whose later ones are in slot 0)
     if (begins && hgl == 0 && tid == 0) {
@@ -291,7 +313,8 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
     more = !str.even && at < at_end;
   } else {
     const int n = max(sp.hi - sp.lo, 0);
-    const int chunk = (((n + p.nsplit - 1) / p.nsplit) + kDecChunk - 1) / kDecChunk * kDecChunk;
+    const int share = p.nsplit > 1 ? (int)((unsigned)(n + p.nsplit - 1) / (unsigned)p.nsplit) : n;
+    const int chunk = (share + kDecChunk - 1) / kDecChunk * kDecChunk;
     start = sp.lo + (int)blockIdx.z * chunk;
     end = min(start + chunk, sp.hi);
     if (!(p.flags & kDecFinal)) {
@@ -330,21 +353,21 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
     }
   }
 
-  // ---- q rows of this group -> LDS (fp32): one 16-byte load per thread and chunk,
-  // row index clamped (rows past the group are zeroed after the load)
+  // ---- q rows of this group -> LDS (fp32)
   // A head dim HDr = p.HD below the kernel width HD (a multiple of 8) runs with zero columns
   // HDr..HD-1 in q, K and V (rows in memory are HDr long); only HDr output columns are kept.
   bool qsplit;
   {
-  const DecArgs p = dec_reload();
+  const DecArgs p = args();
   qsplit = p.rotary != 0;
-  for (int i = tid; i < 16 * RCH; i += 256) {
-    const int g = i / RCH, c = i % RCH;
-    const bool cok = 8 * c < HDr;
-    const u32x4 raw = *(const u32x4*)((const T*)p.q + row_of(b, min(g, hg - 1)) * HDr + (cok ? 8 * c : 0));
-    const V8 v = bitcast<V8>(raw);
 #pragma unroll
-    for (int e = 0; e < 8; e++) qsh[g][8 * c + e] = g < hg && cok ? (float)v[e] : 0.0f;
+  for (int u = 0; u < NQI; u++) {
+    const int i = tid + 256 * u, g = i / RCH, c = i % RCH;
+    const bool cok = 8 * c < HDr;
+    const V8 v = bitcast<V8>(qraw[u]);
+    if (i < 16 * RCH)
+#pragma unroll
+      for (int e = 0; e < 8; e++) qsh[g][8 * c + e] = g < hg && cok ? (float)v[e] : 0.0f;
   }
   __syncthreads();
   if (p.rotary) {
@@ -382,7 +405,7 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
   float m_run = -INFINITY, l_run = 0.0f;
   const float c_log2 = p.scale * kLog2e;
   const int tok = row_tok(min(lh, hg - 1)), qpos = ctx + tok;  // this lane's row (lh)
-  const int rlo = max(dec_lo(p, b, ctx, tok), start), rhi = min(dec_hi(p, ctx, tok, append), end);
+  const int rlo = max(dec_lo(p, b, ctx, tok), start), rspan = max(min(dec_hi(p, ctx, tok, append), end) - rlo, 0);
   const float slope = (FEAT && p.alibi && lh < hg) ? p.alibi[kvh * p.gqa + (r0 + lh - tok * p.gqa)] : 0.0f;
   const T* Kc = (const T*)p.Kc;
   const T* Vc = (const T*)p.Vc;
@@ -399,7 +422,9 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
   constexpr int NVI = kDecKeys * RCH / 64;  // K (and V) row loads per lane per chunk
   const int last = end - 1;
   auto vkey = [&](int kc0, int i) { return min(kc0 + (64 * i + lane) / RCH, last); };
-  int vblk[SPT ? 1 : NVI], sblk[2], sidx[2];  // (sblk: as read; sidx: their indices)
+  // (entries are kept as read, and made pages where the rows are loaded: any use of one here would wait
+  // for it, chunk by chunk; sidx: indices of sblk)
+  int vblk[SPT ? 1 : NVI], sblk[2], sidx[2];
   auto table = [&](int kc0) {
     if constexpr (SPT) {
       const int b0 = kc0 >> page_shift, bl = last >> page_shift;  // wave-uniform
@@ -410,20 +435,17 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < NVI; i++) {
-        const int e = vkey(kc0, i) >> page_shift;
-        vblk[i] = entry(bt[e & tmask], e);
-      }
+      for (int i = 0; i < NVI; i++) vblk[i] = bt[(vkey(kc0, i) >> page_shift) & tmask];
     }
   };
   // entry of load i's row: page (key >> page_shift) - (kc0 >> page_shift) of the chunk's two
   // (a key clamped to `last` lies in the chunk's last page, whose index the table clamped too)
-  auto blk_of = [&](int kc0, int i) {
+  auto blk_of = [&](int kc0, int i, const int (&pg)[2]) {
     if constexpr (SPT) {
       const int j = (vkey(kc0, i) >> page_shift) - (kc0 >> page_shift);
-      return j <= 0 ? entry(sblk[0], sidx[0]) : entry(sblk[1], sidx[1]);
+      return j <= 0 ? pg[0] : pg[1];
     } else {
-      return vblk[i];
+      return entry(vblk[i], vkey(kc0, i) >> page_shift);
     }
   };
   auto row_off = [&](int blk, int key) -> long long {
@@ -440,10 +462,15 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
   // The cache rows are read once per step: non-temporal loads keep them from displacing the
   // block table and q in the caches (C4: 368.6 -> 360.3 us for the partial kernel).
   auto load = [&](int kc0, u32x4 (&kr)[NVI], u32x4 (&vr)[NVI]) {
+    int pg[2] = {0, 0};   // (formed on the scalar unit: after the selection it took 18 VALU per chunk)
+    if constexpr (SPT) {
+#pragma unroll
+      for (int j = 0; j < 2; j++) pg[j] = __builtin_amdgcn_readfirstlane(entry(sblk[j], sidx[j]));
+    }
 #pragma unroll
     for (int i = 0; i < NVI; i++) {
       const int ch = (64 * i + lane) % RCH;
-      const long long off = row_off(blk_of(kc0, i), vkey(kc0, i)) + (vok[i] ? 8 * ch : 0);
+      const long long off = row_off(blk_of(kc0, i, pg), vkey(kc0, i)) + (vok[i] ? 8 * ch : 0);
       kr[i] = __builtin_nontemporal_load((const u32x4*)(Kc + off));
       vr[i] = __builtin_nontemporal_load((const u32x4*)(Vc + off));
     }
@@ -527,7 +554,7 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
       } else {
         t = s[r] * c_log2;
       }
-      t = ((key >= rlo) & (key < rhi)) ? t : -INFINITY;
+      t = (unsigned)(key - rlo) < (unsigned)rspan ? t : -INFINITY;
       s[r] = t;
       mx = fmaxf(mx, t);
     }
@@ -574,7 +601,7 @@ __global__ __launch_bounds__(256) void dec_partial_kernel(DecArgs p) {
 #pragma unroll
     for (int r = 0; r < 4; r++) red_o[(wave * 16 + lh) * HD + 16 * db + 4 * lg + r] = oacc[db][r];
   __syncthreads();
-  const DecArgs pe = dec_reload();
+  const DecArgs pe = args();
   for (int i = tid; i < hg * HDr; i += 256) {
     const int g = i / HDr, d = i % HDr;
     float gm = -INFINITY;
@@ -932,7 +959,7 @@ static int launch_dec_partial(const FableDecParams& p, dim3 grid, int page_shift
     a.ngrp = dec_groups(p);
     a.flags = flags;
     a.parts = parts;
-    a.pad = 0;
+    a.nkv = p.NH / p.gqa;
     hipLaunchKernelGGL((dec_partial_kernel<T, HD, decltype(ft)::value, decltype(sp)::value, decltype(sh)::value>), grid, dim3(256), 0, st, a);
   };
   using Y = std::integral_constant<bool, true>;
@@ -1000,7 +1027,7 @@ static int launch_dec_share(const FableDecParams& p, hipStream_t st, const void*
   const bool fuse = dec_fuses_append<T>(p, nv);
   if (nk && !fuse)
     if (int rc = launch_dec_append<T, HD>(p, st, nk, nv)) return rc;
-  if (int rc = launch_dec_partial<T, HD>(p, dim3((unsigned)(X * dec_share_wgs(p))), __builtin_ctz((unsigned)p.page), nk ? kDecAppend : 0, parts,
+  if (int rc = launch_dec_partial<T, HD>(p, dim3((unsigned)X, (unsigned)dec_share_wgs(p)), __builtin_ctz((unsigned)p.page), nk ? kDecAppend : 0, parts,
                                          st, fuse ? nk : nullptr, nv))
     return rc;
   hipLaunchKernelGGL((dec_combine_kernel<T, HD, 8, true>), dim3(p.batch * p.nq, p.NH), dim3(HD), 0, st, p, ngrp);
