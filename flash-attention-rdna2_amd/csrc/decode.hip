@@ -82,7 +82,8 @@ __device__ __forceinline__ DecSpan dec_span(const FableDecParams& p, int b, int 
 // sequence has one at least):
 //  * even: `parts` workgroups per (K/V head, row group); each sequence is cut into runs of `per`
 //    units, `per` the least for which the runs fit the parts, so every workgroup has one run at
-//    most. Taken where that is at most a quarter above an even share (few or alike sequences).
+//    most. Taken where that is at most a quarter above an even share (few or alike sequences), or
+//    kSegUnits units: a stream's workgroup pays a second segment, which costs about as much.
 //  * stream: otherwise (many sequences of unequal lengths) the sequences' units follow one another
 //    and each workgroup (two per part when there are more sequences than parts) takes as many, whatever sequences they belong to.
 // A sequence that lies in one workgroup is finished there; of the others each writes a partial record
@@ -134,18 +135,18 @@ struct DecShare {
   __device__ __forceinline__ void init(const FableDecParams& p, int append, int parts, int lane) {
     load(p, append, 0, lane);
     total = sum(p, append, lane, [](int u) { return u; });
-    const int least = max((int)((unsigned)(total + parts - 1) / (unsigned)parts), kMinUnits);
+    const int least = max((int)((unsigned)(total + parts - 1) / (unsigned)parts), 1);
     even = false;
     if (p.batch <= parts) {
 #pragma nounroll
-      for (per = least; 4 * per <= 5 * least; per += max(per >> 4, 1)) {
+      for (per = least; 4 * per <= 5 * least || per <= least + kSegUnits; per += max(per >> 4, 1)) {
         if (sum(p, append, lane, [=](int u) { return (int)((unsigned)(u + per - 1) / (unsigned)per); }) <= parts) {
           even = true;
           break;
         }
       }
     }
-    if (!even) per = p.batch <= parts ? least : max((least + 1) / 2, kMinUnits);
+    if (!even) per = p.batch <= parts ? least : (least + 1) / 2;
   }
   // items: runs (even) or units (stream) of a sequence
   __device__ __forceinline__ int items(int u) const { return even ? (int)((unsigned)(u + per - 1) / (unsigned)per) : u; }
@@ -170,7 +171,9 @@ struct DecShare {
       return base + n;
     }
   }
-  static constexpr int kMinUnits = 4;
+  // (at least 4 units per run and streams from a quarter above the even share on: 24 sequences of 500 keys, Hq 32 /
+  // Hk 8, D 128, 21.3 us, 19.0 now; 3 of 500 13.7 and 11.6; 5 of 300 14.1 and 11.2)
+  static constexpr int kSegUnits = 6;
 };
 
 // floats ahead of the records: two ints per sequence, for the combine
@@ -1353,12 +1356,13 @@ static int dec_checked(FableDecParams p, int dtype, void* stream, const void* ne
 // Whether the shares are worked out on the device: fp16/bf16, no count of the caller's, pages of at
 // least 16 rows, a table that can hold kShareBytes of keys and values, and a batch that equal
 // splits would not spread evenly over the parts (more sequences than parts, or a count that
-// does not divide them). The shares take 2-3 us (in the partial kernel, and a combine that is always
-// launched), which batches of short sequences do not win back (32 x 500 keys, Hq 32 / Hk 8: 15.9 us
-// with one workgroup per sequence and head, 18.9 with shares; 7 x 769-12319 keys of two heads 20.7
-// and 20.9; 16 x 100-3000 keys of 16 D-64 heads 35.5 and 31.8; 48 x 64-8192 keys, Hq 64 / Hk 8,
-// 155 and 135). Where equal splits fill the parts they stay: sequences of one length are then
-// shared evenly without (16 x 32768 keys 311 and 314 us; eight of 1000 to 16000 keys 68 and 53).
+// does not divide them). The shares take 1-2 us (ahead of the first load, and in a combine that is always
+// launched), which short sequences under a table for long ones do not win back (3 x 500 keys, Hq 32 / Hk 8,
+// D 128: 10.2 us in equal splits, 11.6 shared; 24 x 500 15.8 and 19.0; 64 x 500 26.5 and 29.1), while long ones
+// of unequal lengths gain more (12 of 750-8000 keys 65.6 and 39.7, 24 of 333-8000 123 and 78, 48 x 64-8192
+// of Hq 64 / Hk 8 155 and 135): the lengths are not known here, the size of the table is. A batch that divides the
+// parts keeps equal splits, which share sequences of one length evenly without (16 x 32768 keys 311 and 314 us)
+// but leave unequal ones waiting for the longest (eight of 1000 to 16000 keys 68 us, 53 if shared).
 constexpr long long kShareBytes = 128LL << 20;
 static bool dec_shares(const FableDecParams& p, int dtype) {
   if (dtype == FA_F32 || p.nsplit > 0 || p.batch < 2 || p.gqa <= 0 || p.page < 16) return false;
