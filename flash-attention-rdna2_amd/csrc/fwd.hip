@@ -66,11 +66,19 @@ __global__ __launch_bounds__(256) void fwd_split_combine_kernel(FableFwdParams p
   }
   float ls[NMAX];
   f32x4 ov[NMAX];
+  // (paged instances: a share without keys writes its LSE only; many shares then load first the LSEs and O
+  // where there is one)
+  constexpr bool kTwo = PG && NMAX > 8;
 #pragma unroll
   for (int k = 0; k < NMAX; k++) {
     const long long rk = (long long)min(k, sp.n - 1) * sp.rows + r;
     ls[k] = sp.lse[rk];
-    ov[k] = *(const f32x4*)(sp.o + rk * p.HD + 4 * c);
+    if (!kTwo) ov[k] = *(const f32x4*)(sp.o + rk * p.HD + 4 * c);
+  }
+  if constexpr (kTwo) {
+#pragma unroll
+    for (int k = 0; k < NMAX; k++)
+      if (k < sp.n && ls[k] != -INFINITY) ov[k] = *(const f32x4*)(sp.o + ((long long)k * sp.rows + r) * p.HD + 4 * c);
   }
   float m = -INFINITY;
 #pragma unroll
@@ -84,7 +92,7 @@ __global__ __launch_bounds__(256) void fwd_split_combine_kernel(FableFwdParams p
       if (k < sp.n) {
         const float wk = __expf(ls[k] - m);
         wsum += wk;
-        acc += wk * ov[k];
+        if (!PG || ls[k] != -INFINITY) acc += wk * ov[k];
       }
     }
   }

@@ -61,6 +61,9 @@ struct FwdCfg {
   static_assert(HD % 32 == 0 && BC % 32 == 0, "shape");
 };
 
+// least keys of a paged instance's share (64: 1.05x slower over 66 calls of 64-256 rows; 256: 1.08x over
+// batch 1 with up to 600 keys, alike elsewhere)
+constexpr int kPagedShareKeys = 128;
 // (the fields of a paged instance's argument; constants for the others)
 __device__ __forceinline__ int paged_leftpad(const FwdPaged& pg, int z) { return pg.leftpad ? max(pg.leftpad[z], 0) : 0; }
 __device__ __forceinline__ int paged_leftpad(const NoPaged&, int) { return 0; }
@@ -164,10 +167,20 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
   int kstart = (bk0 / C::BC) * C::BC;
   int ntiles = bk1 > bk0 ? (bk1 - kstart + C::BC - 1) / C::BC : 0;
   if (sp.n > 1) {  // this workgroup's share of the key tiles: a contiguous run of them
-    const int per = (ntiles + sp.n - 1) / sp.n;
+    const int per = max((ntiles + sp.n - 1) / sp.n, PG ? kPagedShareKeys / C::BC : 1);
     const int t0 = min(split * per, ntiles), t1 = min(t0 + per, ntiles);
     kstart += t0 * C::BC;
     ntiles = t1 - t0;
+    if constexpr (PG) {
+      // (the share count follows from what the table can hold: a short cache leaves most shares without
+      // keys, and cut into single tiles it wrote more partials than it read keys. 16 tokens of 8 heads over up to
+      // 600 keys under a table of 32768, 8 K/V heads, D 128, batch 4: 41 -> 28 us)
+      if (ntiles == 0) {
+        for (int r = tid; r < min(C::BR, SQ - qb); r += C::NT)
+          sp.lse[(long long)split * sp.rows + (long long)w * C::BR + r] = -INFINITY;
+        return;
+      }
+    }
   }
 
   // ---- Q (B operands) in registers: lane holds query qw + 32i + l32, head-dim 16ds + 8hh..+7.
