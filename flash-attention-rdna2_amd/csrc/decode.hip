@@ -1199,7 +1199,9 @@ namespace fa {
 // rotated tokens to each of two requests with 1000-7000 cached keys (Hq 32 / Hk 8, D 128, bf16):
 // 1710 us -> 203 us. At 64 rows the tile kernel takes 0.11-0.92x the decode kernel's time (batch 1
 // to 32, 500 to 32000 keys, D 64 to 256; 16 tokens of 4 heads over 32000 keys 227 -> 51 us), at
-// 512 rows 0.07-0.39x.
+// 512 rows 0.07-0.39x. (Where a table for many keys holds a few hundred, batches of 1 to 4 with up to 256
+// rows pay the three kernels' latency: 64 rows over 600 keys under a table of 32768, batch 1, 20 us, 14 before.
+// The keys are not known here.)
 constexpr int kTileRows = 64;
 // (A window of 0 keys, which leaves no key visible, has no form in the forward's bounds: the decode
 // kernel serves it; so does it tables of 2^31 entries and more.)
@@ -1208,9 +1210,10 @@ static bool dec_uses_tiles(const FableDecParams& p, int dtype) {
          (long long)p.batch * p.max_blocks <= 0x7FFFFFFF && p.window != 0 && p.HD > 0 && p.HD <= 256 && p.HD % 8 == 0;
 }
 
-// One workgroup per new token, before the tile kernel: the token's k (rotated) and v rows go to
+// Before the tile kernel, gridDim.y workgroups per new token: the token's k (rotated) and v rows go to
 // the cache, and its q rows, rotated in fp32, to two 16-bit tensors whose sum is the rotated q to
-// 2^-16 (bf16) or 2^-22 (fp16) of its value, as the decode kernel carries it.
+// 2^-16 (bf16) or 2^-22 (fp16) of its value, as the decode kernel carries it. (One workgroup per
+// token walked 64 tokens of 64 + 8 heads in 14.5 us; now 4.6.)
 template <typename T>
 __global__ __launch_bounds__(256) void dec_prep_kernel(FableDecParams p, const T* nk, const T* nv, T* qhi, T* qlo, int page_shift) {
   const int b = blockIdx.x / p.nq, tk = blockIdx.x % p.nq, NKV = p.NH / p.gqa, HDr = p.HD;
@@ -1225,9 +1228,10 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(FableDecParams p, const T
   }
   const long long tok = (long long)b * p.nq + tk;
   const T* q = (const T*)p.q + tok * p.NH * HDr;
+  const int t0 = blockIdx.y * 256 + threadIdx.x, step = gridDim.y * 256;
   const int nh = qhi ? p.NH : 0, total = nh + (ok ? NKV : 0);  // heads to rotate: q, then k
   // rotated pairs: item i is pair i % half of head i / half
-  for (int i = threadIdx.x; i < total * half; i += 256) {
+  for (int i = t0; i < total * half; i += step) {
     const int g = i / half, j = i - g * half;
     const float c = p.cos[rp * half + j], s = p.sin[rp * half + j];
     const int ia = p.rotary == 1 ? j : 2 * j, ib = p.rotary == 1 ? j + half : 2 * j + 1;
@@ -1249,7 +1253,7 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(FableDecParams p, const T
   }
   // columns past the rotary width, and v
   const int rest = HDr - rdim;
-  for (int i = threadIdx.x; i < total * rest; i += 256) {
+  for (int i = t0; i < total * rest; i += step) {
     const int g = i / rest, d = rdim + i - g * rest;
     if (g < nh) {
       const long long o = (tok * p.NH + g) * HDr + d;
@@ -1260,7 +1264,7 @@ __global__ __launch_bounds__(256) void dec_prep_kernel(FableDecParams p, const T
     }
   }
   if (ok)
-    for (int i = threadIdx.x; i < NKV * HDr / 8; i += 256)
+    for (int i = t0; i < NKV * HDr / 8; i += step)
       *(u32x4*)((T*)p.Vc + dst + 8 * i) = *(const u32x4*)(nv + tok * NKV * HDr + 8 * i);
 }
 
@@ -1312,7 +1316,11 @@ static int launch_dec_tiles(const FableDecParams& p, int dtype, int nsplit, char
   if (p.rotary || nk) {
     T* qhi = p.rotary ? (T*)ws : nullptr;
     T* qlo = p.rotary ? (T*)(ws + qb) : nullptr;
-    hipLaunchKernelGGL((dec_prep_kernel<T>), dim3((unsigned)((long long)p.batch * p.nq)), dim3(256), 0, st, p, (const T*)nk, (const T*)nv,
+    // (few tokens: workgroups for every 256 items of a token's walk; many fill the chip with one each)
+    const long long tokens = (long long)p.batch * p.nq, items = (long long)(p.NH + p.NH / p.gqa) * p.HD / 2;
+    long long slices = 2048 / tokens < (items + 255) / 256 ? 2048 / tokens : (items + 255) / 256;
+    slices = slices > 1 ? slices : 1;
+    hipLaunchKernelGGL((dec_prep_kernel<T>), dim3((unsigned)tokens, (unsigned)slices), dim3(256), 0, st, p, (const T*)nk, (const T*)nv,
                        qhi, qlo, pg.page_shift);
     if (int rc = launch_status("fable_attn_dec (append)")) return rc;
     if (p.rotary) {
