@@ -274,6 +274,12 @@ __device__ __forceinline__ int xcd_remap(int L, int N) {
   return x * per + (x < rem ? x : rem) + idx;
 }
 
+// An XCD hands its workgroups to its four shader engines in turn, whatever each has left to do. Where
+// the items of R groups follow one another (u-major), R of 2, 4 or 8 gives an engine the same groups
+// for good, and with packed sequences of unequal lengths one engine sets the run time. Turned by
+// xcd_turn(R, u) at step u, every group visits every engine.
+__device__ __forceinline__ int xcd_turn(int R, int u) { return R == 2 ? u >> 1 : u; }
+
 // blockIdx.x -> work index for a grid of N = (K/V groups) x gqa x U work items: work index
 // w = (group * gqa + sibling) * U + u, where a K/V group is one K/V head of one sequence, its
 // gqa query heads (siblings) read the same K/V, and u runs over the U items of one query head
@@ -292,6 +298,9 @@ __device__ __forceinline__ int xcd_remap(int L, int N) {
 //    (causal, head dim 256), and over the 4 heads per XCD of causal S=16384 H=32 it read 1.6x
 //    the HBM bytes (1.80 vs 1.12 GB per launch) for the same time.
 //  * Groups past the last full round of 8 are cut into 8 contiguous ranges.
+//  * `rotate`: see xcd_turn (the paged forward, whose sibling heads are rows of one item: 8 prompts of
+//    315-2000 rows over 2600-6000 keys, 16 / 4 heads, D 128 650 -> 392 us, D 64 468 -> 271; D 128
+//    with 16 / 2 heads 660 -> 520).
 // u-major limits (items per XCD): the forward kernels keep the 4 heads per XCD of long causal
 // sequences group after group; the backward kernels gain from u-major up to 512. Dense plain
 // causal forward grids up to head dim 128 run u-major up to kFwdUMajorCausal (their q tiles
@@ -300,7 +309,7 @@ __device__ __forceinline__ int xcd_remap(int L, int N) {
 // 1.18x, D64 1.13-1.17x, C2 1.00-1.015x. Non-causal tiles are all alike, and u-major only
 // spread a CU's concurrent workgroups over more heads (B4 S4096 non-causal 0.92x).
 constexpr int kFwdUMajor = 128, kBwdUMajor = 512, kFwdUMajorCausal = 512;
-__device__ __forceinline__ int xcd_group_remap(int L, int N, int U, int gqa, int umajor_max) {
+__device__ __forceinline__ int xcd_group_remap(int L, int N, int U, int gqa, int umajor_max, bool rotate = false) {
   constexpr int kXcd = 8;
   const int G = U * gqa;                   // items per K/V group
   const int R = N / G / kXcd;              // groups per XCD in the full rounds
@@ -309,7 +318,7 @@ __device__ __forceinline__ int xcd_group_remap(int L, int N, int U, int gqa, int
   const int x = L % kXcd, k = L / kXcd;    // k < R * G
   if (R * G > umajor_max) return (x + kXcd * (k / G)) * G + k % G;
   const int u = k / (R * gqa), v = k % (R * gqa);
-  const int group = x + kXcd * (v / gqa), sib = v % gqa;
+  const int g = v / gqa, sib = v % gqa, group = x + kXcd * (rotate ? (g + xcd_turn(R, u)) % R : g);
   return (group * gqa + sib) * U + u;
 }
 

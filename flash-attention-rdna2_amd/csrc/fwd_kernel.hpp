@@ -109,7 +109,7 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
                                                                 : kFwdUMajor;
   // (PG: items are (sequence, K/V head, tile of packed rows); h is the group's first q head)
   const int gp = PG ? p.gqa : 1, nheads = p.NH / gp;
-  const int w = xcd_group_remap(blockIdx.x - split * nitems, nitems, nqt, PG ? 1 : p.gqa, umax);
+  const int w = xcd_group_remap(blockIdx.x - split * nitems, nitems, nqt, PG ? 1 : p.gqa, umax, PG);
   const int qti = w % nqt, zh = w / nqt;
   const int h = (zh % nheads) * gp, z = zh / nheads;
   const int qt = (PG ? p.causal != 0 : CAUSAL) ? (nqt - 1 - qti) : qti;

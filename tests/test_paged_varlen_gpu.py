@@ -114,3 +114,18 @@ def test_pages_before_the_window_are_not_read(D, page, window):
         vc[bt[z, lo // page].item(), :lo % page] = float("nan")
         hidden[z, :lo // page] = 3 * nb
     assert torch.equal(f(hidden), want)
+
+
+@pytest.mark.parametrize("batch,Hk,gqa", [(8, 2, 4), (8, 4, 2), (8, 8, 1), (12, 2, 4), (9, 3, 2), (3, 1, 4)])
+def test_paged_work_order(batch, Hk, gqa):
+    """The order of the work items (the groups of an XCD turned step by step): every tile of every prompt,
+    whatever the count of K/V groups per XCD (2, 4, 8, 3, 3 and some left over, none full), their lengths
+    unequal."""
+    import torch
+    r = np.random.default_rng(batch * Hk)
+    lq = [int(x) for x in r.integers(1, 700, batch)]
+    lk = [n + int(x) for n, x in zip(lq, r.integers(0, 500, batch))]
+    lq[batch // 2], lk[0] = 900, 1900
+    lk[batch // 2] = 1000
+    got, want = _call(("order", 64, Hk * gqa, Hk, 16, lq, lk, {}), torch.bfloat16)
+    assert orc.rel_rms(got.float().cpu().numpy(), want.float().cpu().numpy()) <= 2 * TOL["bf16"]
