@@ -1204,10 +1204,10 @@ namespace fa {
 // The keys are not known here.)
 constexpr int kTileRows = 64;
 // (A window of 0 keys, which leaves no key visible, has no form in the forward's bounds: the decode
-// kernel serves it; so does it tables of 2^31 entries and more.)
+// kernel serves it; so does it tables of 2^31 entries, and pages of 2^31 elements, and more.)
 static bool dec_uses_tiles(const FableDecParams& p, int dtype) {
   return (dtype == FA_F16 || dtype == FA_BF16) && p.gqa > 0 && (long long)p.nq * p.gqa >= kTileRows && p.page >= 16 &&
-         (long long)p.batch * p.max_blocks <= 0x7FFFFFFF && p.window != 0 && p.HD > 0 && p.HD <= 256 && p.HD % 8 == 0;
+         (long long)p.batch * p.max_blocks <= 0x7FFFFFFF && (long long)(p.NH / p.gqa) * p.HD * p.page <= 0x7FFFFFFF && p.window != 0 && p.HD > 0 && p.HD <= 256 && p.HD % 8 == 0;
 }
 
 // Before the tile kernel, gridDim.y workgroups per new token: the token's k (rotated) and v rows go to

@@ -188,7 +188,8 @@ namespace fa {
 // whether the paged instances serve the call: fp16/bf16, no dropout, pages of at least 16 rows, a
 // head dim whose kernel width is 64, 128 or 256 (the other widths would run with a third of their
 // columns zero: for those a gather and the packed forward is the faster way), row strides of which 16
-// rows stay within the 32-bit offsets of a load, a table of fewer than 2^31 entries
+// rows stay within the 32-bit offsets of a load, pages under 2^31 elements apart, a table of fewer than
+// 2^31 entries
 static bool paged_served(const FableFwdParams& p, const FablePagedKV& kv, int dtype) {
   if (dtype != FA_F16 && dtype != FA_BF16) return false;
   if (p.HD <= 0 || p.HD > 256 || p.HD % 8 || p.dropout_p > 0.0f) return false;
@@ -196,6 +197,7 @@ static bool paged_served(const FableFwdParams& p, const FablePagedKV& kv, int dt
   constexpr long long kMaxRow = 0x7FFFFFFF / (16 * 2);   // elements
   if (p.sK.s < 0 || p.sK.s > kMaxRow || p.sV.s < 0 || p.sV.s > kMaxRow) return false;
   if ((long long)p.batch * kv.max_blocks > 0x7FFFFFFF) return false;
+  if (kv.k_page_stride < 0 || kv.k_page_stride > 0x7FFFFFFF || kv.v_page_stride < 0 || kv.v_page_stride > 0x7FFFFFFF) return false;
   return (w == 64 || w == 128 || w == 256) && kv.page >= 16 && (kv.page & (kv.page - 1)) == 0;
 }
 

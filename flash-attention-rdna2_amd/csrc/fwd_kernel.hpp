@@ -309,27 +309,34 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
   constexpr int NE = PG ? C::KJ : 1;
   static_assert(!PG || (kRowStep && 64 % C::DCH == 0 && 64 / C::DCH <= 16), "paged loads");
   int ent[NE], ekey = kstart, pg_cur[NE], pg_prev[NE];  // next K tile's entries and first key
-  const int wrow = tid / 64 * (64 / C::DCH);            // first row of the wave's first load
-  auto pg_index = [&](int j) {
+  // (All of this is uniform and stays on the scalar unit, in 32-bit products and ranges. With the wave's first
+  // row in a vector register and 64-bit ones, a tile took 38 vector and 113 scalar instructions more than
+  // over contiguous rows, now 10 and 60: 8 prompts of 315-2000 rows over 2600-6000 keys, 8 / 8 heads,
+  // D 128 277 -> 266 us, D 256 746 -> 654; 16 / 4 heads, D 256 1040 -> 899.)
+  const int wrow = __builtin_amdgcn_readfirstlane(tid >> 6) * (64 / C::DCH);  // first row of the wave's first load
+  constexpr int RW = 64 / C::DCH;                                             // rows of a load
+  auto pg_index = [&](int j) {   // entry of the sequence's row of the table
     if constexpr (PG)
-      return z * pg.max_blocks + (min(max(ekey + wrow + j * RSTEP, FEAT ? bk0 : 0), kvalid - 1) >> pg.page_shift);
+      return min(max(ekey + wrow + j * RSTEP, FEAT ? bk0 : 0), kvalid - 1) >> pg.page_shift;
     else
       return 0;
   };
   auto pg_fetch = [&]() {
     if constexpr (PG) {
+      const auto r = buf_rsrc32(pg.table + (long long)__builtin_amdgcn_readfirstlane(z) * (pg.max_blocks & pg.tmask), (unsigned)pg.max_blocks * 4u);
 #pragma unroll
-      for (int j = 0; j < NE; j++) ent[j] = pg.table[pg_index(j) & pg.tmask];
+      for (int j = 0; j < NE; j++) ent[j] = __builtin_amdgcn_raw_buffer_load_b32(r, (pg_index(j) & pg.tmask) * 4, 0, 0);
     }
   };
-  auto pg_load = [&](bool first, u32x4 (&ld)[C::KJ], const T* base, int key0, const int (&page)[NE], long long spg,
-                     long long srow, const int (&off)[C::KJ]) {
+  auto pg_load = [&](bool first, u32x4 (&ld)[C::KJ], const T* base, int key0, const int (&page)[NE], unsigned spg,
+                     unsigned srow, const int (&off)[C::KJ]) {
     if constexpr (PG) {
 #pragma unroll
       for (int j = 0; j < NE; j++) {
         const int key = __builtin_amdgcn_readfirstlane(key0 + wrow + j * RSTEP);
-        const int in = key & ((1 << pg.page_shift) - 1);
-        const auto r = buf_rsrc(base + page[j] * spg + in * srow, (long long)(kvalid - key) * srow * 2);
+        const unsigned in = key & ((1 << pg.page_shift) - 1);
+        const unsigned rows = __builtin_amdgcn_readfirstlane(min(max(kvalid - key, 0), RW));   // (a med3: vector only)
+        const auto r = buf_rsrc32(base + ((uint64_t)(unsigned)page[j] * spg + (uint64_t)in * srow), rows * srow * 2u);
         ld[j] = buf_load16(r, FEAT && first && key + lane / C::DCH < bk0 ? kBufZero : off[j]);
       }
     }
@@ -349,9 +356,10 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
 #pragma unroll
       for (int j = 0; j < NE; j++) {
         pg_prev[j] = pg_cur[j];
-        pg_cur[j] = __builtin_amdgcn_readfirstlane((ent[j] & pg.tmask) | (pg_index(j) & ~pg.tmask));
+        pg_cur[j] = __builtin_amdgcn_readfirstlane(ent[j]);
+        if (!pg.tmask) pg_cur[j] = __builtin_amdgcn_readfirstlane(z * pg.max_blocks + pg_index(j));
       }
-      pg_load(first, ldk, Kg, ekey, pg_cur, pg.kpg, p.sK.s, koff);
+      pg_load(first, ldk, Kg, ekey, pg_cur, (unsigned)pg.kpg, (unsigned)p.sK.s, koff);
       ekey += C::BC;
       pg_fetch();
       return;
@@ -365,7 +373,7 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
   // (PG: `ahead` K tiles have been loaded past this V tile, 0 or 1)
   auto gload_v = [&](int ahead = 1, bool first = false) {
     if constexpr (PG) {
-      pg_load(first, ldv, Vg, ekey - (1 + ahead) * C::BC, ahead ? pg_prev : pg_cur, pg.vpg, p.sV.s, voff);
+      pg_load(first, ldv, Vg, ekey - (1 + ahead) * C::BC, ahead ? pg_prev : pg_cur, (unsigned)pg.vpg, (unsigned)p.sV.s, voff);
       return;
     }
     const auto r = buf_rsrc(v_cur, v_left);

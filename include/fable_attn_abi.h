@@ -301,8 +301,8 @@ int fable_attn_fwd_ws(FableFwdParams p, int dtype, void* ws, int64_t ws_bytes, v
  * caches [num_blocks, page, NH/gqa, HD]; p.sK / p.sV give the strides of a head (.h) and of a row
  * inside a page (.s), k_page_stride / v_page_stride those of a page (elements). cu_k (or seqused_k)
  * gives the key counts; entries past a sequence's last page are not read. fp16/bf16, no dropout,
- * page a power of two of at least 16, kernel widths 64, 128 and 256, row strides up to 128 MiB, fewer
- * than 2^31 table entries: for any other call the
+ * page a power of two of at least 16, kernel widths 64, 128 and 256, row strides up to 128 MiB, page
+ * strides and table entries under 2^31: for any other call the
  * workspace query returns -2 (gather the pages and call fable_attn_fwd); -1: an invalid call. The
  * workspace serves a key split, as in fable_attn_fwd_ws. The reference gathers the pages in Python
  * (flash_attn_interface.py:455-470). */

@@ -307,12 +307,13 @@ def test_paged_prompts_served():
     from fable_attn import _lib
     L = _lib.load()
 
-    def served(D=128, page=16, row=None, vrow=None, blocks=64, batch=3):
+    def served(D=128, page=16, row=None, vrow=None, blocks=64, batch=3, kpage=None, vpage=None):
         p = _fwd_params(B=batch, H=8, SQ=64, SK=64, D=D, varlen=True)
         p.sK.s, p.sV.s = row or 4 * D, vrow or row or 4 * D
-        return L.fable_attn_fwd_paged_ws_bytes(p, _lib.FablePagedKV(0, blocks, page, 16 * 4 * D, 16 * 4 * D), _lib.FA_BF16) >= 0
+        return L.fable_attn_fwd_paged_ws_bytes(p, _lib.FablePagedKV(0, blocks, page, kpage or 16 * 4 * D, vpage or 16 * 4 * D), _lib.FA_BF16) >= 0
     assert served() and served(D=64) and served(D=256) and served(page=256)
     assert not served(D=96) and not served(page=8) and not served(page=24)
     most = (2 ** 31 - 1) // 32
     assert served(row=most // 8 * 8) and not served(row=most // 8 * 8 + 8) and not served(vrow=1 << 27)
     assert not served(row=1 << 31) and not served(blocks=1 << 26, batch=32)
+    assert served(kpage=2 ** 31 - 8) and not served(kpage=2 ** 31) and not served(vpage=2 ** 31)
