@@ -927,6 +927,8 @@ constexpr long long kBwdPersistMaxSteps = 16;
 // samples of 64-2048 rows, 32 / 8 heads 1720 -> 1480 us (one group at a time 1600, so with the longest
 // first 1518), not causal 3233 -> 2500; 8 of 1000-8000 rows, 16 / 4 heads 4959 -> 3459; 60 of 16-700
 // rows 544 -> 530; 64 of 20-200 rows 158 -> 160; 8 of 2048 rows 1048 -> 1052.
+// Within a chunk the groups are turned step by step (xcd_turn): 8 of 200-2000 rows, 32 / 8 heads, causal, D 128
+// 496 -> 395, not causal 822 -> 703.
 // Groups that make no two full chunks leave a last chunk too small for the XCD: causal ones then run side
 // by side (4000 + 2500 + 100 rows, 32 / 8 heads, D 96: 741 us in chunks of two groups and one, 649 as
 // one, 659 without the order; 24 of 64-2048 rows, 8 / 2 heads 509, 430, 509), others, whose key blocks are
@@ -948,7 +950,7 @@ __device__ __forceinline__ int bwd_packed_item(const FableBwdParams& p, int nkt,
     const int x = L % kBwdXcd, k = L / kBwdXcd, c0 = max(kBwdChunkKeys / p.SK, 1), cg = R >= 2 * c0 ? c0 : p.causal ? R : 1;
     const int c = k / (cg * nkt), kk = k - c * cg * nkt, n = min(cg, R - c * cg);
     u = kk / n;
-    group = x + kBwdXcd * (c * cg + kk - u * n);
+    group = x + kBwdXcd * (c * cg + (kk - u * n + xcd_turn(n, u)) % n);
   }
   const int r = group / p.Hk, kvh = group - r * p.Hk, lane = threadIdx.x & 63;
   const int len = lane < p.B ? bwd_seq(p, lane).SQ : 0;
