@@ -150,3 +150,28 @@ def test_split_counts(splits):
     o, l, _, _ = run_kernel(c, "f16", num_splits=splits)
     o_ref, l_ref = run_oracle(c, "f16")
     check(o, l, o_ref, l_ref, "f16", f"tiles in {splits} splits")
+
+
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+def test_largest_probability_is_not_rounded(dt, softcap):
+    """One key of logit b > 0 behind 70 keys of logit 0, values 1 and 0: the result is the probability of the
+    one, whose numerator is exactly 1 in 16 bits when the row's own maximum is its exponent's base. Then
+    only the result is rounded, by half a unit in its last place (of 8 significant bits in bf16, 11 in
+    fp16: at most 2^-8 and 2^-11 of the value; 1e-5 for the fp32 sums); against an older maximum the
+    numerator e^b is rounded as well."""
+    import torch
+
+    from fable_attn import _C
+    B, nq, D, page, n = 40, 64, 64, 128, 70
+    t = {"f16": torch.float16, "bf16": torch.bfloat16}[dt]
+    b = torch.arange(B, device="cuda") / 64 + 3.0            # exact in both types
+    q, kc, vc = torch.zeros(B, nq, 1, D, device="cuda", dtype=t), *(torch.zeros(B, page, 1, D, device="cuda", dtype=t) for _ in range(2))
+    q[..., 0] = 1
+    kc[:, n, 0, 0], vc[:, n] = b.to(t), 1
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    out, _ = _C.dec(q, kc, vc, torch.arange(B, dtype=torch.int32, device="cuda").view(B, 1), i32([n + 1] * B), None, None, None,
+                    None, False, 1.0, -1, 0, None, False, softcap)
+    x = b.double() if not softcap else softcap * torch.tanh(b.double() / softcap)
+    want = (x.exp() / (x.exp() + n)).view(B, 1, 1, 1)
+    assert ((out.double() - want).abs() / want).max() <= {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt] + 1e-5
