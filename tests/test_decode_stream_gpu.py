@@ -4,8 +4,9 @@ the fp64 decode oracle with the bounds of the decode tests: batches of unequal l
 end inside a workgroup's share, span several of them, or are empty; more sequences than a wave has
 lanes; several tokens and heads packed into groups of 16 rows (with the last group partly filled);
 K/V head counts that do not divide the CUs; every kernel width; the append written by the
-workgroups that read the new keys, with a left pad past them, both rotary forms and a partial
-width; a dense cache read without a block table; and the same call replayed as a graph."""
+workgroups that read the new keys, with a left pad past them and both rotary forms; a dense cache read
+without a block table. Which path a call takes is asserted from the workspace it asks for
+(test_shared_path). Replays of a captured shared call are in test_graph_gpu.py."""
 import numpy as np
 import pytest
 
@@ -55,11 +56,13 @@ def widen(c, bytes_held=1 << 28):
     return c
 
 
-@pytest.mark.parametrize("wide", [True, False], ids=["shared", "fixed"])
+# (the rule also leaves four of CASES on equal splits under the wide table: batches of 3 and 2 that divide the
+# parts, and pages under 16 rows; SHARED holds such heads and groups on the shared path)
+@pytest.mark.parametrize("wide", [True, False], ids=["wide", "narrow"])
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 def test_stream_parity(case, dt, wide):
-    print(f"[stream] {case[0]} {dt} {'shared' if wide else 'fixed'}", flush=True)
+    print(f"[stream] {case[0]} {dt} {'wide' if wide else 'narrow'}", flush=True)
     c = make_case(case, dt)
     c = widen(c) if wide else c
     o, l, kc, vc = run_kernel(c, dt)
@@ -173,3 +176,84 @@ def test_append_of_a_misaligned_new_token():
     _lib.check(L.fable_attn_dec(p, _lib.FA_BF16, torch.cuda.current_stream().cuda_stream, nk.data_ptr(), nv.data_ptr()), "dec")
     torch.cuda.synchronize()
     assert torch.equal(vc[0, 100], nv[0, 0]) and torch.equal(kc[0, 100], nk[0, 0])
+
+
+def shared(batch, nq, NH, Hk, D, page, max_blocks, append):
+    """Whether such a call is shared out on the device: its workspace is then two ints per sequence and two
+    records of 16 rows for each workgroup of a grid of one per part (two if there are more sequences than
+    parts), not a partial per row and split."""
+    from fable_attn import _lib
+    L = _lib.load()
+    p = _lib.FableDecParams()
+    p.batch, p.NH, p.gqa, p.HD, p.page, p.max_blocks, p.nq, p.window, p.scale = batch, NH, NH // Hk, D, page, max_blocks, nq, -1, 1.0
+    X = Hk * -(-nq * (NH // Hk) // 16)
+    parts = 256 // X
+    if parts * X < 224:
+        parts = -(-512 // X)
+    parts = max(min(parts, batch * (-(-max_blocks * page // 64) + 1)), 1)
+    wgs = parts if batch <= parts else 2 * parts
+    want = ((2 * batch + 63) // 64 * 64 + wgs * 2 * X * 16 * (D + 2)) * 4
+    return L.fable_attn_dec_ws_bytes(p, _lib.FA_BF16, int(append)) == want
+
+
+# name, HD, NH, gqa, ctx(list per batch), window, rotary, append, leftpad, nq, softcap, alibi, page
+SHARED = [
+    ("96 kv heads", 64, 96, 1, [500, 3, 200, 0, 77], -1, 0, True, 0, 1, 0.0, False, 16),
+    ("20 heads in a group", 128, 40, 20, [900, 40, 0, 300, 1000], -1, 0, True, 0, 2, 0.0, False, 16),
+    ("17 heads in a group, one token", 128, 34, 17, [900, 40, 0, 300, 1000], -1, 1, True, 0, 1, 0.0, False, 16),
+    ("short, many parts", 128, 2, 2, [1, 63, 64, 65, 0, 300, 128], -1, 0, False, 0, 1, 0.0, False, 16),
+    ("alike, 24 sequences", 128, 8, 1, [500] * 24, -1, 0, False, 0, 1, 0.0, False, 16),
+]
+
+
+@pytest.mark.parametrize("case", SHARED, ids=[c[0] for c in SHARED])
+def test_shared_path(case):
+    name, HD, NH, gqa, ctx, _, _, append, _, nq, _, _, page = case
+    c = widen(make_case(case, "bf16"))
+    assert shared(len(ctx), nq, NH, NH // gqa, HD, page, c["bt"].shape[1], append)
+    o, l, _, _ = run_kernel(c, "bf16")
+    o_ref, l_ref = run_oracle(c, "bf16")
+    check(o, l, o_ref, l_ref, "bf16", "shared " + name)
+
+
+def test_append_by_several_row_groups():
+    """One token of 20 heads per K/V head, a single sequence: two row groups write the one new key."""
+    c = make_case(("20 heads, one token", 128, 40, 20, [700], -1, 1, True, 0, 1, 0.0, False, 16), "bf16")
+    o, l, _, vc = run_kernel(c, "bf16")
+    o_ref, l_ref = run_oracle(c, "bf16")
+    check(o, l, o_ref, l_ref, "bf16", "append by two row groups")
+    assert np.array_equal(to_np(vc)[c["bt"][0, 700 // 16], 700 % 16], c["nv"][0, 0])
+
+
+@pytest.mark.parametrize("gqa", [4, 20])
+def test_shared_dense_cache_without_table(gqa):
+    """A dense cache large enough to be shared out, read and appended to without a block table, against the
+    table spelt out (whose append runs ahead in a kernel of its own), bit for bit."""
+    import torch
+
+    from fable_attn import _lib
+    L = _lib.load()
+    B, Hk, D, cap = 5, 2, 128, 65536
+    H = gqa * Hk
+    assert shared(B, 1, H, Hk, D, cap, 1, True)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=torch.bfloat16)
+    q, nk, nv, kc0, vc0 = rnd(B, 1, H, D), rnd(B, 1, Hk, D), rnd(B, 1, Hk, D), rnd(B, cap, Hk, D), rnd(B, cap, Hk, D)
+    lens = torch.tensor([9000, 0, 1, 640, 65535], dtype=torch.int32, device="cuda")
+    res = []
+    for table in (None, torch.arange(B, dtype=torch.int32, device="cuda").view(B, 1)):
+        kc, vc, out = kc0.clone(), vc0.clone(), torch.empty_like(q)
+        p = _lib.FableDecParams()
+        p.q, p.Kc, p.Vc, p.o, p.ctx_len = q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), lens.data_ptr()
+        p.block_table = table.data_ptr() if table is not None else None
+        p.batch, p.NH, p.gqa, p.HD, p.page, p.max_blocks, p.nq, p.window, p.scale = B, H, gqa, D, cap, 1, 1, -1, D ** -0.5
+        n = L.fable_attn_dec_ws_bytes(p, _lib.FA_BF16, 1)
+        ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+        st = torch.cuda.current_stream().cuda_stream
+        _lib.check(L.fable_attn_dec_ws(p, _lib.FA_BF16, ws.data_ptr(), n, st, nk.data_ptr(), nv.data_ptr()), "dec")
+        torch.cuda.synchronize()
+        res.append((out, kc, vc))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+    z = torch.arange(B, device="cuda")
+    assert torch.equal(res[0][1][z, lens.long()], nk[:, 0]) and torch.equal(res[0][2][z, lens.long()], nv[:, 0])

@@ -7,7 +7,7 @@ the same inputs: bitwise, since the graph runs the same kernels on the same data
 
 Covered: flash_attn_func on a grid that takes the key split (two kernels and a workspace) and on
 one that does not, and flash_attn_with_kvcache decode over a paged cache with several splits
-(scratch) and with cache lengths changed between replays."""
+(scratch) or with its keys shared out on the device, and with cache lengths changed between replays."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -96,5 +96,31 @@ def test_kvcache_decode_graph_replays():
 
     from fable_attn import _C
     assert _C.num_splits(B, 1, Hq, Hq // Hk, bt.shape[1] * page, 0) > 1, "the decode must split"
+    call = lambda: flash_attn_with_kvcache(q, kc, vc, cache_seqlens=lens, block_table=bt, causal=True)
+    assert _replays(call, refresh, call) == 0.0
+
+
+def test_shared_decode_graph_replays():
+    """A decode whose keys are shared out on the device (a wide table, a batch that does not divide the
+    parts), with new lengths at every replay: from all alike to one sequence alone."""
+    import torch
+
+    from fable_attn.flash_attn_interface import flash_attn_with_kvcache
+    from tests.test_decode_stream_gpu import shared
+    print("[graph] shared decode", flush=True)
+    B, Hq, Hk, D, page, nb, cols = 7, 32, 8, 128, 16, 256, 4096
+    g = torch.Generator(device="cuda").manual_seed(2)
+    kc, vc = (torch.randn(B * nb, page, Hk, D, device="cuda", dtype=torch.bfloat16, generator=g) for _ in range(2))
+    bt = torch.randperm(B * nb, generator=torch.Generator().manual_seed(3)).view(B, nb).int()
+    bt = torch.cat([bt, bt[:, :1].expand(B, cols - nb)], 1).contiguous().cuda()   # (never read past nb)
+    assert shared(B, 1, Hq, Hk, D, page, cols, False)
+    lens = torch.full((B,), 4000, dtype=torch.int32, device="cuda")
+    q = torch.randn(B, 1, Hq, D, device="cuda", dtype=torch.bfloat16, generator=g)
+
+    def refresh(i):
+        q.copy_(torch.randn(q.shape, device="cuda", dtype=q.dtype, generator=g))
+        lens.copy_(torch.tensor([[4000] * 7, [4096, 1, 0, 63, 64, 65, 2000], [0, 0, 0, 4096, 0, 0, 0], [17 + 300 * z for z in range(7)]][i % 4],
+                                dtype=torch.int32))
+
     call = lambda: flash_attn_with_kvcache(q, kc, vc, cache_seqlens=lens, block_table=bt, causal=True)
     assert _replays(call, refresh, call) == 0.0
