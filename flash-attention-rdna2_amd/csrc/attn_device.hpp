@@ -180,6 +180,8 @@ __device__ __forceinline__ uint32_t dropout_bound(float p) {
 // What bounds it is VALU issue: 14 64-bit and 4 32-bit products, 18 xors and 4 others per score
 // (all of them issue at one rate on gfx950), against some 80 for the ten full rounds. Encoder
 // layers of B32 S509 H16 D64 fp16: the forward 359 -> 250 us, the pair dK/dV kernel 758 -> 625 us.
+// (The 4-wave forward at D 64, which serves windows with dropout, spills 18-25 VGPRs for the bits: B4 S2048
+// H16 bf16, window 256, 133 -> 96 us all the same.)
 template <int N, class Off>
 __device__ __forceinline__ uint32_t dropout_bits(uint64_t seed, uint64_t idx0, uint64_t span, uint32_t bound, Off&& off) {
   static_assert(N <= 32, "one word of bits");
@@ -322,7 +324,7 @@ __device__ __forceinline__ int xcd_group_remap(int L, int N, int U, int gqa, int
   const int x = L % kXcd, k = L / kXcd;    // k < R * G
   if (R * G > umajor_max) return (x + kXcd * (k / G)) * G + k % G;
   const int u = k / (R * gqa), v = k % (R * gqa);
-  const int g = v / gqa, sib = v % gqa, group = x + kXcd * (rotate ? (g + xcd_turn(R, u)) % R : g);
+  const int group = x + kXcd * (rotate ? (v / gqa + xcd_turn(R, u)) % R : v / gqa), sib = v % gqa;
   return (group * gqa + sib) * U + u;
 }
 

@@ -167,7 +167,8 @@ fwd_kernel(FableFwdParams p, int nqt, FwdSplit sp, PGT pg) {
   int kstart = (bk0 / C::BC) * C::BC;
   int ntiles = bk1 > bk0 ? (bk1 - kstart + C::BC - 1) / C::BC : 0;
   if (sp.n > 1) {  // this workgroup's share of the key tiles: a contiguous run of them
-    const int per = max((ntiles + sp.n - 1) / sp.n, PG ? kPagedShareKeys / C::BC : 1);
+    int per = (ntiles + sp.n - 1) / sp.n;
+    if (PG) per = max(per, kPagedShareKeys / C::BC);
     const int t0 = min(split * per, ntiles), t1 = min(t0 + per, ntiles);
     kstart += t0 * C::BC;
     ntiles = t1 - t0;
