@@ -45,11 +45,17 @@ __device__ __forceinline__ void query_range_b(const FableBwdParams& p, int k0, i
   }
 }
 
-// Logit transforms of a FEAT kernel, one per step loop, chosen by a uniform switch outside it
-// (bwd_with_mode): plain (windows, dropout), alibi, softcap (alibi too, with slope 0 where there
-// is none). With the flags tested inside the loop, every score of every window or dropout call
-// went through the alibi term, two uniform branches and the mask: encoder layers with dropout
-// (B32 S509 H16 D64 fp16, interior tiles mostly) ran the pair dK/dV kernel in 625 us, now 360.
+// Logit transforms of a FEAT kernel, chosen by a uniform switch (bwd_with_mode) outside the pair dK/dV
+// kernel's step loop, and once per tile in the others: plain (windows, dropout), alibi, softcap (alibi
+// too, with slope 0 where there is none). With the flags tested per score, every score of every
+// window or dropout call went through the alibi term, two uniform branches and the mask: encoder layers
+// with dropout (B32 S509 H16 D64 fp16, interior tiles mostly) ran the pair kernel in 625 us, now 360.
+// The pair kernel holds three copies of its loop and pays for it in registers: 8-106 VGPRs spilled per
+// feature instance (dropout with the plain copy alone: 0-8), where one loop with tests spilled 0-57.
+// All of them gained all the same, backward of B4 S2048 H16 causal bf16, before the switch and with it: D 64
+// window 256 184 and 127 us, alibi 382 and 246, softcap 417 and 348; D 128 222 and 197, 411 and 325, 474 and
+// 381; packed short samples (the persistent grid, 64 of 100-512 rows, H 16) D 64 376 and 281, 397 and 299, 413 and
+// 334, D 128 529 and 450, 553 and 490, 566 and 541.
 enum : int { kBwdPlain = 0, kBwdAlibi = 1, kBwdCap = 2 };
 template <bool FEAT, typename F>
 __device__ __forceinline__ void bwd_with_mode(const FableBwdParams& p, F&& f) {

@@ -1212,7 +1212,8 @@ static bool dec_uses_tiles(const FableDecParams& p, int dtype) {
 
 // Before the tile kernel, gridDim.y workgroups per new token: the token's k (rotated) and v rows go to
 // the cache, and its q rows, rotated in fp32, to two 16-bit tensors whose sum is the rotated q to
-// 2^-16 (bf16) or 2^-22 (fp16) of its value, as the decode kernel carries it. (One workgroup per
+// 2^-16 (bf16) or 2^-22 (fp16) of its value, as the decode kernel carries it; in fp16 no better than
+// 2^-25 absolute (the low part of values under 2^-3 is subnormal). (One workgroup per
 // token walked 64 tokens of 64 + 8 heads in 14.5 us; now 4.6.)
 template <typename T>
 __global__ __launch_bounds__(256) void dec_prep_kernel(FableDecParams p, const T* nk, const T* nv, T* qhi, T* qlo, int page_shift) {

@@ -340,7 +340,9 @@ int fable_attn_dec(FableDecParams p, int dtype, void* stream, const void* new_k,
  * split count, 0 for the library's choice (at most 32 splits on the tile path, 512 elsewhere).
  * p.block_table may be NULL in fp16/bf16: sequence b's pages are then b*max_blocks, b*max_blocks+1,
  * ... (a dense cache). fable_attn_dec_ws_bytes gives the bytes to pass (256-byte aligned device memory, scratch per call); `append` tells whether
- * new_k/new_v will be passed. Same results as fable_attn_dec up to fp32 summation order. */
+ * new_k/new_v will be passed. Same results as fable_attn_dec up to fp32 summation order. The tokens of
+ * a call share the reads of K and V: a V row that is not finite reaches the results of the tokens that
+ * do not see it too (as in the forward, whose masked keys meet probabilities of 0). */
 int64_t fable_attn_dec_ws_bytes(FableDecParams p, int dtype, int append);
 int fable_attn_dec_ws(FableDecParams p, int dtype, void* ws, int64_t ws_bytes, void* stream, const void* new_k,
                       const void* new_v);
