@@ -1202,12 +1202,18 @@ namespace fa {
 // 512 rows 0.07-0.39x. (Where a table for many keys holds a few hundred, batches of 1 to 4 with up to 256
 // rows pay the three kernels' latency: 64 rows over 600 keys under a table of 32768, batch 1, 20 us, 14 before.
 // The keys are not known here.)
-constexpr int kTileRows = 64;
+// With few K/V heads and sequences the tile kernel has few tiles, each in at most 32 splits, and the decode
+// kernel up to 512 splits of every 16 rows: up to kTileStreams (sequence, K/V head, 16 rows) the decode kernel
+// keeps the call. One token, 64 heads of one K/V head, D 128: batch 1, 8000 keys 18 us and 24 on the tiles,
+// 32000 28 and 49, batch 4 26 and 25, 49 and 52; past it batch 16, 8000 keys 46 and 35. 128 heads: batch 2,
+// 32000 keys 49 and 56, batch 4 82 and 57.
+constexpr int kTileRows = 64, kTileStreams = 16;
 // (A window of 0 keys, which leaves no key visible, has no form in the forward's bounds: the decode
 // kernel serves it; so does it tables of 2^31 entries, and pages of 2^31 elements, and more.)
 static bool dec_uses_tiles(const FableDecParams& p, int dtype) {
+  if (p.gqa <= 0 || (long long)p.batch * (p.NH / p.gqa) * dec_groups(p) <= kTileStreams) return false;
   return (dtype == FA_F16 || dtype == FA_BF16) && p.gqa > 0 && (long long)p.nq * p.gqa >= kTileRows && p.page >= 16 &&
-         (long long)p.batch * p.max_blocks <= 0x7FFFFFFF && (long long)(p.NH / p.gqa) * p.HD * p.page <= 0x7FFFFFFF && p.window != 0 && p.HD > 0 && p.HD <= 256 && p.HD % 8 == 0;
+         (long long)p.batch * p.max_blocks <= 0x7FFFFFFF && p.max_blocks < (1 << 29) && (long long)(p.NH / p.gqa) * p.HD * p.page <= 0x7FFFFFFF && p.window != 0 && p.HD > 0 && p.HD <= 256 && p.HD % 8 == 0;
 }
 
 // Before the tile kernel, gridDim.y workgroups per new token: the token's k (rotated) and v rows go to

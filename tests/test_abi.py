@@ -292,12 +292,12 @@ def test_decode_split_count_of_many_tokens():
 
     def need(n):
         p = _lib.FableDecParams()
-        p.batch, p.NH, p.gqa, p.HD, p.page, p.max_blocks, p.nq, p.window, p.scale = 1, 8, 8, 128, 16, 512, 16, -1, 0.1
+        p.batch, p.NH, p.gqa, p.HD, p.page, p.max_blocks, p.nq, p.window, p.scale = 3, 8, 8, 128, 16, 512, 16, -1, 0.1
         p.nsplit = n
         return L.fable_attn_dec_ws_bytes(p, _lib.FA_BF16, 1)
     assert need(0) > 0 and need(1) == 0
     rows = need(2) // 2 // (128 * 4 + 4)
-    assert rows >= 128 and all(need(n) == n * rows * (128 * 4 + 4) for n in (2, 3, 8, 32))
+    assert rows >= 3 * 128 and all(need(n) == n * rows * (128 * 4 + 4) for n in (2, 3, 8, 32))
     assert need(100) == need(32)
 
 
@@ -317,3 +317,18 @@ def test_paged_prompts_served():
     assert served(row=most // 8 * 8) and not served(row=most // 8 * 8 + 8) and not served(vrow=1 << 27)
     assert not served(row=1 << 31) and not served(blocks=1 << 26, batch=32)
     assert served(kpage=2 ** 31 - 8) and not served(kpage=2 ** 31) and not served(vpage=2 ** 31)
+
+
+def test_few_rows_stay_on_the_decode_kernel():
+    """Up to 16 (sequence, K/V head, 16 rows) the decode kernel keeps a call of 64 rows and more: its
+    workspace is a partial (HD + 2 floats) of every row and split, not one of whole tiles."""
+    from fable_attn import _lib
+    L = _lib.load()
+
+    def tiles(batch, NH, gqa, nq, n=2):
+        p = _lib.FableDecParams()
+        p.batch, p.NH, p.gqa, p.HD, p.page, p.max_blocks, p.nq, p.window, p.scale, p.nsplit = batch, NH, gqa, 128, 16, 512, nq, -1, 0.1, n
+        return L.fable_attn_dec_ws_bytes(p, _lib.FA_BF16, 0) != batch * nq * NH * n * (128 + 2) * 4
+    assert not tiles(1, 64, 64, 1) and not tiles(4, 64, 64, 1) and tiles(5, 64, 64, 1)
+    assert not tiles(2, 8, 8, 16) and tiles(3, 8, 8, 16)
+    assert not tiles(1, 1, 1, 256) and tiles(1, 1, 1, 257) and tiles(1, 8, 2, 40) and not tiles(8, 8, 1, 63)

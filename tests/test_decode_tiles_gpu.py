@@ -146,7 +146,7 @@ def test_window_of_no_keys(nq, append):
 
 @pytest.mark.parametrize("splits", [1, 2, 5, 32, 100])
 def test_split_counts(splits):
-    c = make_case(("splits", 128, 16, 8, [3000, 70, 0], -1, 1, True, 0, 17, 0.0, False, 16), "f16")
+    c = make_case(("splits", 128, 16, 8, [3000, 70, 0], -1, 1, True, 0, 17, 0.0, False, 16), "f16")   # (54 groups of 16 rows)
     o, l, _, _ = run_kernel(c, "f16", num_splits=splits)
     o_ref, l_ref = run_oracle(c, "f16")
     check(o, l, o_ref, l_ref, "f16", f"tiles in {splits} splits")
@@ -175,3 +175,29 @@ def test_largest_probability_is_not_rounded(dt, softcap):
     x = b.double() if not softcap else softcap * torch.tanh(b.double() / softcap)
     want = (x.exp() / (x.exp() + n)).view(B, 1, 1, 1)
     assert ((out.double() - want).abs() / want).max() <= {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt] + 1e-5
+
+
+# Calls of few sequences and K/V heads stay on the decode kernel (up to 16 groups of 16 rows: some of CASES and
+# HIDDEN): the same shapes with more K/V heads, on the tiles.
+# name, HD, NH, gqa, ctx(list per batch), window, rotary, append, leftpad, nq, softcap, alibi, page
+MORE_HEADS = [
+    ("128 rows rotary", 128, 24, 8, [700], -1, 1, True, 0, 16, 0.0, False, 64),
+    ("no append rotary", 128, 24, 8, [900, 33], -1, 1, False, 0, 12, 0.0, False, 16),
+    ("window no append rotary", 128, 24, 8, [1200, 90], 100, 1, False, 0, 12, 0.0, False, 16),
+    ("window split", 128, 24, 8, [5003], 2000, 0, True, 0, 12, 0.0, False, 16),
+    ("split long", 128, 24, 8, [6000], -1, 1, True, 0, 17, 0.0, False, 16),
+    ("split ragged", 64, 16, 8, [5000, 3, 900], -1, 0, True, 0, 9, 0.0, False, 16),
+    ("64 heads, one token", 128, 64, 64, [3000, 0, 7, 900, 64], -1, 1, True, 0, 1, 0.0, False, 16),
+    ("16 groups: decode kernel", 128, 64, 64, [3000, 0, 7, 900], -1, 1, True, 0, 1, 0.0, False, 16),
+]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("case", MORE_HEADS, ids=[c[0] for c in MORE_HEADS])
+def test_tiles_parity_more_heads(case, dt):
+    test_tiles_parity(case, dt)
+
+
+@pytest.mark.parametrize("case", MORE_HEADS[2:4], ids=[c[0] for c in MORE_HEADS[2:4]])
+def test_hidden_more_heads(case):
+    test_nothing_below_the_first_visible_key_is_read(case, "bf16")
