@@ -1197,7 +1197,7 @@ namespace fa {
 // runs on the tile kernel of the forward (fwd_kernel over FwdPaged): the decode kernel reads a
 // sequence's K/V once per new token, which for a chunk of a prompt is all its time. Appending 512
 // rotated tokens to each of two requests with 1000-7000 cached keys (Hq 32 / Hk 8, D 128, bf16):
-// 1710 us -> 203 us. At 64 rows the tile kernel takes 0.11-0.92x the decode kernel's time (batch 1
+// 1710 us -> 197 us. At 64 rows the tile kernel takes 0.11-0.92x the decode kernel's time (batch 1
 // to 32, 500 to 32000 keys, D 64 to 256; 16 tokens of 4 heads over 32000 keys 227 -> 51 us), at
 // 512 rows 0.07-0.39x. (Where a table for many keys holds a few hundred, batches of 1 to 4 with up to 256
 // rows pay the three kernels' latency: 64 rows over 600 keys under a table of 32768, batch 1, 20 us, 14 before.
