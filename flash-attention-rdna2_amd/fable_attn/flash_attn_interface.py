@@ -494,7 +494,24 @@ def _pages_as_packed(k_cache, v_cache, block_table, cu_seqlens_k, seqused_k):
     return flat(k_cache), flat(v_cache), cu, used, span
 
 
-def _paged_prefill(q, k_cache, v_cache, block_table, cu_q, cu_k, max_sq, seqused_q, seqused_k, **kw):
+# Packed prompts with head dims past 128 gather their pages from this many query-key pairs on (by the longest
+# lengths), where a K/V head has more than _GATHER_ROWS query rows in a sequence. One wave per SIMD waits out the
+# page addresses of every 32-key tile there (1.35x the time of contiguous rows), which on long prompts costs more
+# than the gather, and that costs the less the more rows share its K/V heads. D 256, bf16, times read in place /
+# gathered: 16 / 4 heads, 4 prompts of up to 500 rows over 1500 keys (48M pairs) 85 / 132 us, 4 of 2000 over 6000
+# (768M) 752 / 627, 1 of 4000 over 12000 (768M) 971 / 758; 16 / 2 heads, 8 of 500 over 1500 (96M) 136 / 143, 4 of 1000 over
+# 3000 (192M) 246 / 243; 16 / 8 heads, 4 of 2000 over 6000 (4000 rows) 546 / 660, 8 of 4000 over 12000 3051 / 2644.
+# Up to head dim 128 reading in place is 1.06-2.9x the faster at any size.
+_GATHER_PAIRS, _GATHER_ROWS = 160_000_000, 4096
+
+
+def _gather_pays(batch, heads, heads_k, max_sq, max_sk, d):
+    """Whether packed prompts gather their pages though the kernel could read them in place."""
+    return (d > 128 and heads // heads_k * max_sq > _GATHER_ROWS
+            and batch * heads * max_sq * max_sk > _GATHER_PAIRS)
+
+
+def _paged_prefill(q, k_cache, v_cache, block_table, cu_q, cu_k, max_sq, max_sk, seqused_q, seqused_k, **kw):
     """Packed prompts over a paged cache without gathering the pages: the kernel reads K/V through
     the block table. None sends the call to the gather (and to its checks): a gradient, dropout,
     tensors or strides that the kernel cannot read in place, widths or pages without a paged
@@ -516,6 +533,10 @@ def _paged_prefill(q, k_cache, v_cache, block_table, cu_q, cu_k, max_sq, seqused
         return None
     spec = _normalize(q, k_cache[0], v_cache[0], head_axis=1, **kw) if k_cache.shape[0] else None
     if spec is None:
+        return None
+    span = int(max_sk) if max_sk else block_table.shape[1] * page
+    if (spec.wl < 0 and not spec.chunk   # (these bound the keys of a row)
+            and _gather_pays(block_table.shape[0], q.shape[1], k_cache.shape[2], int(max_sq), span, D)):
         return None
     idx = lambda t: _as_index(t, dev) if t is not None else None
     return _C.fwd_paged(q, k_cache, v_cache, idx(block_table), idx(cu_q), idx(cu_k), int(max_sq), spec.scale,
@@ -541,8 +562,8 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
         raise ValueError(f"fable_attn: varlen expects (total, nheads, headdim), got {tuple(q.shape)}")
     if block_table is not None:
         if not dropout_p and qv is None and not return_attn_probs:
-            out = _paged_prefill(q, k, v, block_table, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, seqused_q,
-                                 seqused_k, softmax_scale=softmax_scale, causal=causal,
+            out = _paged_prefill(q, k, v, block_table, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
+                                 seqused_q, seqused_k, softmax_scale=softmax_scale, causal=causal,
                                  window_size=window_size, softcap=softcap, alibi_slopes=alibi_slopes,
                                  attention_chunk=attention_chunk, descale=(q_descale, k_descale, v_descale),
                                  hints=(num_splits, pack_gqa, sm_margin))

@@ -361,3 +361,13 @@ def test_kvcache_append_refused_into_a_temporary(fake):
     with pytest.raises(NotImplementedError):
         t = kc.transpose(1, 2)
         fai.flash_attn_with_kvcache(q, t, t, k=nk, v=nk, block_table=bt)
+
+
+def test_long_wide_prompts_gather_their_pages():
+    """Where packed prompts over a paged cache leave the paged kernel for the gather: head dims past 128, more
+    than 4096 query rows per K/V head and 160M query-key pairs, both by the longest lengths."""
+    g = fai._gather_pays
+    assert g(1, 16, 4, 4000, 12000, 256) and g(4, 16, 4, 2000, 6000, 232)
+    assert not g(1, 16, 4, 4000, 12000, 128) and not g(64, 16, 4, 4000, 12000, 64)
+    assert not g(8, 16, 16, 4096, 12000, 256) and g(8, 16, 16, 4097, 12000, 256)
+    assert not g(1, 16, 2, 1000, 10000, 256) and g(1, 16, 2, 1000, 10001, 256)

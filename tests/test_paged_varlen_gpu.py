@@ -129,3 +129,26 @@ def test_paged_work_order(batch, Hk, gqa):
     lk[batch // 2] = 1000
     got, want = _call(("order", 64, Hk * gqa, Hk, 16, lq, lk, {}), torch.bfloat16)
     assert orc.rel_rms(got.float().cpu().numpy(), want.float().cpu().numpy()) <= 2 * TOL["bf16"]
+
+
+@pytest.mark.parametrize("max_sk", [1500, None, 12000])
+def test_wide_prompts_on_both_sides_of_the_gather(max_sk, monkeypatch):
+    """Head dim 256 read in place or gathered, as max_seqlen_k (a bound, or None for the table's) says: the
+    same result to the rounding of both."""
+    import torch
+
+    from fable_attn import _C, flash_attn_varlen_func
+    seen = []
+    fwd_paged = _C.fwd_paged
+    monkeypatch.setattr(_C, "fwd_paged", lambda *a, **k: seen.append(1) or fwd_paged(*a, **k))
+    g = torch.Generator(device="cuda").manual_seed(4)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=torch.bfloat16)
+    lq, lk, H, Hk, page, cols = [1030, 40], [1500, 900], 8, 1, 64, 192
+    kc, vc, q = rnd(48, page, Hk, 256), rnd(48, page, Hk, 256), rnd(sum(lq), H, 256)
+    bt = torch.randperm(48, generator=torch.Generator().manual_seed(5)).view(2, 24).int()
+    bt = torch.cat([bt, bt[:, :1].expand(2, cols - 24)], 1).contiguous().cuda()
+    cu = lambda n: torch.tensor([0] + list(np.cumsum(n)), dtype=torch.int32, device="cuda")
+    f = lambda mk: flash_attn_varlen_func(q, kc, vc, cu(lq), cu(lk), max(lq), mk, block_table=bt, causal=True)
+    got = f(max_sk)
+    assert len(seen) == (max_sk == 1500)   # 24.7M pairs; the table's 12288 keys or 12000: 200M
+    assert orc.rel_rms(got.float().cpu().numpy(), f(1500).float().cpu().numpy()) <= 2 * TOL["bf16"]
