@@ -263,10 +263,16 @@ int launch_fwd_f32(const FableFwdParams& p, hipStream_t st) {
   // 250). Width 128: below the same grid 4 waves and 32-key tiles, three workgroups' tiles per CU
   // where the 8-wave shape with 64 keys holds one (B2 S1000 H8 causal 147 -> 107 us); at 512
   // workgroups the two are alike (B8 S512 H16 109 us each), past it the 8-wave shape, which reads K and V
-  // half as often, is the faster one (B1 S3000 H32/8 causal 734 and 781, B4 S2048 H16/4 causal 637 and 811).
+  // half as often, is the faster one (B1 S3000 H32/8 causal 734 and 781, B4 S2048 H16/4 causal 637 and 811)
+  // (causal B16 S500 H16/4 1.34x, with alibi or dropout alike). Not with a left window (whose rows span few
+  // tiles: causal, window 300, B8 S1000 H8 0.87x, B1 S3000 H32/8 0.96x), nor where rows of up to 1000 fill the
+  // 128-row workgroups worse than 64-row ones (B30 S400 H8/1 0.93x). Capped logits keep the 4-wave shape: the
+  // cap times the rounding of a logit is past the fp32 tolerances of results that are compared, and the
+  // two shapes round differently.
   const bool small = (long long)((p.SQ + 127) / 128) * p.NH * p.batch < 512;
+  const bool wide = !small && p.win_left < 0 && p.softcap <= 0.0f && (p.SQ >= 1000 || (p.SQ + 127) / 128 * 2 == (p.SQ + 63) / 64);
   if (p.HD <= 64) return small ? launch_f32<F32Cfg<64, 64, 4, 2>>(p, st) : launch_f32<F32Cfg<64, 64, 8, 2>>(p, st);
-  if (p.HD <= 128) return small ? launch_f32<F32Cfg<128, 32, 4, 2>>(p, st) : launch_f32<F32Cfg<128, 64, 8, 2>>(p, st);
+  if (p.HD <= 128) return wide ? launch_f32<F32Cfg<128, 64, 8, 2>>(p, st) : launch_f32<F32Cfg<128, 32, 4, 2>>(p, st);
   return launch_f32<F32Cfg<256, 32, 8, 2>>(p, st);
 }
 
